@@ -473,4 +473,53 @@ __device__ __forceinline__ uint32_t text_match32(const DevIndex &ix, uint32_t ds
   return min(min(m, nb), lim);
 }
 
+// A small interval on the text (expanded index): the rows' suffixes, in row
+// order.  Feeding the same bases to all of them keeps that order.
+constexpr uint32_t kTextRows = 4;
+struct TextRows {
+  uint32_t q[kTextRows];
+  uint32_t n;
+};
+
+// The suffixes of rows k..l (l - k < kTextRows).
+__device__ __forceinline__ TextRows text_rows(const DevDir &D, uint32_t k, uint32_t l) {
+  TextRows R;
+  R.n = l - k + 1u;
+#pragma unroll
+  for (uint32_t j = 0; j < kTextRows; ++j) R.q[j] = D.sa[k + min(j, R.n - 1u)];
+  return R;
+}
+
+// Feeds W[i], W[i + d], ... (cnt bases) to every row at once, each compared
+// with the text before its suffix, and keeps the rows that match all of them
+// (moved on by cnt), in order.  An interval of a few rows that stays narrow
+// (a repeat of few copies) would otherwise take an LF query per base.
+template <bool STAGED>
+__device__ __forceinline__ void text_feed(const DevIndex &ix, uint32_t dsel, uint32_t comp,
+                                          const uint32_t *slot, const uint8_t *W, int32_t i,
+                                          int32_t d, int32_t cnt, TextRows &R) {
+  while (cnt > 0 && R.n) {
+    const uint32_t lim = min((uint32_t)cnt, STAGED ? 32u : 16u);
+    uint32_t kept = 0u, v[kTextRows] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (uint32_t j = 0; j < kTextRows; ++j) {
+      if (j >= R.n || R.q[j] < lim) continue;
+      const uint32_t m = STAGED ? text_match32(ix, dsel, comp, R.q[j], slot, i, d, lim)
+                                : text_match(ix, dsel, comp, R.q[j], W, i, d, lim);
+      if (m < lim) continue;
+      const uint32_t q = R.q[j] - lim;
+      if (kept == 0u) v[0] = q;
+      else if (kept == 1u) v[1] = q;
+      else if (kept == 2u) v[2] = q;
+      else v[3] = q;
+      kept++;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kTextRows; ++j) R.q[j] = v[j];
+    R.n = kept;
+    i += (int32_t)lim * d;
+    cnt -= (int32_t)lim;
+  }
+}
+
 }  // namespace fmi

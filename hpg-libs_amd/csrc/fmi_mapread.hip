@@ -13,9 +13,13 @@
 // positions and handed over from last to first with the secondary flag
 // (bwt.c:2190-2233).
 //
-// Lanes stride over the reads; a lane keeps the current strand's alignments
-// in its scratch slice (at most filter + 1 of them: a strand's rows number
-// l - k + 1 <= filter + 1 once the count has passed) for the dedup.
+// Two launches.  map_single_kernel, a thread per read, settles every read of
+// at most kStagedMaxLen bases whose strands have at most one row each (no
+// dedup, no count to filter) and marks the others in counts;
+// map_reads_kernel's lanes stride over the marked reads, a lane keeping the
+// current strand's alignments in its scratch slice (at most filter + 1 of
+// them: a strand's rows number l - k + 1 <= filter + 1 once the count has
+// passed) for the dedup.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -48,18 +52,139 @@ struct MapParams {
   MapTmp *scratch;            // lanes * (filter + 1)
 };
 
-// BWExactSearchBackward of the whole read from [0, n] on one view.
-__device__ void exact_interval(const DevDir &D, uint32_t comp, uint32_t n, const uint8_t *W,
-                               int32_t len, uint32_t &k, uint32_t &l) {
-  k = 0u;
-  l = n;
-  for (int32_t i = len - 1; i >= 0; --i) {
+// A read's count while the read waits for map_reads_kernel (a count is at
+// most 2 (filter + 1)).
+constexpr uint32_t kMapWaits = 0xFFFFFFFFu;
+
+// BWExactSearchBackward of the whole read from [0, n] on one view: whether its
+// interval is not empty (an empty one is not formed: no caller sees it), and
+// then the rows k..l (R.n = 0), or, where the search ended on the text of an
+// expanded index, its rows' suffixes (R).  kt, lt: the interval of the read's
+// last K bases, from the k-mer table (K = 0: none).  STAGED: the read's bases
+// come from the thread's LDS slot.
+template <bool STAGED>
+__device__ __forceinline__ bool live_interval(const DevIndex &ix, uint32_t dsel, uint32_t comp,
+                                              const uint8_t *W, int32_t len, const uint32_t *slot,
+                                              uint32_t K, uint32_t kt, uint32_t lt, uint32_t &k,
+                                              uint32_t &l, TextRows &R) {
+  const DevDir &D = dir_of(ix, dsel);
+  k = K ? kt : 0u;
+  l = K ? lt : ix.n;
+  R.n = 0u;
+  if (k > l) return false;
+  for (int32_t i = len - 1 - (int32_t)K; i >= 0; --i) {
+    if (l - k < kTextRows && ix.text != nullptr) {
+      R = text_rows(D, k, l);
+      text_feed<STAGED>(ix, dsel, comp, slot, W, i, -1, i + 1, R);
+      return R.n != 0u;
+    }
     uint32_t a, b;
-    if (lf_read(D, k, l, W + i, comp, a, b) > 3u) { k = n + 1u; l = n; return; }
+    const uint32_t sym = STAGED ? lf_sym(D, k, l, lds_base(slot, i), comp, a, b)
+                                : lf_read(D, k, l, W + i, comp, a, b);
+    if (sym > 3u || a > b) return false;
     k = a;
     l = b;
-    if (k > l) return;
   }
+  return true;
+}
+
+// The contig of an occurrence at text position key of len bases (binsearch,
+// search/io.h:43-64): its index + 1, or 0 when it lies in none.
+__device__ __forceinline__ uint32_t contig_of(const uint64_t *koff, uint32_t kcount, uint64_t key,
+                                              uint64_t len) {
+  uint32_t lo = 0, cnt = kcount;       // upper_bound of key in koff[0 .. kcount)
+  while (cnt > 0) {
+    const uint32_t w = cnt / 2;
+    if (koff[lo + w] <= key) { lo += w + 1; cnt -= w + 1; }
+    else cnt = w;
+  }
+  return lo == 0 || key + len > koff[lo] ? 0u : lo;
+}
+
+__device__ __forceinline__ void store_mapping(fmi_read_mapping *out, uint64_t pos, uint32_t chrom,
+                                              uint32_t rd, uint32_t strand, uint32_t secondary,
+                                              int32_t len) {
+  fmi_read_mapping o;
+  o.position = pos;
+  o.chromosome = chrom;
+  o.read = rd;
+  o.strand = (uint8_t)strand;
+  o.secondary = (uint8_t)secondary;
+  o.cigar_len = (uint16_t)len;
+  o.pad = 0u;
+  *out = o;
+}
+
+// One thread per read.  The read is packed into the thread's LDS slot once
+// for both strands, both strands' table entries are read together, and a
+// search that has narrowed to at most four rows goes on against their text,
+// 32 bases a compare: about six dependent loads for a read that occurs once
+// where an LF step per base and strand took 100 and more.  Bound by those loads' lines
+// (an entry per strand, then SA and text for one of them); the slots
+// (24 KB a workgroup) leave 6 workgroups a CU.  500 K reads of 100 bases over
+// 64 Mbp: 151 us, and 140 for the marked reads, where one launch of 64 K
+// lanes (the scratch allows no more) took 1540.
+__global__ __launch_bounds__(256) void map_single_kernel(MapParams P) {
+  __shared__ uint32_t slots[kReadRecordWords * 256u];
+  const uint32_t rd = blockIdx.x * 256u + threadIdx.x;
+  if (rd >= P.nreads) return;
+  const uint64_t off = P.offsets[rd];
+  const uint64_t len64 = P.offsets[rd + 1] - off;
+  if (len64 < 5 || len64 > kMaxReadLen) {
+    P.counts[rd] = 0;
+    P.status[rd] = len64 < 5 ? 2u : 4u;
+    return;
+  }
+  if (len64 > kStagedMaxLen) {
+    P.counts[rd] = kMapWaits;
+    return;
+  }
+  const uint8_t *W = P.reads + off;
+  const int32_t len = (int32_t)len64;
+  uint32_t *slot = slots + threadIdx.x;
+  stage_read(W, (uint32_t)len, slot);
+  const uint32_t n = P.ix.n;
+  uint32_t K = P.ix.kmer_k;
+  uint64_t e[2] = {0ull, 0ull};
+  bool dead = false;
+  if (K && len >= (int32_t)K) {
+    uint64_t w;
+    uint32_t nb;
+    lds_window(slot, len - 1, -1, w, nb);
+    const uint32_t kmask = (1u << (2u * K)) - 1u;
+    dead = (nb & ((1u << K) - 1u)) != 0u;      // an N occurs nowhere
+    const uint32_t code = (uint32_t)w & kmask;
+    if (!dead) {
+      e[0] = P.ix.kmer[0][code];
+      e[1] = P.ix.kmer[1][code ^ kmask];
+    }
+  } else {
+    K = 0u;
+  }
+  uint32_t nout = 0;
+  for (uint32_t strand = 0; strand < 2u && !dead; ++strand) {
+    // + strand: BACKWARD; - strand: FORWARD_REV (bwt.c:1996-2001)
+    uint32_t k, l;
+    TextRows R;
+    if (!live_interval<true>(P.ix, strand, strand, W, len, slot, K, (uint32_t)e[strand],
+                             (uint32_t)(e[strand] >> 32), k, l, R))
+      continue;
+    if (R.n ? R.n != 1u : k != l) {
+      P.counts[rd] = kMapWaits;
+      return;
+    }
+    const uint32_t q = R.n ? R.q[0] : sa_value(dir_of(P.ix, strand), P.ix.ratio, n, k);
+    // direction: the record's dir is 0; + keeps it, - flips it
+    const uint64_t key = strand ? (uint64_t)n + 1u - q - (uint64_t)len - 1u : (uint64_t)q;
+    const uint32_t c = contig_of(P.koff, P.kcount, key, (uint64_t)len);
+    if (c == 0u) continue;
+    if (nout < P.cap)
+      store_mapping(P.out + (uint64_t)rd * P.cap + nout, P.kstart[c - 1] + (key - P.koff[c - 1]),
+                    c - 1u, rd, strand, nout > 0 ? 1u : 0u, len);
+    ++nout;
+  }
+  P.counts[rd] = nout;
+  P.status[rd] = 0;
 }
 
 __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
@@ -68,41 +193,43 @@ __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
   MapTmp *tmp = P.scratch + (uint64_t)lane * (P.filter + 1u);
   const uint32_t n = P.ix.n;
   for (uint32_t rd = lane; rd < P.nreads; rd += lanes) {
+    if (P.counts[rd] != kMapWaits) continue;
     const uint64_t off = P.offsets[rd];
-    const uint64_t len64 = P.offsets[rd + 1] - off;
     const uint8_t *W = P.reads + off;
     fmi_read_mapping *out = P.out + (uint64_t)rd * P.cap;
-    if (len64 < 5 || len64 > kMaxReadLen) {
-      P.counts[rd] = 0;
-      P.status[rd] = len64 < 5 ? 2u : 4u;
-      continue;
+    const int32_t len = (int32_t)(P.offsets[rd + 1] - off);
+    const uint32_t K = P.ix.kmer_k && len >= (int32_t)P.ix.kmer_k ? P.ix.kmer_k : 0u;
+    uint32_t code = 0u, bad = 0u;
+    for (uint32_t j = 0; j < K; ++j) {
+      const uint32_t s = W[len - 1 - (int32_t)j];
+      bad |= s > 3u ? 1u : 0u;
+      code |= (s & 3u) << (2u * j);
     }
-    const int32_t len = (int32_t)len64;
     uint64_t tot = 0;
     uint32_t nout = 0;
     uint8_t st = 0;
     for (int type = 1; type >= 0; --type) {
       // + strand: BACKWARD; - strand: FORWARD_REV (bwt.c:1996-2001)
-      const DevDir &D = type ? P.ix.d[0] : P.ix.d[1];
+      const uint32_t dsel = type ? 0u : 1u;
+      const DevDir &D = dir_of(P.ix, dsel);
       uint32_t k, l;
-      exact_interval(D, type ? 0u : 1u, n, W, len, k, l);
+      TextRows R;
+      const uint64_t e = K && !bad ? P.ix.kmer[dsel][dsel ? code ^ ((1u << (2u * K)) - 1u) : code]
+                                   : 0ull;
       uint32_t m = 0;
-      if (k <= l) {
+      if (!bad && live_interval<false>(P.ix, dsel, dsel, W, len, nullptr, K, (uint32_t)e,
+                                       (uint32_t)(e >> 32), k, l, R)) {
+        if (R.n) { k = 0u; l = R.n - 1u; }             // the rows' suffixes are known
         tot += (uint64_t)(l - k);
         if (tot > P.filter) { st |= 1u; break; }
         for (uint32_t j = k; j <= l; ++j) {
           // direction: the record's dir is 0; + keeps it, - flips it
-          const uint64_t sa = sa_value(D, P.ix.ratio, n, j);
+          const uint64_t sa = R.n ? pick4(R.q, j) : sa_value(D, P.ix.ratio, n, j);
           const uint64_t key = type ? sa : (uint64_t)n + 1u - sa - (uint64_t)len - 1u;
-          uint32_t lo = 0, cnt = P.kcount;   // upper_bound of key in koff[0 .. kcount)
-          while (cnt > 0) {
-            const uint32_t w = cnt / 2;
-            if (P.koff[lo + w] <= key) { lo += w + 1; cnt -= w + 1; }
-            else cnt = w;
-          }
-          if (lo == 0 || key + (uint64_t)len > P.koff[lo]) continue;
-          tmp[m].pos = P.kstart[lo - 1] + (key - P.koff[lo - 1]);
-          tmp[m].chrom = lo - 1;
+          const uint32_t c = contig_of(P.koff, P.kcount, key, (uint64_t)len);
+          if (c == 0u) continue;
+          tmp[m].pos = P.kstart[c - 1] + (key - P.koff[c - 1]);
+          tmp[m].chrom = c - 1u;
           tmp[m].del = 0u;
           ++m;
         }
@@ -125,14 +252,8 @@ __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
           continue;
         }
         if (nout < P.cap) {
-          fmi_read_mapping &o = out[nout];
-          o.position = tmp[a].pos;
-          o.chromosome = tmp[a].chrom;
-          o.read = rd;
-          o.strand = (uint8_t)(type ? 0 : 1);
-          o.secondary = (uint8_t)(nout > 0 ? 1 : 0);
-          o.cigar_len = (uint16_t)len;
-          o.pad = 0u;
+          store_mapping(out + nout, tmp[a].pos, tmp[a].chrom, rd, type ? 0u : 1u,
+                        nout > 0 ? 1u : 0u, len);
         }
         ++nout;
       }
@@ -167,6 +288,7 @@ hipError_t launch_map_reads(const DevIndex &ix, const uint8_t *reads, const uint
   if (nreads == 0 || lanes == 0) return hipSuccess;
   MapParams P{ix,     reads,  offsets, koff,   kstart, kcount, nreads, filter, cap,
               out,    counts, status,  static_cast<MapTmp *>(scratch)};
+  hipLaunchKernelGGL(map_single_kernel, dim3((nreads + 255u) / 256u), dim3(256), 0, s, P);
   hipLaunchKernelGGL(map_reads_kernel, dim3(lanes / 256), dim3(256), 0, s, P);
   return hipGetLastError();
 }

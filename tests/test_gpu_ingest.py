@@ -97,3 +97,23 @@ def test_server_fastq_requests(gpu_engine):
     finally:
         srv.close()
         ix.close()
+
+
+@pytest.mark.parametrize("kind", ["tile edges", "empty reads", "one long read", "tiny"])
+def test_fastq_encode_tiles(gpu_engine, kind):
+    """Reads that end on, before and after the 8192-byte tiles of the encoding
+    kernel, more reads in a tile than it stages ends for, one read over many
+    tiles, and batches of a few bytes, each from every 16-byte alignment."""
+    hp = gpu_engine
+    rng = np.random.default_rng(146)
+    lens = {"tile edges": [8190, 0, 8191, 8192, 1, 8160, 15, 16, 17, 4095, 4096],
+            "empty reads": [0] * 5000 + [3, 0, 2] * 400 + [0] * 1030,
+            "one long read": [70_001],
+            "tiny": [1]}[kind]
+    texts = [LETTERS[rng.integers(0, 16, n)].tobytes() for n in lens]
+    for lead in range(16):
+        seq, di = hp.fastq_batch([b"G" * lead] + texts if lead else texts)
+        first = 1 if lead else 0
+        codes, offs = hp.fastq_encode_batch(seq, di[first:])
+        assert np.array_equal(codes, hp.encode_bases(b"".join(texts))), lead
+        assert np.array_equal(offs, np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64))

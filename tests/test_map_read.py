@@ -170,3 +170,49 @@ def test_gpu_map_reads_vs_oracle(gpu_engine, planted, expanded):
     finally:
         batch.free()
         ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stage", ["compact", "table", "expanded", "expanded + table"])
+def test_map_read_lengths(gpu_engine, stage):
+    """Reads around the limits of the two launches -- 256 bases staged in LDS
+    and longer, a k-mer's length, 5 and 1000 bases -- that occur once, several
+    times (also across the text's start and end) or not at all, against the
+    oracle."""
+    hp = gpu_engine
+    rng = np.random.default_rng(12)
+    g = rng.integers(0, 4, 30_000).astype(np.uint8)
+    g[20_000:21_500] = g[1_000:2_500]                # two copies of 1500 bases
+    lens = [4, 5, 7, 8, 9, 31, 32, 33, 63, 64, 65, 255, 256, 257, 272, 999, 1000]
+    reads = []
+    for L in lens:
+        for p in (0, 1_100, 20_100, 5_000, len(g) - L):
+            r = g[p:p + L].copy()
+            reads += [r, COMP[r][::-1].copy()]
+            bad = r.copy()
+            bad[L // 2] = 4
+            reads += [bad, rng.integers(0, 4, L).astype(np.uint8)]
+    koff = np.array([0, 9_000, 30_000], np.uint64)
+    kstart = np.ones(2, np.uint64)
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(kstart, np.array([9_000, 21_000], np.uint64))
+    ix.to_device()
+    o = fo.Oracle(bwts=(*ix.bwt(0), *ix.bwt(1)), ratio=16)
+    if "expanded" in stage:
+        ix.expand()
+    if "table" in stage:
+        ix.kmer_table(8)
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads).astype(np.uint8), offs)
+    try:
+        for filt, cap in ((3, 2), (50, 8)):
+            st, cnt, recs = hp.map_reads_batch(ix, batch, filt, cap)
+            for i, W in enumerate(reads):
+                ost, orecs, ototal = o.map_read(W, filt, koff, kstart, read=i, cap=cap)
+                assert (int(st[i]), int(cnt[i])) == (ost, ototal), (filt, i, len(W))
+                m = min(ototal, cap)
+                for key in ("position", "chromosome", "read", "strand", "secondary", "cigar_len"):
+                    assert np.array_equal(recs[i, :m][key], orecs[key]), (filt, i, key)
+    finally:
+        batch.free()
+        ix.close()
