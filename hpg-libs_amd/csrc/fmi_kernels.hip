@@ -1289,20 +1289,30 @@ struct LocateParams {
   uint32_t *nrows;
 };
 
+// A lane reads its interval and writes its row count; the rows of a
+// wavefront's 64 intervals are then shared out among its lanes (wave_items).
+// Bound by the records read and a 64-byte piece written per located row.  A
+// thread per (interval, slot of cap) launched cap threads with a 64-bit
+// division each for the one row most intervals have.  grid.y: the wavefronts
+// that share one set of 64 intervals (item_parts).
 __global__ __launch_bounds__(256) void locate_kernel(LocateParams P) {
   const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t iv = g / P.cap;
-  const uint32_t j = (uint32_t)(g - iv * P.cap);
-  if (iv >= P.nintervals) return;
-  const int64_t k = P.k[iv * P.stride], l = P.l[iv * P.stride];
-  // Rows outside 0..n are not in the index: such an interval yields no rows.
-  const bool valid = k >= 0 && l <= (int64_t)P.ix.n;
-  const int64_t cnt = (valid && k <= l) ? (l - k + 1) : 0;
-  const uint32_t rows = cnt < (int64_t)P.cap ? (uint32_t)cnt : P.cap;
-  if (j == 0) P.nrows[iv] = rows;
-  if (j >= rows) return;
+  const uint64_t wave0 = g & ~63ull;             // the wavefront's first interval
+  uint32_t rows = 0u;
+  if (g < P.nintervals) {
+    const int64_t k = P.k[g * P.stride], l = P.l[g * P.stride];
+    // Rows outside 0..n are not in the index: such an interval yields no rows.
+    const bool valid = k >= 0 && l <= (int64_t)P.ix.n;
+    const int64_t cnt = (valid && k <= l) ? (l - k + 1) : 0;
+    rows = cnt < (int64_t)P.cap ? (uint32_t)cnt : P.cap;
+    if (blockIdx.y == 0u) P.nrows[g] = rows;
+  }
   const DevDir &D = dir_of(P.ix, P.dsel);
-  P.pos[iv * P.cap + j] = sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)(k + j));
+  wave_items(rows, blockIdx.y, gridDim.y, [&](uint32_t s, uint64_t j) {
+    const uint64_t iv = wave0 + s;
+    P.pos[iv * P.cap + j] =
+        sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)((uint64_t)P.k[iv * P.stride] + j));
+  });
 }
 
 // --------------------------------------------------------------------------
@@ -1400,16 +1410,10 @@ struct ResolveParams {
   uint64_t *coord;
 };
 
-__global__ __launch_bounds__(256) void resolve_kernel(ResolveParams P) {
-  const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t per_slot = (uint64_t)P.cap * P.row_cap;
-  const uint64_t slot = g / per_slot;
-  if (slot >= P.nslots) return;
-  const uint32_t rem = (uint32_t)(g - slot * per_slot);
-  const uint32_t h = rem / P.row_cap, j = rem - h * P.row_cap;
-  const uint32_t stored = min(P.counts[slot], P.cap);
-  const uint64_t o = slot * per_slot + (uint64_t)h * P.row_cap + j;
-  if (h >= stored) return;
+// Row j of stored record h of slot `slot`.
+__device__ __forceinline__ void resolve_row(const ResolveParams &P, uint64_t slot, uint64_t h,
+                                            uint32_t j) {
+  const uint64_t o = (slot * P.cap + h) * P.row_cap + j;
   const fmi_hit hit = P.hits[slot * P.cap + h];
   const bool valid = hit.k >= 0 && hit.l <= (int64_t)P.ix.n;
   const int64_t nrows = (valid && hit.k <= hit.l) ? hit.l - hit.k + 1 : 0;
@@ -1443,6 +1447,19 @@ __global__ __launch_bounds__(256) void resolve_kernel(ResolveParams P) {
     P.chrom[o] = -1;
     P.coord[o] = 0;
   }
+}
+
+// A lane reads its slot's record count; the (record, row) pairs of a
+// wavefront's 64 slots are then shared out among its lanes (wave_items): most
+// slots hold no record or one.  A thread per (slot, record of cap, row of
+// row_cap) launched 90 M threads for 700 K reads at cap 16 and row_cap 4.
+__global__ __launch_bounds__(256) void resolve_kernel(ResolveParams P) {
+  const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t wave0 = g & ~63ull;             // the wavefront's first slot
+  const uint64_t stored = g < P.nslots ? min(P.counts[g], P.cap) : 0u;
+  wave_items(stored * P.row_cap, blockIdx.y, gridDim.y, [&](uint32_t s, uint64_t t) {
+    resolve_row(P, wave0 + s, t / P.row_cap, (uint32_t)(t % P.row_cap));
+  });
 }
 
 // --------------------------------------------------------------------------
@@ -1771,14 +1788,23 @@ hipError_t launch_vhelper(const DevIndex &ix, bool mm_only, uint32_t strand_mask
   return hipGetLastError();
 }
 
+// Wavefronts per 64 lanes of wave_items: one where there are enough to fill
+// the device (256 CUs of 32), else as many as fill it, at most one per 64 items
+// the 64 lanes can bring (a few wide intervals are rows enough for all).
+static uint32_t item_parts(uint64_t lanes, uint64_t items_per_lane) {
+  const uint64_t waves = (lanes + 63) / 64;
+  const uint64_t fill = std::max<uint64_t>(8192 / std::max<uint64_t>(waves, 1), 1);
+  return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(fill, items_per_lane), 8192);
+}
+
 hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, const int64_t *l,
                          uint32_t stride, uint32_t nintervals, uint32_t cap, uint64_t *pos,
                          uint32_t *nrows, hipStream_t s) {
   LocateParams P{ix, dsel, nintervals, cap, stride, k, l, pos, nrows};
-  const uint64_t total = (uint64_t)nintervals * cap;
-  const uint64_t grid = (total + 255) / 256;
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL(locate_kernel, dim3((uint32_t)grid), dim3(256), 0, s, P);
+  const uint64_t grid = ((uint64_t)nintervals + 255) / 256;
+  if (grid == 0 || cap == 0) return hipSuccess;
+  hipLaunchKernelGGL(locate_kernel, dim3((uint32_t)grid, item_parts(nintervals, cap)), dim3(256), 0,
+                     s, P);
   return hipGetLastError();
 }
 
@@ -1822,10 +1848,11 @@ hipError_t launch_resolve(const DevIndex &ix, const fmi_hit *hits, const uint32_
                           hipStream_t s) {
   ResolveParams P{ix, hits, counts, offsets, koff, kstart, 2u * nreads, cap, row_cap, kcount,
                   record_len, chrom, coord};
-  const uint64_t total = (uint64_t)2 * nreads * cap * row_cap;
-  const uint64_t grid = (total + 255) / 256;
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL(resolve_kernel, dim3((uint32_t)grid), dim3(256), 0, s, P);
+  const uint64_t grid = (2ull * nreads + 255) / 256;
+  if (grid == 0 || cap == 0 || row_cap == 0) return hipSuccess;
+  hipLaunchKernelGGL(resolve_kernel,
+                     dim3((uint32_t)grid, item_parts(2ull * nreads, (uint64_t)cap * row_cap)),
+                     dim3(256), 0, s, P);
   return hipGetLastError();
 }
 
