@@ -405,6 +405,7 @@ void fmi_index_free(fmi_index *ix) {
     (void)hipSetDevice(ix->device);
     (void)hipFree(ix->d_mem);
     (void)hipFree(ix->d_full);
+    (void)hipFree(ix->d_ctx);
     (void)hipFree(ix->d_kmer);
     (void)hipFree(ix->d_koffset);
     (void)hipFree(ix->d_kstart);
@@ -477,6 +478,29 @@ int fmi_index_expand(fmi_index *ix) {
   ix->dev.text = text;
   ix->d_full = mem;
   ix->full_bytes = bytes;
+  // The row contexts, 8 bytes per base, only where they leave at least as
+  // much memory free as they take: the searches do without them.
+  size_t free_bytes = 0, total_bytes = 0;
+  if (ix->n && hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && free_bytes >= 4 * arr) {
+    void *ctx = nullptr;
+    if (hipMalloc(&ctx, 2 * arr) != hipSuccess) {
+      (void)hipGetLastError();
+      return FMI_OK;
+    }
+    for (int d = 0; d < 2 && e == hipSuccess; ++d)
+      e = fmi::launch_row_contexts(ix->dev, (uint32_t)d,
+                                   reinterpret_cast<uint32_t *>(static_cast<char *>(ctx) + d * arr),
+                                   nullptr);
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e != hipSuccess) {
+      (void)hipFree(ctx);
+      return hip_fail(e, "row context launch");
+    }
+    for (int d = 0; d < 2; ++d)
+      ix->dev.d[d].ctx = reinterpret_cast<const uint32_t *>(static_cast<char *>(ctx) + d * arr);
+    ix->d_ctx = ctx;
+    ix->full_bytes += 2 * arr;
+  }
   return FMI_OK;
 }
 

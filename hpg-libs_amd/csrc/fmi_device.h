@@ -529,25 +529,26 @@ __device__ __forceinline__ void text_feed(const DevIndex &ix, uint32_t dsel, uin
 // Lane i brings count items; f(s, j) is called for item j of lane s's, the 64
 // lanes taking consecutive items, so a lane without items works on another's.
 // Every lane of the wavefront calls it.  Of `parts` wavefronts that bring the
-// same counts, number `part` takes every parts-th 64 items.
-template <class F>
-__device__ __forceinline__ void wave_items(uint64_t count, uint32_t part, uint32_t parts, F f) {
+// same counts, number `part` takes every parts-th 64 items.  T: a type that
+// holds 64 lanes' items (32-bit shuffles cost half of 64-bit ones).
+template <class T, class F>
+__device__ __forceinline__ void wave_items(T count, uint32_t part, uint32_t parts, F f) {
   const uint32_t lane = threadIdx.x & 63u;
-  unsigned long long incl = count;               // items of lanes 0..i
+  T incl = count;                                // items of lanes 0..i
 #pragma unroll
   for (uint32_t d = 1u; d < 64u; d <<= 1) {
-    const unsigned long long v = __shfl_up(incl, d);
+    const T v = __shfl_up(incl, d);
     if (lane >= d) incl += v;
   }
-  const unsigned long long total = __shfl(incl, 63), excl = incl - count;
-  for (unsigned long long base = 64ull * part; base < total; base += 64ull * parts) {
-    const unsigned long long t = base + lane;
+  const T total = __shfl(incl, 63), excl = incl - count;
+  for (T base = 64u * (T)part; base < total; base += 64u * (T)parts) {
+    const T t = base + lane;
     uint32_t s = 0u;                             // the first lane whose items reach past t
 #pragma unroll
     for (uint32_t d = 32u; d >= 1u; d >>= 1)
       if (__shfl(incl, (int)(s + d - 1u)) <= t) s += d;
-    const unsigned long long first = __shfl(excl, (int)min(s, 63u));
-    if (t < total) f(s, (uint64_t)(t - first));
+    const T first = __shfl(excl, (int)min(s, 63u));
+    if (t < total) f(s, t - first);
   }
 }
 

@@ -42,6 +42,11 @@ struct DevDir {
   const uint32_t *R;     // R[j / ratio] = ISA[j] for text positions j % ratio == 0
   const uint32_t *sa;    // full SA (n + 1), or NULL: see fmi_index_expand
   const uint32_t *isa;   // full ISA (n + 1), or NULL
+  // Row contexts (n + 1), or NULL: the 16 text bases that LF steps from the
+  // row's suffix would meet (X[q-1], X[q-2], ... for the BWT of X), 2 bits
+  // each, 0 past the text's start.  The rows of an interval are neighbours
+  // here, so one line tells for 16 of them how any 16 bases extend them.
+  const uint32_t *ctx;
   uint32_t C[4];         // # symbols < b
   uint32_t dollar;       // row holding '$'
   uint32_t dollar_blk;   // dollar / 192

@@ -72,6 +72,8 @@ hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, co
 // Full SA / ISA of one direction from its samples (sa, isa: n + 1 entries).
 hipError_t launch_expand(const DevDir &D, uint32_t n, uint32_t ratio, uint32_t *sa, uint32_t *isa,
                          hipStream_t s);
+// The row contexts of one direction (n + 1 words) of an expanded index.
+hipError_t launch_row_contexts(const DevIndex &ix, uint32_t dsel, uint32_t *ctx, hipStream_t s);
 // X packed 2 bits per base ((n + 15) / 16 words) from the backward direction.
 hipError_t launch_kmer_table(const DevDir &D, uint32_t n, uint32_t k, uint64_t *out, hipStream_t s);
 hipError_t launch_pack_text(const DevDir &D, uint32_t n, const uint32_t *isa, uint32_t *text,

@@ -1295,6 +1295,7 @@ struct LocateParams {
 // thread per (interval, slot of cap) launched cap threads with a 64-bit
 // division each for the one row most intervals have.  grid.y: the wavefronts
 // that share one set of 64 intervals (item_parts).
+template <class T>
 __global__ __launch_bounds__(256) void locate_kernel(LocateParams P) {
   const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t wave0 = g & ~63ull;             // the wavefront's first interval
@@ -1308,7 +1309,7 @@ __global__ __launch_bounds__(256) void locate_kernel(LocateParams P) {
     if (blockIdx.y == 0u) P.nrows[g] = rows;
   }
   const DevDir &D = dir_of(P.ix, P.dsel);
-  wave_items(rows, blockIdx.y, gridDim.y, [&](uint32_t s, uint64_t j) {
+  wave_items<T>(rows, blockIdx.y, gridDim.y, [&](uint32_t s, T j) {
     const uint64_t iv = wave0 + s;
     P.pos[iv * P.cap + j] =
         sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)((uint64_t)P.k[iv * P.stride] + j));
@@ -1374,6 +1375,15 @@ __global__ __launch_bounds__(256) void expand_walk_kernel(DevDir D, uint32_t n, 
     row = pick4(D.C, c) + occ_blk(B, D.dollar_blk, D.dollar_off, j, c, o) + 1u;
     --pos;
   }
+}
+
+// The 16 text bases before every row's suffix, in LF order (DevDir::ctx).
+__global__ __launch_bounds__(256) void row_context_kernel(DevIndex ix, uint32_t dsel,
+                                                          uint32_t *ctx) {
+  const uint32_t *sa = dsel ? ix.d[1].sa : ix.d[0].sa;
+  for (uint64_t r = (uint64_t)blockIdx.x * 256u + threadIdx.x; r <= ix.n;
+       r += (uint64_t)gridDim.x * 256u)
+    ctx[r] = sa[r] ? (uint32_t)text_window32(ix, dsel, sa[r]) : 0u;   // none before X[0]
 }
 
 // X[j] is the BWT symbol of the row of suffix j + 1.
@@ -1453,11 +1463,12 @@ __device__ __forceinline__ void resolve_row(const ResolveParams &P, uint64_t slo
 // wavefront's 64 slots are then shared out among its lanes (wave_items): most
 // slots hold no record or one.  A thread per (slot, record of cap, row of
 // row_cap) launched 90 M threads for 700 K reads at cap 16 and row_cap 4.
+template <class T>
 __global__ __launch_bounds__(256) void resolve_kernel(ResolveParams P) {
   const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t wave0 = g & ~63ull;             // the wavefront's first slot
-  const uint64_t stored = g < P.nslots ? min(P.counts[g], P.cap) : 0u;
-  wave_items(stored * P.row_cap, blockIdx.y, gridDim.y, [&](uint32_t s, uint64_t t) {
+  const T stored = g < P.nslots ? min(P.counts[g], P.cap) : 0u;
+  wave_items<T>(stored * P.row_cap, blockIdx.y, gridDim.y, [&](uint32_t s, T t) {
     resolve_row(P, wave0 + s, t / P.row_cap, (uint32_t)(t % P.row_cap));
   });
 }
@@ -1789,12 +1800,13 @@ hipError_t launch_vhelper(const DevIndex &ix, bool mm_only, uint32_t strand_mask
 }
 
 // Wavefronts per 64 lanes of wave_items: one where there are enough to fill
-// the device (256 CUs of 32), else as many as fill it, at most one per 64 items
-// the 64 lanes can bring (a few wide intervals are rows enough for all).
+// the device twice (256 CUs of 32), else as many as do, at most one per 64
+// items the 64 lanes can bring.  Few wide intervals need them: 1 M rows of one
+// interval take 12 us, as a thread per row did, where 8192 took 18.
 static uint32_t item_parts(uint64_t lanes, uint64_t items_per_lane) {
   const uint64_t waves = (lanes + 63) / 64;
-  const uint64_t fill = std::max<uint64_t>(8192 / std::max<uint64_t>(waves, 1), 1);
-  return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(fill, items_per_lane), 8192);
+  const uint64_t fill = std::max<uint64_t>(16384 / std::max<uint64_t>(waves, 1), 1);
+  return (uint32_t)std::min<uint64_t>(fill, items_per_lane);
 }
 
 hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, const int64_t *l,
@@ -1803,8 +1815,9 @@ hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, co
   LocateParams P{ix, dsel, nintervals, cap, stride, k, l, pos, nrows};
   const uint64_t grid = ((uint64_t)nintervals + 255) / 256;
   if (grid == 0 || cap == 0) return hipSuccess;
-  hipLaunchKernelGGL(locate_kernel, dim3((uint32_t)grid, item_parts(nintervals, cap)), dim3(256), 0,
-                     s, P);
+  const dim3 g((uint32_t)grid, item_parts(nintervals, cap));
+  if (cap < (1u << 26)) hipLaunchKernelGGL(locate_kernel<uint32_t>, g, dim3(256), 0, s, P);
+  else hipLaunchKernelGGL(locate_kernel<unsigned long long>, g, dim3(256), 0, s, P);
   return hipGetLastError();
 }
 
@@ -1820,6 +1833,12 @@ hipError_t launch_kmer_table(const DevDir &D, uint32_t n, uint32_t k, uint64_t *
   const uint64_t count = 1ull << (2 * k);
   const uint64_t grid = std::min<uint64_t>((count + 255) / 256, 65536ull);
   hipLaunchKernelGGL(kmer_table_kernel, dim3((uint32_t)grid), dim3(256), 0, s, D, n, k, count, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_row_contexts(const DevIndex &ix, uint32_t dsel, uint32_t *ctx, hipStream_t s) {
+  const uint64_t grid = std::min<uint64_t>(((uint64_t)ix.n + 256) / 256, 65536ull);
+  hipLaunchKernelGGL(row_context_kernel, dim3((uint32_t)grid), dim3(256), 0, s, ix, dsel, ctx);
   return hipGetLastError();
 }
 
@@ -1850,9 +1869,10 @@ hipError_t launch_resolve(const DevIndex &ix, const fmi_hit *hits, const uint32_
                   record_len, chrom, coord};
   const uint64_t grid = (2ull * nreads + 255) / 256;
   if (grid == 0 || cap == 0 || row_cap == 0) return hipSuccess;
-  hipLaunchKernelGGL(resolve_kernel,
-                     dim3((uint32_t)grid, item_parts(2ull * nreads, (uint64_t)cap * row_cap)),
-                     dim3(256), 0, s, P);
+  const uint64_t per_slot = (uint64_t)cap * row_cap;
+  const dim3 g((uint32_t)grid, item_parts(2ull * nreads, per_slot));
+  if (per_slot < (1u << 26)) hipLaunchKernelGGL(resolve_kernel<uint32_t>, g, dim3(256), 0, s, P);
+  else hipLaunchKernelGGL(resolve_kernel<unsigned long long>, g, dim3(256), 0, s, P);
   return hipGetLastError();
 }
 

@@ -12,6 +12,7 @@
 //      with len = seq_end - seq_start (one short, bwt.c:1214), region record.
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstring>   // rocprim's texture_cache_iterator uses memset
 
 #include <rocprim/rocprim.hpp>
@@ -25,6 +26,7 @@
 #include "fmi_index.h"
 #include "fmi_internal.h"
 #include "fmi_vhelper.h"
+#include "fmi_window.h"
 
 namespace fmi {
 
@@ -52,6 +54,29 @@ __device__ __forceinline__ uint64_t owner(const uint64_t *base, uint64_t n, uint
     else hi = mid;
   }
   return lo;
+}
+
+// owner for the lanes of a wavefront that hold consecutive g's (lane i:
+// g0 + i, g0 + i < total): the owners of the first and the last by 64 probes a
+// round of the whole wavefront, then a lane's own among those between them.
+// Every lane of the wavefront calls it; lanes past total get any answer.
+__device__ __forceinline__ uint64_t wave_owner(const uint64_t *base, uint64_t n, uint64_t total,
+                                               uint64_t g0) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint64_t ends[2];
+#pragma unroll
+  for (uint32_t e = 0; e < 2u; ++e) {
+    const uint64_t g = e ? min(g0 + 63u, total - 1u) : g0;
+    uint64_t lo = e ? ends[0] : 0u, hi = n;
+    while (hi - lo > 1u) {
+      const uint64_t step = (hi - lo + 63u) / 64u, idx = lo + lane * step;
+      const uint64_t yes = __ballot(lane == 0u || (idx < hi && base[idx] <= g));
+      lo += (63u - (uint32_t)__builtin_clzll(yes)) * step;
+      hi = min(lo + step, hi);
+    }
+    ends[e] = lo;
+  }
+  return ends[0] + owner(base + ends[0], ends[1] - ends[0] + 1u, g0 + lane);
 }
 
 struct SeedParams {
@@ -240,6 +265,25 @@ struct InexactParams {
   uint8_t *status;
 };
 
+// What a record says of its error, as the list stores it (no error fields
+// without an error): final_pos where it is assigned, the change of the length
+// and final_err (bwt.c:1499-1530).
+__device__ __forceinline__ void record_errors(const VhRec &r, uint32_t type, int32_t len,
+                                              int32_t &final_pos, int32_t &dl,
+                                              int32_t &final_err) {
+  const uint32_t error = r.nmm ? r.kind : 0u;
+  const int32_t pos = r.nmm ? r.err_pos : 0;
+  dl = error == FMI_DELETION ? -1 : (error == FMI_INSERTION ? 1 : 0);
+  if (error == FMI_DELETION || pos == 0 || pos == len - 1) {
+    final_pos = type ? pos : len - 1 - pos;
+  } else if (error == FMI_INSERTION) {
+    if (type) final_pos = r.dir ? pos : pos + 1;
+    else final_pos = r.dir ? len - pos : len - pos - 1;
+  }
+  // -1 mismatch, SEED_INSERTION 1, SEED_DELETION 2
+  final_err = error == FMI_MISMATCH ? -1 : (error == FMI_DELETION ? 1 : 2);
+}
+
 // Regions of one strand's records (bwt.c:1490-1588), in record order.
 struct RegionSink {
   const InexactParams *P;
@@ -248,31 +292,25 @@ struct RegionSink {
   int32_t start, len;
   int32_t *final_pos;
   uint8_t st;
-  __device__ void add(const VhRec &r) {
+  __device__ __forceinline__ void add(const VhRec &r) {
+    add(r, (type ? r.dir : !r.dir) ? 1u : 0u, WinIv{r.k, kWinNone, r.l - r.k + 1u});
+  }
+  // The record's interval on direction dsel: its first row, or that row's
+  // suffix, and its rows.
+  __device__ __forceinline__ void add(const VhRec &r, uint32_t dsel, const WinIv &iv) {
     if (nrec++ >= P->rec_cap) { st |= 1; return; }   // the reference's list holds 20000
-    // a record as the list stores it: no error fields without an error
-    const uint32_t error = r.nmm ? r.kind : 0u;
-    const int32_t pos = r.nmm ? r.err_pos : 0;
-    int64_t len_calc = len;
-    if (error == FMI_DELETION) len_calc--;
-    else if (error == FMI_INSERTION) len_calc++;
-    if (error == FMI_DELETION || pos == 0 || pos == len - 1) {
-      *final_pos = type ? pos : len - 1 - pos;
-    } else if (error == FMI_INSERTION) {
-      if (type) *final_pos = r.dir ? pos : pos + 1;
-      else *final_pos = r.dir ? len - pos : len - pos - 1;
-    }
-    int32_t final_err = error == FMI_MISMATCH ? -1 : (error == FMI_DELETION ? 1 : 2);
-    final_err += start;                    // -1 mismatch, SEED_INSERTION 1, SEED_DELETION 2
-    const int64_t k = r.k, l = r.l;
-    const int64_t l0 = (l - k + 1) < 50 ? l : k + 1;   // bwt.c:1539-1547
-    const uint32_t direction = type ? r.dir : !r.dir;
+    int32_t dl, final_err;
+    record_errors(r, type, len, *final_pos, dl, final_err);
+    final_err += start;
+    const int64_t len_calc = (int64_t)len + dl;
+    const DevDir &D = dir_of(P->ix, dsel);
+    const uint32_t rows = iv.rows < 50u ? iv.rows : 2u;    // bwt.c:1539-1547
+    const uint32_t k = iv.q != kWinNone && rows > 1u ? D.isa[iv.q] : iv.k;
     const uint64_t size_sa = (uint64_t)P->ix.n + 1;
-    for (int64_t j = k; j <= l0; ++j) {
-      const uint64_t key =
-          direction ? size_sa - sa_value(P->ix.d[1], P->ix.ratio, P->ix.n, (uint32_t)j) -
-                          (uint64_t)len_calc - 1
-                    : sa_value(P->ix.d[0], P->ix.ratio, P->ix.n, (uint32_t)j);
+    for (uint32_t j = 0; j < rows; ++j) {
+      const uint64_t sa = iv.q != kWinNone && j == 0u ? iv.q
+                                                      : sa_value(D, P->ix.ratio, P->ix.n, k + j);
+      const uint64_t key = dsel ? size_sa - sa - (uint64_t)len_calc - 1 : sa;
       uint64_t lo = 0, size = P->kcount;    // binsearch, search/io.h:43-64
       while (size > 0) {
         const uint64_t w = size / 2;
@@ -299,27 +337,233 @@ struct RegionSink {
   }
 };
 
+// A lane's m regions at out deduplicated within 10 bp (bwt.c:1593-1615), the
+// mark kept in pad[0], and handed over from the last to the first
+// (bwt.c:1616-1626), in place; returns how many stay.
+__device__ __forceinline__ uint32_t dedup_list(fmi_inexact_region *out, uint32_t m) {
+  for (int32_t a1 = (int32_t)m - 1; a1 >= 1; --a1) {
+    if (out[a1].pad[0]) continue;
+    const uint64_t s1 = out[a1].start;
+    const uint32_t c1 = out[a1].chrom_idx;
+    for (int32_t a2 = a1 - 1; a2 >= 0; --a2) {
+      const int32_t d = (int32_t)(uint32_t)(s1 - out[a2].start);
+      const int64_t dist = d < 0 ? -(int64_t)d : (int64_t)d;
+      if (c1 == out[a2].chrom_idx && dist < 10 && !out[a2].pad[0]) out[a2].pad[0] = 1;
+    }
+  }
+  uint32_t kept = 0;
+  for (uint32_t i = 0; i < m; ++i) {
+    if (out[i].pad[0]) continue;
+    const fmi_inexact_region R = out[i];
+    out[kept++] = R;
+  }
+  for (uint32_t i = 0; i < kept / 2; ++i) {
+    const fmi_inexact_region x = out[i];
+    out[i] = out[kept - 1 - i];
+    out[kept - 1 - i] = x;
+  }
+  return kept;
+}
+
+// ---- windows by row contexts: the records of a window and strand are kept
+// (16 bytes each) and become regions together, one region a lane.
+constexpr uint32_t kWinRecs = 64;      // records and rows a wavefront takes at once
+constexpr uint8_t kWinRedo = 0x80;     // status of a window with more of them
+
+// A kept record: x the first row, or (known) that row's suffix; y its rows (as
+// many as it gives regions for) | known << 8 | direction << 9 | (len_calc - len
+// + 1) << 10; z pos_err, w type_err.
+struct RecordSink {
+  uint4 *list;
+  uint32_t n, total, nrec, rec_cap, type;
+  int32_t start, len;
+  int32_t final_pos;
+  uint8_t st;
+  __device__ __forceinline__ void add(const VhRec &r, uint32_t dsel, const WinIv &iv) {
+    if (nrec++ >= rec_cap) { st |= 1; return; }      // the reference's list holds 20000
+    int32_t dl, final_err;
+    record_errors(r, type, len, final_pos, dl, final_err);
+    const uint32_t rows = iv.rows < 50u ? iv.rows : 2u;        // bwt.c:1539-1547
+    const bool known = iv.q != kWinNone;
+    const uint4 v = make_uint4(known ? iv.q : iv.k,
+                               rows | (known ? 1u << 8 : 0u) | (dsel << 9) |
+                                   ((uint32_t)(dl + 1) << 10),
+                               (uint32_t)final_pos, (uint32_t)(final_err + start));
+    if (n < kWinRecs) list[n] = v;
+    n++;
+    total += rows;
+  }
+};
+
+// The region of row j of a kept record: its start and contig, or contig 0
+// where the occurrence crosses a contig's end.
+__device__ __forceinline__ void record_region(const InexactParams &P, const uint4 &rec, uint32_t j,
+                                              int32_t len, uint64_t &start, uint32_t &chrom) {
+  const uint32_t dsel = (rec.y >> 9) & 1u, rows = rec.y & 0xFFu;
+  const bool known = ((rec.y >> 8) & 1u) != 0u;
+  const DevDir &D = dir_of(P.ix, dsel);
+  const uint64_t len_calc = (uint64_t)((int64_t)len + (int64_t)((rec.y >> 10) & 3u) - 1);
+  uint32_t sa;
+  if (known && j == 0u) sa = rec.x;
+  else sa = D.sa[(known && rows > 1u ? D.isa[rec.x] : rec.x) + j];
+  const uint64_t key = dsel ? (uint64_t)P.ix.n + 1u - sa - len_calc - 1u : (uint64_t)sa;
+  uint64_t lo = 0, size = P.kcount;        // binsearch, search/io.h:43-64
+  while (size > 0) {
+    const uint64_t w = size / 2;
+    if (P.koff[lo + w] <= key) { lo += w + 1; size -= w + 1; }
+    else size = w;
+  }
+  chrom = 0u;
+  start = 0ull;
+  if (lo >= 1 && key + len_calc <= P.koff[lo]) {
+    chrom = (uint32_t)lo;
+    start = P.kstart[lo - 1] + (key - P.koff[lo - 1]) + 1;
+  }
+}
+
+struct WinOf {                       // what a window's regions have in common
+  uint32_t read, aux_s, aux_e, seq_len, seed_id, strand;
+  int32_t len;
+};
+
+// A region as three 16-byte pieces.
+__device__ __forceinline__ void store_region(fmi_inexact_region *dst, const WinOf &w,
+                                             uint64_t start, uint32_t chrom, const uint4 &rec,
+                                             uint32_t mark) {
+  const uint64_t end = start + (uint64_t)(int64_t)w.len - 1u;
+  uint4 *d = reinterpret_cast<uint4 *>(dst);
+  d[0] = make_uint4((uint32_t)start, (uint32_t)(start >> 32), (uint32_t)end, (uint32_t)(end >> 32));
+  d[1] = make_uint4(chrom, w.read, w.aux_s | (w.aux_e << 16), w.seq_len | (w.seed_id << 16));
+  d[2] = make_uint4(rec.z, rec.w, w.strand | (mark << 8), 0u);
+}
+static_assert(sizeof(fmi_inexact_region) == 48 && offsetof(fmi_inexact_region, chrom_idx) == 16 &&
+                  offsetof(fmi_inexact_region, seq_start) == 24 &&
+                  offsetof(fmi_inexact_region, pos_err) == 32 &&
+                  offsetof(fmi_inexact_region, strand) == 40,
+              "fmi_inexact_region layout");
+
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int src) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, src);
+}
+
+// Turns every lane's kept records (n of them with `total` rows, at most
+// kWinRecs; n = 0: none) into its slot's list: the regions in record and row
+// order, the dedup, the hand-over from the last to the first.  A lane with one
+// row does it alone, all such lanes together; any other list is taken by the
+// whole wavefront, a row a lane, and leaves the registers once.  Slots past
+// the list hold what the list held there before the hand-over, marked in
+// pad[0] where it was dropped.  Every lane of the wavefront calls it; returns
+// the regions kept.
+__device__ __forceinline__ uint32_t regions_of(const InexactParams &P, const RecordSink &S,
+                                               uint32_t n, const WinOf &w,
+                                               fmi_inexact_region *out, uint8_t &st) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t kept = 0u;
+  if (n == 1u && S.total == 1u) {
+    uint64_t start;
+    uint32_t chrom;
+    const uint4 rec = S.list[0];
+    record_region(P, rec, 0u, w.len, start, chrom);
+    if (chrom) {
+      store_region(out, w, start, chrom, rec, 0u);
+      kept = 1u;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");   // the lists, read by other lanes
+  for (uint64_t todo = __ballot(n > 0u && S.total > 1u); todo; todo &= todo - 1ull) {
+    const int src = (int)__builtin_ctzll(todo);
+    const uint4 *list = reinterpret_cast<const uint4 *>(
+        ((uint64_t)lane_value((uint32_t)((uintptr_t)S.list >> 32), src) << 32) |
+        lane_value((uint32_t)(uintptr_t)S.list, src));
+    fmi_inexact_region *dst = reinterpret_cast<fmi_inexact_region *>(
+        ((uint64_t)lane_value((uint32_t)((uintptr_t)out >> 32), src) << 32) |
+        lane_value((uint32_t)(uintptr_t)out, src));
+    const uint32_t nr = lane_value(n, src);
+    const WinOf ws{lane_value(w.read, src),    lane_value(w.aux_s, src),
+                   lane_value(w.aux_e, src),   lane_value(w.seq_len, src),
+                   lane_value(w.seed_id, src), lane_value(w.strand, src),
+                   (int32_t)lane_value((uint32_t)w.len, src)};
+    uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+    if (lane < nr) rec = list[lane];
+    uint32_t incl = rec.y & 0xFFu;             // rows of records 0..lane
+    const uint32_t own = incl;
+#pragma unroll
+    for (uint32_t d = 1u; d < 64u; d <<= 1) {
+      const uint32_t v = __shfl_up(incl, d);
+      if (lane >= d) incl += v;
+    }
+    uint32_t ri = 0u;                          // the record of row `lane`
+#pragma unroll
+    for (uint32_t d = 32u; d >= 1u; d >>= 1)
+      if (__shfl(incl, (int)(ri + d - 1u)) <= lane) ri += d;
+    const uint32_t rows = lane_value(incl, 63);
+    const int at = (int)min(ri, 63u);
+    const uint32_t first = __shfl(incl - own, at);
+    const uint4 mine = make_uint4(__shfl(rec.x, at), __shfl(rec.y, at), __shfl(rec.z, at),
+                                  __shfl(rec.w, at));
+    uint64_t start = 0ull;
+    uint32_t chrom = 0u;
+    if (lane < rows) record_region(P, mine, lane - first, ws.len, start, chrom);
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint64_t valid = __ballot(chrom != 0u);
+    const uint32_t rank = (uint32_t)__popcll(valid & below);
+    const bool in = chrom != 0u && rank < P.region_cap;
+    const uint64_t all = __ballot(in);
+    // within 10 bp (bwt.c:1593-1615): from the last region to the first, one
+    // not yet dropped drops every earlier one of its chromosome that near
+    bool gone = !in;
+    for (uint64_t left = all; left;) {
+      const int a = 63 - (int)__builtin_clzll(left);
+      left ^= 1ull << a;
+      if (!((__ballot(!gone) >> a) & 1ull)) continue;
+      const uint64_t s1 = ((uint64_t)lane_value((uint32_t)(start >> 32), a) << 32) |
+                          lane_value((uint32_t)start, a);
+      const int32_t d = (int32_t)(uint32_t)(s1 - start);
+      const int64_t dist = d < 0 ? -(int64_t)d : (int64_t)d;
+      if ((int)lane < a && lane_value(chrom, a) == chrom && dist < 10) gone = true;
+    }
+    const uint64_t stay = __ballot(!gone);
+    const uint32_t k = (uint32_t)__popcll(stay);
+    if (in && rank >= k) store_region(dst + rank, ws, start, chrom, mine, gone ? 1u : 0u);
+    if (!gone)
+      store_region(dst + (k - 1u - (uint32_t)__popcll(stay & below)), ws, start, chrom, mine, 0u);
+    if ((int)lane == src) {
+      kept = k;
+      if ((uint32_t)__popcll(valid) > P.region_cap) st |= 2;
+    }
+  }
+  return kept;
+}
+
 // Held to 128 VGPRs for 4 waves per SIMD (157 unbounded: 3 waves): a lane's
 // windows are chains of dependent loads, so a fourth wave to hide them pays
 // for the few registers spilled (83.3 -> 76.7 ms on 8 M windows of 18 bases
 // over 64 Mbp).  REGS (seed_size <= 32): the window's bases are packed into
 // registers once (vh_regs) for both strands, so the helper's LF steps and
 // comparisons read no read bytes from memory.
-template <bool REGS>
+// REDO: only the windows that context_seed_kernel left (status kWinRedo).
+template <bool REGS, bool REDO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void inexact_seed_kernel(InexactParams P) {
+  __shared__ uint32_t words[REDO ? kWinWords * 256u : 1u];
   const uint64_t lane = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   uint2 *vb = P.vscratch + lane * (uint64_t)(P.seed_size + 3);
-  for (uint64_t g = lane; g < P.nwin; g += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t rd = owner(P.win_base, P.nreads, g);
+  const uint64_t wlane = lane & 63u;
+  // a wavefront's lanes take consecutive windows and go on together
+  for (uint64_t g0 = lane - wlane; g0 < P.nwin; g0 += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t rd0 = wave_owner(P.win_base, P.nreads, P.nwin, g0);
+    const bool mine = g0 + wlane < P.nwin;
+    const uint64_t g = mine ? g0 + wlane : P.nwin - 1u, rd = mine ? rd0 : P.nreads - 1u;
     const uint64_t off = P.offsets[rd];
     const int32_t len = (int32_t)(P.offsets[rd + 1] - off);
     const int32_t w = (int32_t)(g - P.win_base[rd]);
     const int32_t num_seeds = len / (int32_t)P.seed_size;
     const int32_t ws = w * (int32_t)P.seed_size;
     const int32_t we = w < num_seeds ? ws + (int32_t)P.seed_size - 1 : len - 1;
+    if (!mine || (REDO && P.status[2 * g] != kWinRedo)) continue;
+    const bool run = we - ws >= 2;
     int32_t final_pos = 0;
     VhRegs WR{0ull, 0u, ws};
-    if (REGS && we - ws >= 2) WR = vh_regs(P.reads + off, ws, (uint32_t)(we - ws + 1));
+    if (REGS && run) WR = vh_regs(P.reads + off, ws, (uint32_t)(we - ws + 1));
     for (uint32_t s = 0; s < 2; ++s) {
       const uint32_t type = 1u - s;          // bwt.c:1460: type 1 (+) first
       const uint64_t slot = 2 * g + s;
@@ -327,38 +571,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
                    type ? (uint32_t)ws : (uint32_t)(len - we - 1),
                    type ? (uint32_t)we : (uint32_t)(len - ws - 1), (uint32_t)len, (uint32_t)w,
                    ws, we - ws + 1, &final_pos, 0};
-      if (we - ws >= 2) {
-        if (REGS) vh_run(P.ix, WR, ws, we, s, 0u, vb, S);
+      if (run) {
+        if (REDO) win_run(P.ix, WR, ws, we, s, vb, words + threadIdx.x, S);
+        else if (REGS) vh_run(P.ix, WR, ws, we, s, 0u, vb, S);
         else vh_run(P.ix, VhBytes{P.reads + off}, ws, we, s, 0u, vb, S);
       }
-      fmi_inexact_region *out = S.out;
-      const uint32_t m = S.m;
-      // dedup within 10 bp (bwt.c:1593-1615), the mark kept in pad[0]
-      for (int32_t a1 = (int32_t)m - 1; a1 >= 1; --a1) {
-        if (out[a1].pad[0]) continue;
-        const uint64_t s1 = out[a1].start;
-        const uint32_t c1 = out[a1].chrom_idx;
-        for (int32_t a2 = a1 - 1; a2 >= 0; --a2) {
-          const int32_t d = (int32_t)(uint32_t)(s1 - out[a2].start);
-          const int64_t dist = d < 0 ? -(int64_t)d : (int64_t)d;
-          if (c1 == out[a2].chrom_idx && dist < 10 && !out[a2].pad[0]) out[a2].pad[0] = 1;
-        }
-      }
-      // kept regions, handed over from the last to the first (bwt.c:1616-1626)
-      uint32_t kept = 0;
-      for (uint32_t i = 0; i < m; ++i) {
-        if (out[i].pad[0]) continue;
-        const fmi_inexact_region R = out[i];
-        out[kept++] = R;
-      }
-      for (uint32_t i = 0; i < kept / 2; ++i) {
-        const fmi_inexact_region x = out[i];
-        out[i] = out[kept - 1 - i];
-        out[kept - 1 - i] = x;
-      }
-      P.nreg[slot] = kept;
+      P.nreg[slot] = dedup_list(S.out, S.m);
       P.status[slot] = S.st;
     }
+  }
+}
+
+// The same windows on an index with row contexts, seed_size <= kWinMax: they go
+// by their rows' contexts and the k-mer table instead of an LF step per base
+// and branch (win_run), and their records become regions a wavefront at a time
+// (regions_of).  A window with more than kWinRecs records or rows on a
+// strand is left to inexact_seed_kernel.  vscratch: per lane seed_size + 3
+// intervals and kWinRecs records.  At 4 waves per SIMD 31 registers spill;
+// 3 waves (none) took 8.6 ms where 4 took 7.6, 5 waves 10.0 (before the loops
+// were parted).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void context_seed_kernel(InexactParams P) {
+  __shared__ uint32_t words[kWinWords * 256u];
+  const uint64_t lane = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t lanes = (uint64_t)gridDim.x * blockDim.x;
+  uint4 *list = reinterpret_cast<uint4 *>(P.vscratch) + lane * kWinRecs;
+  uint2 *vb = reinterpret_cast<uint2 *>(reinterpret_cast<uint4 *>(P.vscratch) + lanes * kWinRecs) +
+              lane * (uint64_t)(P.seed_size + 3);
+  const uint64_t wlane = lane & 63u;
+  // a wavefront's lanes take consecutive windows and go on together
+  for (uint64_t g0 = lane - wlane; g0 < P.nwin; g0 += lanes) {
+    const uint64_t rd0 = wave_owner(P.win_base, P.nreads, P.nwin, g0);
+    const bool mine = g0 + wlane < P.nwin;
+    const uint64_t g = mine ? g0 + wlane : P.nwin - 1u, rd = mine ? rd0 : P.nreads - 1u;
+    const uint64_t off = P.offsets[rd];
+    const int32_t len = (int32_t)(P.offsets[rd + 1] - off);
+    const int32_t w = (int32_t)(g - P.win_base[rd]);
+    const int32_t num_seeds = len / (int32_t)P.seed_size;
+    const int32_t ws = w * (int32_t)P.seed_size;
+    const int32_t we = w < num_seeds ? ws + (int32_t)P.seed_size - 1 : len - 1;
+    const bool run = mine && we - ws >= 2;
+    int32_t final_pos = 0;
+    bool redo = false;
+    VhRegs WR{0ull, 0u, ws};
+    if (run) WR = vh_regs(P.reads + off, ws, (uint32_t)(we - ws + 1));
+    for (uint32_t s = 0; s < 2; ++s) {
+      const uint32_t type = 1u - s;          // bwt.c:1460: type 1 (+) first
+      const uint64_t slot = 2 * g + s;
+      RecordSink S{list, 0u, 0u, 0u, P.rec_cap, type, ws, we - ws + 1,
+                   final_pos, 0};
+      if (run) win_run(P.ix, WR, ws, we, s, vb, words + threadIdx.x, S);
+      final_pos = S.final_pos;
+      redo |= S.n > kWinRecs || S.total > kWinRecs;
+      const WinOf wo{(uint32_t)rd,
+                     (uint32_t)(uint16_t)(type ? ws : len - we - 1),
+                     (uint32_t)(uint16_t)(type ? we : len - ws - 1),
+                     (uint32_t)(uint16_t)len,
+                     (uint32_t)(uint16_t)w,
+                     s,
+                     we - ws + 1};
+      uint8_t st = S.st;
+      const uint32_t kept =
+          regions_of(P, S, redo ? 0u : S.n, wo, P.out + slot * P.region_cap, st);
+      if (mine) {
+        P.nreg[slot] = kept;
+        P.status[slot] = st;
+      }
+    }
+    if (redo) P.status[2 * g] = kWinRedo;
   }
 }
 
@@ -490,13 +769,25 @@ int map_inexact_seeds(const fmi_index *ix, const uint8_t *reads, const uint64_t 
     const uint64_t per = (uint64_t)(seed_size + 3) * sizeof(uint2);
     const uint64_t max_lanes = std::min<uint64_t>(1ull << 19, ((1ull << 30) / per) / 256 * 256);
     if (lanes > max_lanes) lanes = max_lanes;
-    SEED_TRY(hipMalloc(&vscr, lanes * per));
+    // windows by context: as many lanes as are resident (4 waves per SIMD),
+    // each with its record list too
+    const bool ctx = seed_size <= kWinMax && ix->dev.d[0].ctx;
+    const uint64_t ctx_lanes = std::min<uint64_t>(lanes, 1ull << 18);
+    SEED_TRY(hipMalloc(&vscr, std::max<uint64_t>(
+                                  lanes * per, ctx ? ctx_lanes * (per + kWinRecs * 16ull) : 0ull)));
     InexactParams P{ix->dev, reads, offsets, base, nwin, nreads, seed_size, rec_cap, region_cap,
                     ix->d_koffset, ix->d_kstart, (uint32_t)ix->kstart.size(), vscr, regions,
                     nregions, status};
     // windows are at most seed_size bases (the remainder window is shorter)
-    if (seed_size <= 32u) inexact_seed_kernel<true><<<dim3((uint32_t)(lanes / 256)), 256, 0, s>>>(P);
-    else inexact_seed_kernel<false><<<dim3((uint32_t)(lanes / 256)), 256, 0, s>>>(P);
+    const dim3 grid((uint32_t)(lanes / 256));
+    if (ctx) {
+      context_seed_kernel<<<dim3((uint32_t)(ctx_lanes / 256)), 256, 0, s>>>(P);
+      inexact_seed_kernel<true, true><<<grid, 256, 0, s>>>(P);
+    } else if (seed_size <= 32u) {
+      inexact_seed_kernel<true, false><<<grid, 256, 0, s>>>(P);
+    } else {
+      inexact_seed_kernel<false, false><<<grid, 256, 0, s>>>(P);
+    }
     SEED_TRY(hipGetLastError());
   }
 done:

@@ -139,7 +139,12 @@ void fmi_index_free(fmi_index *ix);
  * searches then continue every single-row interval by comparing the read
  * with the text at that row's suffix (one SA read to enter, one ISA read per
  * record) instead of one occurrence-block load per base; the records are
- * the same.  No reference counterpart (it trades HBM for dependent loads). */
+ * the same.  Where at least twice their size is free after that, the row
+ * contexts of both directions are kept too (the 16 text bases before every
+ * row's suffix, 8 bytes per base; 3.1 Gbp: 25 GB): several searches then tell
+ * from one line how any bases extend the rows of an interval.  Results do not
+ * depend on them.  No reference counterpart (it trades HBM for dependent
+ * loads). */
 int fmi_index_expand(fmi_index *ix);
 /* A table of the interval of every string of k bases in each direction
  * (4^k entries of 8 bytes per direction: k = 12 takes 128 MiB, k = 13 512
@@ -169,7 +174,8 @@ int fmi_index_get_samples(const fmi_index *ix, int forward, uint32_t *S, uint32_
 uint64_t fmi_index_size_sa(const fmi_index *ix);
 uint32_t fmi_index_sa_ratio(const fmi_index *ix);
 /* Bytes of the device copy by part: out[0] occurrence blocks and S / R
- * samples of both directions, out[1] the full SA / ISA and 2-bit text
+ * samples of both directions, out[1] the full SA / ISA, 2-bit text and row
+ * contexts
  * (fmi_index_expand), out[2] the k-mer tables (fmi_index_kmer_table). */
 int fmi_index_device_layout(const fmi_index *ix, uint64_t *out);
 /* Bytes the device copy occupies. */

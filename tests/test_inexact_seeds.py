@@ -152,3 +152,65 @@ def test_gpu_inexact_seeds_vs_oracle(gpu_engine, expanded):
                 assert got.tobytes() == regs.tobytes(), (seed_size, i, t)
     batch.free()
     ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,kmer", [(100_000, 0), (100_000, 6), (100_000, 8), (100_000, 12),
+                                    (100_000, 15), (45, 4), (45, 9)])
+def test_gpu_inexact_windows_by_context(gpu_engine, n, kmer):
+    """Windows of 3 to 29 bases (the row-context path) and 30 (past it) with
+    and without tables, on a text with runs of one base and exact copies
+    (intervals of one row to thousands), for reads that lie on the text's
+    first and last bases, hold N at every place or one error at every place."""
+    hp = gpu_engine
+    rng = np.random.default_rng(51)
+    g = rng.integers(0, 4, n).astype(np.uint8)
+    if n > 1000:
+        g[500:900] = 0
+        g[2000:2300] = np.tile([0, 1], 150)
+        for i in range(90):                          # 90 copies of 40 bases
+            g[5000 + 100 * i:5040 + 100 * i] = g[5000:5040]
+        for i in range(40):
+            g[20000 + 60 * i:20030 + 60 * i] = g[20000:20030]
+    koff, kstart, lens = karyo(n, 2)
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(kstart, kstart + np.array(lens, np.uint64) - 1)
+    ix.to_device()
+    ix.expand()
+    if kmer:
+        ix.kmer_table(kmer)
+    o = fo.Oracle(g, ratio=16)
+    reads = [g[:29], g[:18], g[n - 29:], g[n - 18:], synth.revcomp(g[:18]), synth.revcomp(g[n - 18:])]
+    if n > 1000:
+        reads += [g[600:629], g[890:919], g[2000:2029], g[5000:5029], g[5010:5028], g[20000:20029]]
+    for base in [r.copy() for r in reads[:6]] + [g[7:25], g[9:30]]:
+        for p in range(len(base)):
+            for kind in range(4):
+                w = base.copy()
+                if kind == 0:
+                    w[p] = (w[p] + 1 + rng.integers(0, 3)) % 4
+                elif kind == 1:
+                    w = np.delete(w, p)
+                elif kind == 2:
+                    w = np.insert(w, p, rng.integers(0, 4))
+                else:
+                    w[p] = 4
+                reads.append(w.astype(np.uint8))
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads).astype(np.uint8), offs)
+    try:
+        for seed_size, min_seed in ((3, 1), (4, 3), (10, 3), (16, 5), (18, 16), (23, 3), (28, 3),
+                                    (29, 3), (30, 3)):
+            res = hp.map_inexact_seeds_batch(ix, batch, seed_size, min_seed, 256, 48)
+            for i, W in enumerate(reads):
+                want = o.map_inexact_seeds(W, seed_size, min_seed, koff, kstart, read=i,
+                                           rec_cap=256, region_cap=48)
+                w0 = int(res.window_base[i])
+                for t, (regs, st) in enumerate(want):
+                    w, s = w0 + t // 2, t % 2
+                    assert int(res.status[w, s]) == st, (seed_size, i, t)
+                    got = res.regions(w, s)
+                    assert got.tobytes() == regs.tobytes(), (seed_size, i, t)
+    finally:
+        batch.free()
+        ix.close()
