@@ -216,3 +216,64 @@ def test_gpu_vector_helper_vs_oracle_with_n(gpu_engine):
                 assert fo.hits_equal(hits[i, s, :min(n, cap)], h), (i, s)
     batch.free()
     ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,kmer", [(120_000, 0), (120_000, 7), (120_000, 10), (70, 4), (70, 9)])
+def test_gpu_vector_helper_on_text(gpu_engine, n, kmer):
+    """The expanded index: windows of 3 to 400 bases (row contexts up to 29,
+    the text above, the vectors where more than four rows reach half the
+    window), reads past the 256 bases that are staged, on copies (three and
+    twelve of them), runs of one base and both ends of the text, in both
+    modes and at a capacity that truncates, against the oracle."""
+    hp = gpu_engine
+    rng = np.random.default_rng(81)
+    g = rng.integers(0, 4, n).astype(np.uint8)
+    if n > 1000:
+        g[100:400] = 0
+        for c in range(3):
+            g[2000 + 500 * c:2400 + 500 * c] = g[1000:1400]
+        for c in range(12):
+            g[8000 + 200 * c:8120 + 200 * c] = g[7000:7120]
+    ix = hp.Index.build(g, 16).to_device()
+    ix.expand()
+    if kmer:
+        ix.kmer_table(kmer)
+    o = fo.Oracle(g, ratio=16)
+    reads, bounds = [], []
+    spots = [0, n] + ([1000, 1100, 2050, 7000, 8010, 150, 50_000] if n > 1000 else [20])
+    for L in (3, 4, 7, 15, 28, 29, 30, 31, 32, 45, 64, 65, 100, 255, 256, 257, 400):
+        for p in spots:
+            p = min(p, max(n - L, 0))
+            w = g[p:p + L].copy()
+            for kind in range(5):
+                v = w.copy()
+                e = int(rng.integers(0, len(v)))
+                if kind == 1:
+                    v[e] = (v[e] + 1) % 4
+                elif kind == 2:
+                    v = np.delete(v, e)
+                elif kind == 3:
+                    v = np.insert(v, e, rng.integers(0, 4))
+                elif kind == 4:
+                    v[e] = 4
+                if rng.random() < 0.5:
+                    v = synth.revcomp(v)
+                pre, post = rng.integers(0, 4, rng.integers(0, 18)), rng.integers(0, 4, 5)
+                reads.append(np.concatenate([pre, v, post]).astype(np.uint8))
+                bounds.append((len(pre), len(pre) + len(v) - 1))
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads), offs)
+    try:
+        for mode, cap in ((hp.MODE_EDIT, 40), (hp.MODE_MISMATCH, 40), (hp.MODE_EDIT, 2)):
+            counts, hits = hp.search1_vector_batch(ix, batch, cap=cap, mode=mode,
+                                                   bounds=np.array(bounds, np.int16))
+            for i, W in enumerate(reads):
+                for s in (0, 1):
+                    m, h = o.search1_vector(s, W, *bounds[i], cap=cap,
+                                            mismatch_only=mode == hp.MODE_MISMATCH)[:2]
+                    assert int(counts[i, s]) == m, (i, s, bounds[i])
+                    assert fo.hits_equal(hits[i, s, :min(m, cap)], h), (i, s, bounds[i])
+    finally:
+        batch.free()
+        ix.close()
