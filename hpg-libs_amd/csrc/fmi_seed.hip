@@ -5,9 +5,10 @@
 //   2. one lane per seed: + strand backward search on BACKWARD, - strand
 //      forward search on BACKWARD_REV (both over the seed's seed_len symbols),
 //      the cumulative filter of bwt.c:1250-1269 (a signed 32-bit running
-//      count, as the reference's `int actual_mappings`), rows to resolve
-//   3. exclusive scan of the rows of every (seed, strand)
-//   4. one lane per row: locate (getScompValue) on BACKWARD, binsearch over
+//      count, as the reference's `int actual_mappings`), rows to resolve,
+//      and the rows of every 64 seeds
+//   3. exclusive scan of those sums
+//   4. the rows of 64 seeds shared out in a wavefront: locate (getScompValue) on BACKWARD, binsearch over
 //      the karyotype offsets, the contig-end check key + len <= offset[idx]
 //      with len = seq_end - seq_start (one short, bwt.c:1214), region record.
 #include <hip/hip_runtime.h>
@@ -89,11 +90,32 @@ struct SeedParams {
   int32_t filter;
   fmi_seed_info *info;         // may be NULL
   uint64_t info_cap;
-  uint64_t *rows;              // 2 * nseeds: rows of + then - per seed
-  // 2 * nseeds: k of + and k of - (the first row of each) in the low 32 bits
-  // (rows are below 2^32 on the device), the seed's read in the high 32
-  int64_t *kl;
+  // 2 * nseeds, + then - of every seed: x the first row (or the one row's text
+  // position), y the rows (or kRowKnown)
+  uint2 *slots;
+  uint64_t *sums;              // rows of seeds 64 i .. 64 i + 63
 };
+
+// A slot with one row whose text position is known (rows are below 2^32 - 2).
+constexpr uint32_t kRowKnown = 0xFFFFFFFFu;
+
+// The cumulative filter with the reference's int arithmetic (bwt.c:1250-1269)
+// over the rows cp, cm of the + and - strands: the rows kept of each.
+__device__ __forceinline__ void seed_filter(int32_t filter, uint64_t cp, uint64_t cm, uint32_t &rp,
+                                            uint32_t &rm) {
+  int32_t actual = (int32_t)(uint32_t)cp;
+  rp = actual > filter ? 0u : (uint32_t)cp;
+  actual = (int32_t)((uint32_t)actual + (uint32_t)cm);
+  rm = actual > filter ? 0u : (uint32_t)cm;
+}
+
+// The sum of v over the wavefront's lanes, in every lane.
+__device__ __forceinline__ uint64_t wave_sum(uint64_t v) {
+  unsigned long long x = v;
+#pragma unroll
+  for (uint32_t d = 32u; d >= 1u; d >>= 1) x += __shfl_xor(x, (int)d);
+  return x;
+}
 
 // REGS (seed_len <= 32): the seed's bases are packed into registers once
 // (vh_regs) and every base below comes from there, not from a byte load.
@@ -101,73 +123,169 @@ template <bool REGS>
 __global__ __launch_bounds__(256) void seed_search_kernel(SeedParams P) {
   const DevDir &D = P.ix.d[0];
   const uint32_t n = P.ix.n;
-  for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < P.nseeds;
-       g += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t r = owner(P.seed_base, P.nreads, g);
-    const uint64_t s = (g - P.seed_base[r]) * P.stride;
-    const uint8_t *W = P.reads + P.offsets[r] + s;
-    VhRegs WR{0ull, 0u, 0};
-    if (REGS) WR = vh_regs(W, 0, P.seed_len);
-    auto base = [&](int32_t i) -> uint32_t { return REGS ? WR.at(i) : (uint32_t)W[i]; };
-    // The first k steps of each search from the k-mer table when its k bases
-    // are A/C/G/T and their interval is not empty (else step by step, so a
-    // dead interval is the one the LF steps give).
-    const uint32_t K = P.ix.kmer_k;
-    const bool use_k = K && P.seed_len >= K;
-    // + strand: BWExactSearchBackward over W[0 .. seed_len-1] on BACKWARD
-    uint32_t kp = 0, lp = n;
-    int32_t ip = (int32_t)P.seed_len - 1;
-    // - strand: BWExactSearchForward on BACKWARD_REV (complemented symbols)
-    uint32_t km = 0, lm = n;
-    uint32_t im = 0;
-    if (use_k) {
-      uint32_t cp = 0u, cm = 0u, bad = 0u;
-      for (uint32_t j = 0; j < K; ++j) {
-        const uint32_t sp = base(ip - (int32_t)j), sm = base((int32_t)j);
-        bad |= (sp > 3u || sm > 3u) ? 1u : 0u;
-        cp |= (sp & 3u) << (2u * j);
-        cm |= (sm & 3u) << (2u * j);
-      }
-      cm ^= (1u << (2u * K)) - 1u;
-      if (!bad) {
-        const uint64_t ep = P.ix.kmer[0][cp], em = P.ix.kmer[0][cm];
-        if ((uint32_t)ep <= (uint32_t)(ep >> 32)) {
-          kp = (uint32_t)ep; lp = (uint32_t)(ep >> 32); ip -= (int32_t)K;
+  const uint32_t lane = threadIdx.x & 63u;
+  for (uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; g0 < P.nseeds;
+       g0 += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t own = wave_owner(P.seed_base, P.nreads, P.nseeds, g0);
+    const uint64_t g = g0 + lane;
+    uint32_t rp = 0u, rm = 0u;
+    if (g < P.nseeds) {
+      const uint64_t r = own;
+      const uint64_t s = (g - P.seed_base[r]) * P.stride;
+      const uint8_t *W = P.reads + P.offsets[r] + s;
+      VhRegs WR{0ull, 0u, 0};
+      if (REGS) WR = vh_regs(W, 0, P.seed_len);
+      auto base = [&](int32_t i) -> uint32_t { return REGS ? WR.at(i) : (uint32_t)W[i]; };
+      // The first k steps of each search from the k-mer table when its k bases
+      // are A/C/G/T and their interval is not empty (else step by step, so a
+      // dead interval is the one the LF steps give).
+      const uint32_t K = P.ix.kmer_k;
+      const bool use_k = K && P.seed_len >= K;
+      // + strand: BWExactSearchBackward over W[0 .. seed_len-1] on BACKWARD
+      uint32_t kp = 0, lp = n;
+      int32_t ip = (int32_t)P.seed_len - 1;
+      // - strand: BWExactSearchForward on BACKWARD_REV (complemented symbols)
+      uint32_t km = 0, lm = n;
+      uint32_t im = 0;
+      if (use_k) {
+        uint32_t cp = 0u, cm = 0u, bad = 0u;
+        for (uint32_t j = 0; j < K; ++j) {
+          const uint32_t sp = base(ip - (int32_t)j), sm = base((int32_t)j);
+          bad |= (sp > 3u || sm > 3u) ? 1u : 0u;
+          cp |= (sp & 3u) << (2u * j);
+          cm |= (sm & 3u) << (2u * j);
         }
-        if ((uint32_t)em <= (uint32_t)(em >> 32)) {
-          km = (uint32_t)em; lm = (uint32_t)(em >> 32); im = K;
+        cm ^= (1u << (2u * K)) - 1u;
+        if (!bad) {
+          const uint64_t ep = P.ix.kmer[0][cp], em = P.ix.kmer[0][cm];
+          if ((uint32_t)ep <= (uint32_t)(ep >> 32)) {
+            kp = (uint32_t)ep; lp = (uint32_t)(ep >> 32); ip -= (int32_t)K;
+          }
+          if ((uint32_t)em <= (uint32_t)(em >> 32)) {
+            km = (uint32_t)em; lm = (uint32_t)(em >> 32); im = K;
+          }
         }
       }
+      for (int32_t i = ip; i >= 0; --i) {
+        uint32_t kn, ln;
+        if (lf_sym(D, kp, lp, base(i), 0u, kn, ln) > 3u) { kp = n + 1; lp = n; break; }
+        kp = kn; lp = ln;
+        if (kp > lp) break;
+      }
+      for (uint32_t i = im; i < P.seed_len; ++i) {
+        uint32_t kn, ln;
+        if (lf_sym(D, km, lm, base((int32_t)i), 1u, kn, ln) > 3u) { km = n + 1; lm = n; break; }
+        km = kn; lm = ln;
+        if (km > lm) break;
+      }
+      seed_filter(P.filter, kp <= lp ? (uint64_t)lp - kp + 1u : 0u,
+                  km <= lm ? (uint64_t)lm - km + 1u : 0u, rp, rm);
+      P.slots[2 * g] = make_uint2(kp, rp);
+      P.slots[2 * g + 1] = make_uint2(km, rm);
+      if (P.info && g < P.info_cap) {
+        fmi_seed_info inf;
+        inf.k_plus = kp; inf.l_plus = lp; inf.k_minus = km; inf.l_minus = lm;
+        inf.rows_plus = rp; inf.rows_minus = rm;
+        P.info[g] = inf;
+      }
     }
-    for (int32_t i = ip; i >= 0; --i) {
-      uint32_t kn, ln;
-      if (lf_sym(D, kp, lp, base(i), 0u, kn, ln) > 3u) { kp = n + 1; lp = n; break; }
-      kp = kn; lp = ln;
-      if (kp > lp) break;
+    const uint64_t sum = wave_sum((uint64_t)rp + rm);
+    if (lane == 0u) P.sums[g0 >> 6] = sum;
+  }
+}
+
+// The same on an index with row contexts and a k-mer table, for seeds of
+// kmer_k to 32 bases whose intervals are not asked for (no d_seed_info: where
+// and how an absent seed's search dies is not seen).  A strand is a table
+// entry, the contexts of its rows (those that go on with the seed's last
+// bases) and, for a strand that occurs, the first row's suffix -- its position
+// if it is the only one, else the row of it in the final interval.
+// Bound by random lines: 2 entries, 2-3 of contexts and about one of SA a seed,
+// where the entry and one or two occurrence blocks per base after it took
+// about 9.  47 M seeds of 18 bases over 3.1 Gbp: 9.4 ms, 7.2 with the strands'
+// contexts read one after the other, 6.5 as below (42 G lines/s, of the 47-50
+// that a gather over this much memory reaches).
+__global__ __launch_bounds__(256) void seed_context_kernel(SeedParams P) {
+  const DevDir &D = P.ix.d[0];
+  const uint32_t lane = threadIdx.x & 63u, K = P.ix.kmer_k, L = P.seed_len;
+  for (uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; g0 < P.nseeds;
+       g0 += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t r = wave_owner(P.seed_base, P.nreads, P.nseeds, g0);
+    const uint64_t g = g0 + lane;
+    uint32_t rp = 0u, rm = 0u;
+    if (g < P.nseeds) {
+      const uint64_t s = (g - P.seed_base[r]) * P.stride;
+      const VhRegs W = vh_regs(P.reads + P.offsets[r] + s, 0, L);
+      const uint32_t nmask = L >= 32u ? ~0u : (1u << L) - 1u;
+      WinIv v[2];
+      v[0].rows = v[1].rows = 0u;
+      if ((W.nfl & nmask) == 0u) {                 // an N occurs nowhere
+        const uint64_t v64 = __builtin_bitreverse64(W.code);
+        // + strand: W[L-1], W[L-2], ...; - strand: W[0], W[1], ... complemented
+        const uint64_t code[2] = {(((v64 >> 1) & 0x5555555555555555ull) |
+                                   ((v64 & 0x5555555555555555ull) << 1)) >> (64u - 2u * L),
+                                  ~W.code};
+        const uint32_t km = (1u << (2u * K)) - 1u;
+        const uint64_t e[2] = {P.ix.kmer[0][(uint32_t)code[0] & km],
+                               P.ix.kmer[0][(uint32_t)code[1] & km]};
+// both strands' first rows are read together where they lie in two
+        // 16-byte pieces of contexts (almost all do), then both suffixes
+        const uint32_t gs = L - K, gm = (uint32_t)win_mask(min(gs, 16u));
+        uint4 c[2][2];
+        bool near[2];
+#pragma unroll
+        for (uint32_t t = 0; t < 2u; ++t) {
+          const uint32_t k = (uint32_t)e[t], l = (uint32_t)(e[t] >> 32);
+          near[t] = k <= l && gs >= 1u && gs <= 16u && (k & 3u) + (l - k) < 8u && l - k < 8u;
+          c[t][0] = c[t][1] = opaque4();
+          const uint4 *p = reinterpret_cast<const uint4 *>(D.ctx + (k & ~3u));
+          if (near[t]) {
+            c[t][0] = p[0];
+            if ((k & 3u) + (l - k) >= 4u) c[t][1] = p[1];
+          }
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < 2u; ++t) {
+          const uint32_t k = (uint32_t)e[t], l = (uint32_t)(e[t] >> 32);
+          const uint64_t rest = code[t] >> (2u * K);
+          if (!near[t]) {
+            if (k > l || !win_extend(D, k, l, rest, gs, v[t])) v[t].rows = 0u;
+            continue;
+          }
+          const uint32_t w[8] = {c[t][0].x, c[t][0].y, c[t][0].z, c[t][0].w,
+                                 c[t][1].x, c[t][1].y, c[t][1].z, c[t][1].w};
+          uint32_t hit = 0u;
+#pragma unroll
+          for (uint32_t i = 0; i < 8u; ++i) {
+            const bool in = i >= (k & 3u) && i - (k & 3u) <= l - k;
+            if (in && ((w[i] ^ (uint32_t)rest) & gm) == 0u &&
+                win_real(D, (k & ~3u) + i, w[i], gs))
+              hit |= 1u << i;
+          }
+          v[t].rows = (uint32_t)__builtin_popcount(hit);
+          v[t].k = (k & ~3u) + (uint32_t)__builtin_ctz(hit | 0x100u);   // the first row before
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < 2u; ++t) {
+          if (!near[t]) continue;
+          v[t].q = kWinNone;
+          if (v[t].rows) v[t].q = D.sa[v[t].k] - gs;
+        }
+      }
+      seed_filter(P.filter, v[0].rows, v[1].rows, rp, rm);
+#pragma unroll
+      for (uint32_t t = 0; t < 2u; ++t) {
+        const uint32_t rows = t ? rm : rp;
+        uint2 slot = make_uint2(v[t].k, rows);
+        if (rows && v[t].q != kWinNone) {
+          if (rows == 1u) slot = make_uint2(v[t].q, kRowKnown);
+          else slot.x = D.isa[v[t].q];
+        }
+        P.slots[2 * g + t] = slot;
+      }
     }
-    for (uint32_t i = im; i < P.seed_len; ++i) {
-      uint32_t kn, ln;
-      if (lf_sym(D, km, lm, base((int32_t)i), 1u, kn, ln) > 3u) { km = n + 1; lm = n; break; }
-      km = kn; lm = ln;
-      if (km > lm) break;
-    }
-    // cumulative filter with the reference's int arithmetic
-    int32_t actual = 0;
-    const int64_t cp = (int64_t)lp - (int64_t)kp + 1, cm = (int64_t)lm - (int64_t)km + 1;
-    actual = (int32_t)((uint32_t)actual + (uint32_t)(uint64_t)cp);
-    const uint64_t rp = (actual > P.filter || kp > lp) ? 0 : (uint64_t)cp;
-    actual = (int32_t)((uint32_t)actual + (uint32_t)(uint64_t)cm);
-    const uint64_t rm = (actual > P.filter || km > lm) ? 0 : (uint64_t)cm;
-    P.rows[2 * g] = rp;
-    P.rows[2 * g + 1] = rm;
-    P.kl[2 * g] = (int64_t)((uint64_t)kp | (r << 32));
-    P.kl[2 * g + 1] = (int64_t)((uint64_t)km | (r << 32));
-    if (P.info && g < P.info_cap) {
-      fmi_seed_info inf;
-      inf.k_plus = kp; inf.l_plus = lp; inf.k_minus = km; inf.l_minus = lm;
-      inf.rows_plus = (uint32_t)rp; inf.rows_minus = (uint32_t)rm;
-      P.info[g] = inf;
-    }
+    const uint64_t sum = wave_sum((uint64_t)rp + rm);
+    if (lane == 0u) P.sums[g0 >> 6] = sum;
   }
 }
 
@@ -175,55 +293,98 @@ struct RowParams {
   DevIndex ix;
   const uint64_t *offsets;
   const uint64_t *seed_base;   // nreads + 1
-  const uint64_t *row_base;    // 2 * nseeds exclusive scan
-  const int64_t *kl;           // first row | read << 32 per (seed, strand)
+  const uint64_t *sum_base;    // exclusive scan of the rows of 64 seeds each
+  const uint2 *slots;          // as SeedParams
   const uint64_t *koff;        // kcount + 1
   const uint64_t *kstart;
-  uint64_t nslots, nrows;      // nslots = 2 * nseeds
+  uint64_t nseeds, nrows;      // rows to write
   uint32_t nreads, seed_len, stride, kcount;
   fmi_seed_region *out;
 };
 
+// A wavefront takes 64 seeds, whose rows are neighbours in out, and shares
+// them out among its lanes (wave_items).  Bound by the slots read and the
+// regions written (and a line of SA per row that the search did not locate);
+// a thread per row took a binary search over the scanned row counts, 27
+// dependent loads for 94 M slots: 57 M rows in 3.2 ms (and 0.6 to scan the
+// counts), 2.0 as below.
 __global__ __launch_bounds__(256) void seed_rows_kernel(RowParams P) {
   const DevDir &D = P.ix.d[0];
-  for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < P.nrows;
-       q += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t slot = owner(P.row_base, P.nslots, q);
-    const uint64_t g = slot >> 1;
-    const uint32_t strand = (uint32_t)(slot & 1u);
-    const uint64_t klr = (uint64_t)P.kl[slot];
-    const uint64_t j = (klr & 0xFFFFFFFFull) + (q - P.row_base[slot]);
-    const uint64_t r = klr >> 32;                 // the seed's read, from the search
-    const uint64_t seq_start = (g - P.seed_base[r]) * P.stride;
-    const uint64_t seq_end = seq_start + P.seed_len - 1;
-    const uint64_t seq_len = P.offsets[r + 1] - P.offsets[r];
-    const uint64_t len = seq_end - seq_start;
-    const uint64_t key = sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)j);
-    uint64_t lo = 0, size = P.kcount;          // binsearch, search/io.h:43-64
-    while (size > 0) {
-      const uint64_t w = size / 2;
-      if (P.koff[lo + w] <= key) { lo += w + 1; size -= w + 1; }
-      else size = w;
+  const uint32_t lane = threadIdx.x & 63u;
+  for (uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; g0 < P.nseeds;
+       g0 += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t first = P.sum_base[g0 >> 6];
+    if (first >= P.nrows) continue;
+    const uint64_t own = wave_owner(P.seed_base, P.nreads, P.nseeds, g0);
+    const bool mine = g0 + lane < P.nseeds;
+    uint4 sl = make_uint4(0u, 0u, 0u, 0u);         // + and - of the lane's seed
+    uint32_t seed = 0u, rd = 0u, rlen = 0u;
+    if (mine) {
+      sl = reinterpret_cast<const uint4 *>(P.slots)[g0 + lane];
+      rd = (uint32_t)own;
+      seed = (uint32_t)(g0 + lane - P.seed_base[own]);
+      rlen = (uint32_t)(P.offsets[own + 1] - P.offsets[own]);
     }
-    fmi_seed_region reg;
-    reg.read = (uint32_t)r;
-    reg.seed_id = (uint16_t)(g - P.seed_base[r]);
-    reg.strand = (uint8_t)strand;
-    reg.seq_start = (uint16_t)(strand ? seq_len - seq_end - 1 : seq_start);
-    reg.seq_end = (uint16_t)(strand ? seq_len - seq_start - 1 : seq_end);
-    reg.chrom_idx = (uint32_t)lo;
-    if (lo >= 1 && key + len <= P.koff[lo]) {
-      reg.start = P.kstart[lo - 1] + (key - P.koff[lo - 1]) + 1;
-      reg.end = reg.start + len;
-      reg.valid = 1;
-    } else {
-      reg.start = 0;
-      reg.end = 0;
-      reg.valid = 0;
+    const uint32_t rp = sl.y == kRowKnown ? 1u : sl.y, rm = sl.w == kRowKnown ? 1u : sl.w;
+    uint64_t done = 0;                             // rows of the rounds before
+    const uint64_t rows = (uint64_t)rp + rm, total = wave_sum(rows);
+    unsigned long long incl = rows;                // rows of lanes 0..i
+#pragma unroll
+    for (uint32_t d = 1u; d < 64u; d <<= 1) {
+      const unsigned long long v = __shfl_up(incl, d);
+      if (lane >= d) incl += v;
     }
-    P.out[q] = reg;
+    const unsigned long long excl = incl - rows;
+    for (; done < total && first + done < P.nrows; done += 64u) {
+      const unsigned long long t = done + lane;
+      uint32_t o = 0u;                             // the first lane whose rows reach past t
+#pragma unroll
+      for (uint32_t d = 32u; d >= 1u; d >>= 1)
+        if (__shfl(incl, (int)(o + d - 1u)) <= t) o += d;
+      const int src = (int)min(o, 63u);
+      uint64_t j = t - __shfl(excl, src);
+      const uint32_t np = __shfl(rp, src);
+      const uint32_t strand = j >= np ? 1u : 0u;
+      const uint32_t px = __shfl(sl.x, src), py = __shfl(sl.y, src);
+      const uint32_t mx = __shfl(sl.z, src), my = __shfl(sl.w, src);
+      const uint32_t sid = __shfl(seed, src), read = __shfl(rd, src), seq_len = __shfl(rlen, src);
+      if (t >= total || first + t >= P.nrows) continue;
+      if (strand) j -= np;
+      const uint32_t x = strand ? mx : px;
+      const bool known = (strand ? my : py) == kRowKnown;
+      const uint64_t key = known ? x : sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)(x + j));
+      const uint64_t seq_start = (uint64_t)sid * P.stride;
+      const uint64_t seq_end = seq_start + P.seed_len - 1;
+      const uint64_t len = seq_end - seq_start;
+      uint64_t lo = 0, size = P.kcount;            // binsearch, search/io.h:43-64
+      while (size > 0) {
+        const uint64_t w = size / 2;
+        if (P.koff[lo + w] <= key) { lo += w + 1; size -= w + 1; }
+        else size = w;
+      }
+      uint64_t start = 0, end = 0;
+      uint32_t valid = 0u;
+      if (lo >= 1 && key + len <= P.koff[lo]) {
+        start = P.kstart[lo - 1] + (key - P.koff[lo - 1]) + 1;
+        end = start + len;
+        valid = 1u;
+      }
+      const uint32_t ss = (uint16_t)(strand ? seq_len - seq_end - 1 : seq_start);
+      const uint32_t se = (uint16_t)(strand ? seq_len - seq_start - 1 : seq_end);
+      uint4 *dst = reinterpret_cast<uint4 *>(P.out + first + t);
+      dst[0] = make_uint4((uint32_t)start, (uint32_t)(start >> 32), (uint32_t)end,
+                          (uint32_t)(end >> 32));
+      dst[1] = make_uint4((uint32_t)lo, read, ss | (se << 16),
+                          (uint32_t)(uint16_t)sid | (strand << 16) | (valid << 24));
+    }
   }
 }
+static_assert(sizeof(fmi_seed_region) == 32 && offsetof(fmi_seed_region, chrom_idx) == 16 &&
+                  offsetof(fmi_seed_region, seq_start) == 24 &&
+                  offsetof(fmi_seed_region, seed_id) == 28 &&
+                  offsetof(fmi_seed_region, strand) == 30 &&
+                  offsetof(fmi_seed_region, valid) == 31,
+              "fmi_seed_region layout");
 
 // ---------------------------------------------------------------- inexact seeds
 // bwt_map_inexact_seeds_seq (bwt.c:3262-3302) + bwt_map_inexact_seed
@@ -666,11 +827,11 @@ int seed_map(const fmi_index *ix, const uint8_t *reads, const uint64_t *offsets,
              uint64_t *nrows_out, void *stream, std::string *err) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   int rc = FMI_OK;
-  uint64_t *cnt = nullptr, *base = nullptr, *rows = nullptr, *rbase = nullptr;
-  int64_t *kl = nullptr;
+  uint64_t *cnt = nullptr, *base = nullptr, *sums = nullptr;
+  uint2 *slots = nullptr;
   void *tmp = nullptr;
   size_t tmp_bytes = 0, need = 0;
-  uint64_t nseeds = 0, nrows = 0, last_rows = 0, last_base = 0;
+  uint64_t nseeds = 0, nrows = 0, nsums = 0;
   *nseeds_out = 0;
   *nrows_out = 0;
   SEED_TRY(hipMalloc(&cnt, (uint64_t)(nreads + 1) * 8));
@@ -686,17 +847,22 @@ int seed_map(const fmi_index *ix, const uint8_t *reads, const uint64_t *offsets,
   SEED_TRY(hipStreamSynchronize(s));
   *nseeds_out = nseeds;
   if (nseeds == 0) goto done;
-  SEED_TRY(hipMalloc(&rows, 2 * nseeds * 8));
-  SEED_TRY(hipMalloc(&rbase, 2 * nseeds * 8));
-  SEED_TRY(hipMalloc(&kl, 2 * nseeds * 8));
+  nsums = (nseeds + 63) / 64;
+  SEED_TRY(hipMalloc(&slots, 2 * nseeds * sizeof(uint2)));
+  SEED_TRY(hipMalloc(&sums, (nsums + 1) * 8));
   {
     SeedParams P{ix->dev, reads, offsets, base, nseeds, nreads, seed_len, stride,
-                 (int32_t)(filter > (uint32_t)INT32_MAX ? INT32_MAX : filter), info, info_cap, rows, kl};
-    if (seed_len <= 32u) seed_search_kernel<true><<<grid_for(nseeds), 256, 0, s>>>(P);
+                 (int32_t)(filter > (uint32_t)INT32_MAX ? INT32_MAX : filter), info, info_cap,
+                 slots, sums};
+    const uint32_t K = ix->dev.kmer_k;
+    if (!info && ix->dev.d[0].ctx && K && seed_len >= K && seed_len <= 32u)
+      seed_context_kernel<<<grid_for(nseeds), 256, 0, s>>>(P);
+    else if (seed_len <= 32u) seed_search_kernel<true><<<grid_for(nseeds), 256, 0, s>>>(P);
     else seed_search_kernel<false><<<grid_for(nseeds), 256, 0, s>>>(P);
   }
   SEED_TRY(hipGetLastError());
-  SEED_TRY(rocprim::exclusive_scan(nullptr, need, rows, rbase, (uint64_t)0, 2 * nseeds,
+  // in place, one sum more (any value): the last entry is then the total
+  SEED_TRY(rocprim::exclusive_scan(nullptr, need, sums, sums, (uint64_t)0, nsums + 1,
                                    rocprim::plus<uint64_t>(), s));
   if (need > tmp_bytes) {
     SEED_TRY(hipFree(tmp));
@@ -704,18 +870,16 @@ int seed_map(const fmi_index *ix, const uint8_t *reads, const uint64_t *offsets,
     tmp_bytes = need;
     SEED_TRY(hipMalloc(&tmp, tmp_bytes));
   }
-  SEED_TRY(rocprim::exclusive_scan(tmp, need, rows, rbase, (uint64_t)0, 2 * nseeds,
+  SEED_TRY(rocprim::exclusive_scan(tmp, need, sums, sums, (uint64_t)0, nsums + 1,
                                    rocprim::plus<uint64_t>(), s));
-  SEED_TRY(hipMemcpyAsync(&last_base, rbase + 2 * nseeds - 1, 8, hipMemcpyDeviceToHost, s));
-  SEED_TRY(hipMemcpyAsync(&last_rows, rows + 2 * nseeds - 1, 8, hipMemcpyDeviceToHost, s));
+  SEED_TRY(hipMemcpyAsync(&nrows, sums + nsums, 8, hipMemcpyDeviceToHost, s));
   SEED_TRY(hipStreamSynchronize(s));
-  nrows = last_base + last_rows;
   *nrows_out = nrows;
   if (nrows && region_cap && regions) {
-    RowParams R{ix->dev, offsets, base, rbase, kl, ix->d_koffset, ix->d_kstart, 2 * nseeds,
+    RowParams R{ix->dev, offsets, base, sums, slots, ix->d_koffset, ix->d_kstart, nseeds,
                 nrows < region_cap ? nrows : region_cap, nreads, seed_len, stride,
                 (uint32_t)ix->kstart.size(), regions};
-    seed_rows_kernel<<<grid_for(R.nrows), 256, 0, s>>>(R);
+    seed_rows_kernel<<<grid_for(nseeds), 256, 0, s>>>(R);
     SEED_TRY(hipGetLastError());
   }
 done:
@@ -725,9 +889,8 @@ done:
   }
   (void)hipFree(cnt);
   (void)hipFree(base);
-  (void)hipFree(rows);
-  (void)hipFree(rbase);
-  (void)hipFree(kl);
+  (void)hipFree(sums);
+  (void)hipFree(slots);
   (void)hipFree(tmp);
   return rc;
 }

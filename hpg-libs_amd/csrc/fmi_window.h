@@ -68,20 +68,24 @@ __device__ __forceinline__ bool win_real(const DevDir &D, uint32_t row, uint32_t
   return x == 0u || (t >> (2u * (x - 1u))) != 0u || D.sa[row] >= x;
 }
 
-// f(i, context) for rows k .. k + rows - 1, in order, 16 rows a round of
-// loads (16-byte pieces; the last piece may reach past the rows, not past the
-// array, which is padded to 256 bytes).
-template <class F>
+// f(i, context) for rows k .. k + rows - 1, in order, from 16-byte pieces, U of
+// them a round of loads (the last piece may reach past the rows, not past the
+// array, which is padded to 256 bytes).  A piece that holds none of the rows
+// is not read: a load costs a request per lane, needed or not.
+template <uint32_t U, class F>
 __device__ __forceinline__ void win_rows(const DevDir &D, uint32_t k, uint32_t rows, F f) {
   const uint4 *c = reinterpret_cast<const uint4 *>(D.ctx + (k & ~3u));
   const uint32_t off = k & 3u, end = off + rows;
-  for (uint32_t b = 0; b < end; b += 16u) {
-    uint4 v[4];
+  for (uint32_t b = 0; b < end; b += 4u * U) {
+    uint4 v[U];
+    v[0] = c[b >> 2];
 #pragma unroll
-    for (uint32_t u = 0; u < 4u; ++u)
-      v[u] = c[(b >> 2) + (b + 4u * u < end ? u : 0u)];
+    for (uint32_t u = 1; u < U; ++u) {
+      v[u] = opaque4();
+      if (b + 4u * u < end) v[u] = c[(b >> 2) + u];
+    }
 #pragma unroll
-    for (uint32_t u = 0; u < 4u; ++u) {
+    for (uint32_t u = 0; u < U; ++u) {
       const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
       for (uint32_t e = 0; e < 4u; ++e) {
@@ -142,7 +146,7 @@ __device__ __forceinline__ bool win_extend(const DevDir &D, uint32_t k, uint32_t
   if (g == 0u) return true;
   uint32_t cnt = 0u, first = 0u;
   const uint32_t want = (uint32_t)code, mask = (uint32_t)win_mask(g);
-  win_rows(D, k, l - k + 1u, [&](uint32_t i, uint32_t t) {
+  win_rows<2>(D, k, l - k + 1u, [&](uint32_t i, uint32_t t) {
     if (((t ^ want) & mask) == 0u && win_real(D, k + i, t, g)) {
       if (cnt == 0u) first = i;
       ++cnt;
@@ -246,7 +250,7 @@ __device__ __forceinline__ void win_half(const DevIndex &ix, uint32_t dir, uint3
       ns = (ns | (ns << 1)) & 0x55555555u;
       const uint32_t mN = (uint32_t)win_mask(N), mN1 = mN >> 2;
       uint32_t at = 0u;
-      win_rows(D, k, l - k + 1u, [&](uint32_t i, uint32_t t) {
+      win_rows<4>(D, k, l - k + 1u, [&](uint32_t i, uint32_t t) {
         auto fold = [](uint32_t x) { return (x | (x >> 1)) & 0x55555555u; };
         const uint32_t x0 = (fold(t ^ want) | ns) & mN;
         const uint32_t xd = (fold(t ^ (want >> 2)) | (ns >> 2)) & mN1;

@@ -118,3 +118,63 @@ def test_seed_map_gpu_vs_oracle(gpu_engine):
     ns, nr, regs, _ = hp.seed_map_batch(ix, batch, 18, 5, 1000, region_cap=10, with_info=False)
     assert len(regs) == 10 and nr > 10
     batch.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kmer,seed_len,stride", [(4, 4, 1), (8, 8, 3), (8, 9, 5), (8, 24, 7),
+                                                  (8, 25, 1), (8, 32, 5), (12, 18, 5), (15, 31, 2)])
+def test_gpu_seed_map_by_context(gpu_engine, kmer, seed_len, stride):
+    """The expanded index with a table and no intervals asked for (row
+    contexts), and the same call with them (occurrence blocks): equal to the
+    oracle, for seeds of a k-mer's length to 32 bases, on copies (more rows
+    than one look takes), runs of one base and the text's ends, with N bases,
+    a filter that skips strands, reads without a seed, and room for a part of
+    the regions only."""
+    hp = gpu_engine
+    rng = np.random.default_rng(61)
+    n = 40_000
+    g = rng.integers(0, 4, n).astype(np.uint8)
+    g[500:800] = 2
+    for i in range(120):
+        g[3000 + 50 * i:3034 + 50 * i] = g[3000:3034]
+    koff, kstart = karyotype(n, [9_000, 20_000])
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(kstart, kstart + np.diff(koff) - 1)
+    ix.to_device()
+    ix.expand()
+    ix.kmer_table(kmer)
+    o = fo.Oracle(g, ratio=8)
+    reads = [g[:60], g[n - 60:], g[450:560], g[3000:3080], g[8_970:9_030], g[:3], g[:0], g[100:131]]
+    more, moffs, _ = synth.reads(g, 150, seed=62, sub_rate=0.01, n_rate=0.004,
+                                 lengths=rng.integers(0, 120, 150))
+    reads += [more[int(moffs[i]):int(moffs[i + 1])] for i in range(150)]
+    reads += [synth.revcomp(r) for r in reads[:6]]
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads), offs)
+    try:
+        for filt in (5, 1000):
+            want, winfo = [], []
+            for i, W in enumerate(reads):
+                if len(W) < seed_len:
+                    continue
+                regs, info = o.seed_map(W, seed_len, stride, filt, koff, kstart)
+                regs = regs.copy()
+                regs["read"] = i
+                want.append(regs)
+                winfo.append(info)
+            want, winfo = np.concatenate(want), np.concatenate(winfo)
+            ns, nr, regs, _ = hp.seed_map_batch(ix, batch, seed_len, stride, filt, with_info=False)
+            assert (ns, nr) == (len(winfo), len(want))
+            assert regs.tobytes() == want.tobytes()
+            ns, nr, regs, info = hp.seed_map_batch(ix, batch, seed_len, stride, filt)
+            assert regs.tobytes() == want.tobytes()
+            for c, key in enumerate(("k_plus", "l_plus", "k_minus", "l_minus", "rows_plus",
+                                     "rows_minus")):
+                assert np.array_equal(info[key], winfo[:, c]), key
+            for cap in (1, 63, 64, 65, max(nr - 1, 1)):
+                _, nr2, regs, _ = hp.seed_map_batch(ix, batch, seed_len, stride, filt,
+                                                    region_cap=cap, with_info=False)
+                assert nr2 == nr and regs.tobytes() == want[:cap].tobytes()
+    finally:
+        batch.free()
+        ix.close()
