@@ -42,6 +42,15 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
                           uint32_t *queue, unsigned long long *stats, uint32_t grid_persistent,
                           uint32_t chunk, uint32_t refill_min, bool own_loads, hipStream_t s,
                           void *staged = nullptr);
+// The staged launch's first part on an expanded index (fmi_search1t.hip): the
+// reads searched on the text; those it leaves are appended to list, with their
+// records in rec.  wide: scratch for as many reads; wide_n and list_n are
+// zeroed by the caller.
+hipError_t launch_search1_text(const DevIndex &ix, bool mm_only, uint32_t strand_mask,
+                               const uint8_t *reads, const uint64_t *offsets, uint32_t nreads,
+                               uint32_t cap, fmi_hit *hits, uint32_t *counts, uint32_t *rec,
+                               uint32_t *wide, uint32_t *wide_n, uint32_t *list, uint32_t *list_n,
+                               uint32_t cus, hipStream_t s);
 hipError_t launch_zero(uint32_t *p, uint32_t n, hipStream_t s);
 // Byte fill of bytes bytes with v (a kernel, so a captured graph holds no
 // memset node).

@@ -1138,7 +1138,10 @@ void search1_kernel(S1Params P) {
               const uint32_t len = (uint32_t)(P.offsets[h_task + 1] - P.offsets[h_task]);
               h_len = len > kStagedMaxLen ? 0xFFFFFFFFu : len;   // longer: the unstaged kernel's
             } else {
-              m.task_info(h_task, h_off, h_len, h_kc0, h_kc1);
+              // of a list the reads that fit a slot are the staged kernel's
+              if (P.list && P.offsets[h_task + 1] - P.offsets[h_task] <= kStagedMaxLen)
+                h_len = 0xFFFFFFFFu;
+              else m.task_info(h_task, h_off, h_len, h_kc0, h_kc1);
             }
           }
         }
@@ -1156,7 +1159,7 @@ void search1_kernel(S1Params P) {
           const uint32_t kc1 = __shfl(h_kc1, src);
           const uint32_t off_lo = __shfl((uint32_t)h_off, src);
           const uint32_t off_hi = __shfl((uint32_t)(h_off >> 32), src);
-          if (L.phase == PH_IDLE && rank < avail)
+          if (L.phase == PH_IDLE && rank < avail && len != 0xFFFFFFFFu)
             m.start_with(task, ((uint64_t)off_hi << 32) | off_lo, len, kc0, kc1);
         }
         wq_next += min(avail, nidle);
@@ -1178,21 +1181,26 @@ void search1_kernel(S1Params P) {
 
 // The rows of the records search1_kernel stored as text positions (k's high
 // word kTextRowTag, l = q): k = l = ISA[q] in the record's direction (dir ^
-// strand: the pass's direction).  One thread per (read, strand) slot.
+// strand: the pass's direction).  One thread per (read, strand) slot, of the
+// listed reads where there is a list.
 __global__ __launch_bounds__(256) void text_rows_kernel(DevIndex ix, fmi_hit *hits,
                                                         const uint32_t *counts, uint32_t nslots,
-                                                        uint32_t cap) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nslots) return;
-  const uint32_t c = min(counts[t], cap);
-  uint4 *h = reinterpret_cast<uint4 *>(hits + (size_t)t * cap);
-  for (uint32_t j = 0; j < c; ++j) {
-    const uint4 a = h[2 * j];
-    if (a.y != kTextRowTag) continue;
-    const uint4 b = h[2 * j + 1];
-    const uint32_t dsel = (b.z & 0xFFu) ^ (b.w & 0xFFu);
-    const uint32_t row = (dsel ? ix.d[1].isa : ix.d[0].isa)[a.x];
-    h[2 * j] = make_uint4(row, 0u, row, 0u);
+                                                        uint32_t cap, const uint32_t *list,
+                                                        const uint32_t *list_n) {
+  const uint64_t n = list ? 2ull * *list_n : nslots;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t t = list ? 2u * list[i >> 1] + (uint32_t)(i & 1u) : (uint32_t)i;
+    const uint32_t c = min(counts[t], cap);
+    uint4 *h = reinterpret_cast<uint4 *>(hits + (size_t)t * cap);
+    for (uint32_t j = 0; j < c; ++j) {
+      const uint4 a = h[2 * j];
+      if (a.y != kTextRowTag) continue;
+      const uint4 b = h[2 * j + 1];
+      const uint32_t dsel = (b.z & 0xFFu) ^ (b.w & 0xFFu);
+      const uint32_t row = (dsel ? ix.d[1].isa : ix.d[0].isa)[a.x];
+      h[2 * j] = make_uint4(row, 0u, row, 0u);
+    }
   }
 }
 
@@ -1609,7 +1617,8 @@ hipError_t launch_vector(const DevIndex &ix, uint32_t dsel, uint32_t comp, uint3
 }
 
 uint64_t search1_staged_scratch_bytes(uint32_t nreads) {
-  return ((64ull + 4ull * nreads + 127ull) & ~127ull) + (uint64_t)kRecWords * 4ull * nreads;
+  return ((64ull + 4ull * nreads + 127ull) & ~127ull) + (uint64_t)kRecWords * 4ull * nreads +
+         4ull * nreads;
 }
 
 hipError_t launch_read_records(const uint8_t *reads, const uint64_t *offsets, uint32_t nreads,
@@ -1639,17 +1648,28 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
     const dim3 g(grid_persistent), b(256);
     if (staged && !count && ntasks <= kStagedMaxTasks) {
       // scratch: [0] the unstaged kernel's work counter, [1] the list's
-      // length; the list from byte 64; the records from the next 128 bytes
+      // length, [2] the wide list's; the list from byte 64; the records from
+      // the next 128 bytes, then the wide list
       uint32_t *head = static_cast<uint32_t *>(staged);
       uint32_t *list = head + 16;
       uint32_t *rec = reinterpret_cast<uint32_t *>(static_cast<char *>(staged) +
                                                    ((64ull + 4ull * ntasks + 127ull) & ~127ull));
-      hipError_t e = launch_zero(head, 2, s);
+      hipError_t e = launch_zero(head, 3, s);
       if (e != hipSuccess) return e;
-      RecParams R{reads, offsets, ntasks, rec, list, head + 1};
-      hipLaunchKernelGGL(read_records_kernel, dim3((uint32_t)((8ull * ntasks + 255) / 256)),
-                         dim3(256), 0, s, R);
       P.rec = reinterpret_cast<const uint4 *>(rec);
+      if (text) {
+        // on the text first; the two kernels below take the reads it leaves
+        e = launch_search1_text(ix, mm_only, strand_mask, reads, offsets, ntasks, cap, hits,
+                                counts, rec, rec + (uint64_t)kRecWords * ntasks, head + 2, list,
+                                head + 1, 256u, s);
+        if (e != hipSuccess) return e;
+        P.list = list;
+        P.list_n = head + 1;
+      } else {
+        RecParams R{reads, offsets, ntasks, rec, list, head + 1};
+        hipLaunchKernelGGL(read_records_kernel, dim3((uint32_t)((8ull * ntasks + 255) / 256)),
+                           dim3(256), 0, s, R);
+      }
 #define FMI_S1_STAGED(MM)                                                                      \
   do {                                                                                         \
     if (!text) hipLaunchKernelGGL((search1_kernel<true, MM, false, false, false, true>), g, b, 0, s, P); \
@@ -1692,9 +1712,10 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
     }
   }
   if (!count && ix.text != nullptr && cap > 0) {
-    const uint64_t nslots = 2ull * ntasks;
-    hipLaunchKernelGGL(text_rows_kernel, dim3((uint32_t)((nslots + 255) / 256)), dim3(256), 0, s,
-                       ix, hits, counts, (uint32_t)nslots, cap);
+    const uint64_t nslots = 2ull * ntasks, grid = (nslots + 255) / 256;
+    hipLaunchKernelGGL(text_rows_kernel,
+                       dim3((uint32_t)(P.list ? std::min<uint64_t>(grid, 1024u) : grid)), dim3(256),
+                       0, s, ix, hits, counts, (uint32_t)nslots, cap, P.list, P.list_n);
   }
   return hipGetLastError();
 }

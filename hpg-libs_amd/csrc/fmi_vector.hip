@@ -20,6 +20,7 @@
 #include "fmi_device.h"
 #include "fmi_internal.h"
 #include "fmi_kernels.h"
+#include "fmi_rows.h"
 #include "fmi_vhelper.h"
 #include "fmi_window.h"
 
@@ -68,84 +69,20 @@ __device__ __forceinline__ bool vh_window(const VhParams &P, uint32_t t, const u
          end - start >= 2;
 }
 
-// The read's bases: from the thread's LDS slot (STAGED) or its bytes.
-template <bool STAGED>
-struct VtRead {
-  const uint8_t *W;
-  const uint32_t *slot;
-  __device__ __forceinline__ uint32_t at(int32_t p) const {
-    return STAGED ? lds_base(slot, p) : (uint32_t)W[p];
-  }
-  // How many of the cnt bases W[p], W[p + d], ... equal the text before
-  // suffix q.
-  __device__ __forceinline__ int32_t match(const DevIndex &ix, uint32_t dsel, uint32_t comp,
-                                           uint32_t q, int32_t p, int32_t d, int32_t cnt) const {
-    int32_t done = 0;
-    while (done < cnt) {
-      const uint32_t lim = min(min((uint32_t)(cnt - done), STAGED ? 32u : 16u), q);
-      if (lim == 0u) break;
-      const uint32_t m = STAGED ? text_match32(ix, dsel, comp, q, slot, p + done * d, d, lim)
-                                : text_match(ix, dsel, comp, q, W, p + done * d, d, lim);
-      done += (int32_t)m;
-      q -= m;
-      if (m < lim) break;
-    }
-    return done;
-  }
-};
-
 // One half (dir 0: the backward vector's nodes and the exact record; dir 1:
 // the forward vector's), numbered as in fmi_window.h; false when its interval
 // has more than kTextRows rows at the shortest node.
 template <bool STAGED>
 __device__ __forceinline__ bool vt_half(const DevIndex &ix, uint32_t dir, uint32_t strand,
-                                        const VtRead<STAGED> &rd, int32_t start, int32_t end,
+                                        const ReadBases<STAGED> &rd, int32_t start, int32_t end,
                                         VhRec &r, VtSink &S) {
   const uint32_t dsel = dir ^ strand, comp = strand;
-  const DevDir &D = dir_of(ix, dsel);
   const int32_t L = end - start + 1, d = dir ? 1 : -1, p0 = dir ? start : end;
   const int32_t m0 = dir ? (L - 1) / 2 : L - (L - 1) / 2;
-  // the interval of the first bases, from the longest table that they fill
-  const int32_t K = (int32_t)ix.kmer_k <= m0 ? (int32_t)ix.kmer_k
-                                             : ((int32_t)ix.kmer2_k <= m0 ? (int32_t)ix.kmer2_k : 0);
-  uint32_t k = 0u, l = ix.n;
-  int32_t m = 0;
-  if (K) {
-    uint32_t code = 0u, bad = 0u;
-    if (STAGED) {
-      uint64_t w;
-      uint32_t nb;
-      lds_window(rd.slot, p0, d, w, nb);
-      code = (uint32_t)w & ((1u << (2u * (uint32_t)K)) - 1u);
-      bad = nb & ((1u << (uint32_t)K) - 1u);
-    } else {
-      for (int32_t j = 0; j < K; ++j) {
-        const uint32_t s = rd.W[p0 + j * d];
-        bad |= s > 3u ? 1u : 0u;
-        code |= (s & 3u) << (2u * (uint32_t)j);
-      }
-    }
-    if (bad) return true;                          // an N: no node is alive
-    if (comp) code ^= (1u << (2u * (uint32_t)K)) - 1u;
-    const uint64_t e = (K == (int32_t)ix.kmer_k ? (dsel ? ix.kmer[1] : ix.kmer[0])
-                                                : (dsel ? ix.kmer2[1] : ix.kmer2[0]))[code];
-    k = (uint32_t)e;
-    l = (uint32_t)(e >> 32);
-    if (k > l) return true;
-    m = K;
-  }
-  for (; m < m0 && l - k >= kTextRows; ++m) {
-    uint32_t a, b;
-    if (lf_sym(D, k, l, rd.at(p0 + m * d), comp, a, b) > 3u || a > b) return true;
-    k = a;
-    l = b;
-  }
-  if (l - k >= kTextRows) return false;
-  TextRows R = text_rows(D, k, l);
-  if (m < m0) {
-    text_feed<STAGED>(ix, dsel, comp, rd.slot, rd.W, p0 + m * d, d, m0 - m, R);
-    if (R.n == 0u) return true;
-  }
+  TextRows R;
+  uint32_t k, l;
+  const uint32_t found = search_rows<STAGED>(ix, dsel, comp, rd, p0, d, m0, R, k, l);
+  if (found != kRowsFew) return found == kRowsNone;   // without rows no node is alive
   // how far each row goes on with the window: it ends at a node
   const int32_t N = L - m0;
   int32_t run[kTextRows] = {-1, -1, -1, -1};
@@ -175,43 +112,26 @@ __device__ __forceinline__ bool vt_half(const DevIndex &ix, uint32_t dir, uint32
     cur = a;
     const int32_t c1 = N - 1 - a, p = p0 + (m0 + a) * d;
     const bool last = c1 == 0;
-    const uint32_t insbit = last ? 2u : 1u, mmbit = last ? 1u : 2u;
-    const uint32_t w = rd.at(p), sm = w > 3u ? 4u : (comp ? 3u - w : w);
     r.err_pos = p;
-    uint32_t live = 0u, cnts = 0u;                 // rows per string, 3 bits each
-    uint32_t q[9];                                 // the suffix of its first
+    const NodeStrings T = node_strings<STAGED, false>(ix, dsel, comp, rd, R, run, a, p, d, c1);
 #pragma unroll
-    for (uint32_t j = 0; j < kTextRows; ++j) {
-      if (run[j] < a) continue;
-      const uint32_t qa = R.q[j] - (uint32_t)a;
-      auto put = [&](uint32_t bit, uint32_t x) {
-#pragma unroll
-        for (uint32_t i = 0; i < 9u; ++i)
-          if (i == bit && !((live >> i) & 1u)) q[i] = x;
-        live |= 1u << bit;
-        cnts += 1u << (3u * bit);
+    for (uint32_t i = 0; i < 9u; ++i) {
+      // at the last base the mismatch comes before the insertion
+      auto add = [&](uint32_t bit) {
+        if (!((T.live >> bit) & 1u)) return;
+        const bool isins = (bit & 1u) != 0u;
+        r.pos = last ? -1 : (dir ? end + 1 : start - 1);
+        r.kind = bit == 0u ? FMI_DELETION : (isins ? FMI_INSERTION : FMI_MISMATCH);
+        r.base = bit == 0u ? 0xFFu : (bit - 1u) >> 1;
+        if (isins && last && dir == 0u) {
+          // search.c:1556 stores kind 3, base INSERTION (3), position b
+          r.base = FMI_INSERTION;
+          r.err_pos = (int32_t)((bit - 1u) >> 1);
+        }
+        S.add(r, dsel, WinIv{0u, T.q[bit], (T.cnts >> (3u * bit)) & 7u});
       };
-      if (rd.match(ix, dsel, comp, qa, p + d, d, c1) == c1) put(0u, qa - (uint32_t)c1);
-      if (qa == 0u) continue;
-      const uint32_t b = (uint32_t)text_window32(ix, dsel, qa) & 3u, lb = comp ? 3u - b : b;
-      if (b != sm && rd.match(ix, dsel, comp, qa - 1u, p + d, d, c1) == c1)
-        put(2u * lb + mmbit, qa - 1u - (uint32_t)c1);
-      if (rd.match(ix, dsel, comp, qa - 1u, p, d, c1 + 1) == c1 + 1)
-        put(2u * lb + insbit, qa - 2u - (uint32_t)c1);
-    }
-#pragma unroll
-    for (uint32_t bit = 0; bit < 9u; ++bit) {
-      if (!((live >> bit) & 1u)) continue;
-      const bool isins = bit != 0u && ((bit & 1u) != 0u) == !last;
-      r.pos = last ? -1 : (dir ? end + 1 : start - 1);
-      r.kind = bit == 0u ? FMI_DELETION : (isins ? FMI_INSERTION : FMI_MISMATCH);
-      r.base = bit == 0u ? 0xFFu : (bit - 1u) >> 1;
-      if (isins && last && dir == 0u) {
-        // search.c:1556 stores kind 3, base INSERTION (3), position b
-        r.base = FMI_INSERTION;
-        r.err_pos = (int32_t)((bit - 1u) >> 1);
-      }
-      S.add(r, dsel, WinIv{0u, q[bit], (cnts >> (3u * bit)) & 7u});
+      if (i == 0u || !last) add(i);
+      else add(((i - 1u) ^ 1u) + 1u);
     }
   }
   return true;
@@ -230,7 +150,7 @@ __device__ __forceinline__ uint32_t vt_task(const VhParams &P, uint32_t t, const
   S.start = (int16_t)start;
   S.end = (int16_t)end;
   S.ix = &P.ix;
-  const VtRead<STAGED> rd{W, slot};
+  const ReadBases<STAGED> rd{W, slot};
   VhRec r{0, 0, -1, 0, 0, 0, 0, 0};
   for (uint32_t dir = 0; dir < 2u; ++dir) {
     r.dir = dir;
@@ -242,10 +162,10 @@ __device__ __forceinline__ uint32_t vt_task(const VhParams &P, uint32_t t, const
 // A thread per (read, strand), the read packed into its LDS slot (24 KB a
 // workgroup; longer reads from their bytes).  Bound by the latency of a
 // half's chain -- a table entry, the rows' suffixes, the text under them --
-// with 16 wavefronts a CU (124 registers) to hide it.  250 K reads of 150
-// bases over 64 Mbp: 183 us, where an LF step per base of both vectors on 64 K
+// with 16 wavefronts a CU (held to 128 registers) to hide it.  250 K reads of
+// 150 bases over 64 Mbp: 175 us, where an LF step per base of both vectors on 64 K
 // lanes (their scratch allows no more) took 6.6 ms.
-__global__ __launch_bounds__(256) void vector_text_kernel(VhParams P) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void vector_text_kernel(VhParams P) {
   __shared__ uint32_t slots[kReadRecordWords * 256u];
   const uint64_t t64 = (uint64_t)blockIdx.x * 256u + threadIdx.x;
   if (t64 >= 2ull * P.nreads) return;
