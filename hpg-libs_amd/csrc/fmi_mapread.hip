@@ -14,8 +14,8 @@
 // (bwt.c:2190-2233).
 //
 // Two launches.  map_single_kernel, a thread per read, settles every read of
-// at most kStagedMaxLen bases whose strands have at most one row each (no
-// dedup, no count to filter) and marks the others in counts;
+// at most kStagedMaxLen bases whose strands have at most kTextRows rows each
+// (one on a compact index) and marks the others in counts;
 // map_reads_kernel's lanes stride over the marked reads, a lane keeping the
 // current strand's alignments in its scratch slice (at most filter + 1 of
 // them: a strand's rows number l - k + 1 <= filter + 1 once the count has
@@ -28,6 +28,7 @@
 #include "fmi_device.h"
 #include "fmi_internal.h"
 #include "fmi_kernels.h"
+#include "fmi_rows.h"
 
 namespace fmi {
 
@@ -58,29 +59,31 @@ constexpr uint32_t kMapWaits = 0xFFFFFFFFu;
 
 // BWExactSearchBackward of the whole read from [0, n] on one view: whether its
 // interval is not empty (an empty one is not formed: no caller sees it), and
-// then the rows k..l (R.n = 0), or, where the search ended on the text of an
-// expanded index, its rows' suffixes (R).  kt, lt: the interval of the read's
-// last K bases, from the k-mer table (K = 0: none).  STAGED: the read's bases
-// come from the thread's LDS slot.
+// then its rows' suffixes R, or on a compact index, or where there are more of
+// them, the rows k..l (R.n = 0).
 template <bool STAGED>
 __device__ __forceinline__ bool live_interval(const DevIndex &ix, uint32_t dsel, uint32_t comp,
-                                              const uint8_t *W, int32_t len, const uint32_t *slot,
-                                              uint32_t K, uint32_t kt, uint32_t lt, uint32_t &k,
-                                              uint32_t &l, TextRows &R) {
+                                              const ReadBases<STAGED> &rd, int32_t len,
+                                              uint32_t &k, uint32_t &l, TextRows &R) {
   const DevDir &D = dir_of(ix, dsel);
-  k = K ? kt : 0u;
-  l = K ? lt : ix.n;
   R.n = 0u;
-  if (k > l) return false;
-  for (int32_t i = len - 1 - (int32_t)K; i >= 0; --i) {
-    if (l - k < kTextRows && ix.text != nullptr) {
-      R = text_rows(D, k, l);
-      text_feed<STAGED>(ix, dsel, comp, slot, W, i, -1, i + 1, R);
-      return R.n != 0u;
-    }
+  if (ix.text != nullptr)
+    return search_rows<STAGED>(ix, dsel, comp, rd, len - 1, -1, len, R, k, l) != kRowsNone;
+  const int32_t K = ix.kmer_k && len >= (int32_t)ix.kmer_k ? (int32_t)ix.kmer_k : 0;
+  k = 0u;
+  l = ix.n;
+  if (K) {
+    uint32_t c;
+    if (!rd.code(len - 1, -1, K, comp, c)) return false;
+    const uint64_t e = (dsel ? ix.kmer[1] : ix.kmer[0])[c];
+    k = (uint32_t)e;
+    l = (uint32_t)(e >> 32);
+    if (k > l) return false;
+  }
+  for (int32_t i = len - 1 - K; i >= 0; --i) {
     uint32_t a, b;
-    const uint32_t sym = STAGED ? lf_sym(D, k, l, lds_base(slot, i), comp, a, b)
-                                : lf_read(D, k, l, W + i, comp, a, b);
+    const uint32_t sym = STAGED ? lf_sym(D, k, l, rd.at(i), comp, a, b)
+                                : lf_read(D, k, l, rd.W + i, comp, a, b);
     if (sym > 3u || a > b) return false;
     k = a;
     l = b;
@@ -116,14 +119,14 @@ __device__ __forceinline__ void store_mapping(fmi_read_mapping *out, uint64_t po
 }
 
 // One thread per read.  The read is packed into the thread's LDS slot once
-// for both strands, both strands' table entries are read together, and a
-// search that has narrowed to at most four rows goes on against their text,
-// 32 bases a compare: about six dependent loads for a read that occurs once
-// where an LF step per base and strand took 100 and more.  Bound by those loads' lines
+// for both strands, and each is searched to its rows on the text (search_rows):
+// about six dependent loads for a read that occurs once where an LF step per
+// base and strand took 100 and more.  Bound by those loads' lines
 // (an entry per strand, then SA and text for one of them); the slots
 // (24 KB a workgroup) leave 6 workgroups a CU.  500 K reads of 100 bases over
-// 64 Mbp: 151 us, and 140 for the marked reads, where one launch of 64 K
-// lanes (the scratch allows no more) took 1540.
+// 64 Mbp: 145 us, where one launch of 64 K lanes (the scratch allows no more)
+// took 1540, and 125 went to the marked reads when they were those with more
+// than one row.
 __global__ __launch_bounds__(256) void map_single_kernel(MapParams P) {
   __shared__ uint32_t slots[kReadRecordWords * 256u];
   const uint32_t rd = blockIdx.x * 256u + threadIdx.x;
@@ -144,47 +147,56 @@ __global__ __launch_bounds__(256) void map_single_kernel(MapParams P) {
   uint32_t *slot = slots + threadIdx.x;
   stage_read(W, (uint32_t)len, slot);
   const uint32_t n = P.ix.n;
-  uint32_t K = P.ix.kmer_k;
-  uint64_t e[2] = {0ull, 0ull};
-  bool dead = false;
-  if (K && len >= (int32_t)K) {
-    uint64_t w;
-    uint32_t nb;
-    lds_window(slot, len - 1, -1, w, nb);
-    const uint32_t kmask = (1u << (2u * K)) - 1u;
-    dead = (nb & ((1u << K) - 1u)) != 0u;      // an N occurs nowhere
-    const uint32_t code = (uint32_t)w & kmask;
-    if (!dead) {
-      e[0] = P.ix.kmer[0][code];
-      e[1] = P.ix.kmer[1][code ^ kmask];
-    }
-  } else {
-    K = 0u;
-  }
-  uint32_t nout = 0;
-  for (uint32_t strand = 0; strand < 2u && !dead; ++strand) {
+  const ReadBases<true> bases{W, slot};
+  uint32_t nout = 0, tot = 0;
+  uint8_t st = 0;
+  for (uint32_t strand = 0; strand < 2u; ++strand) {
     // + strand: BACKWARD; - strand: FORWARD_REV (bwt.c:1996-2001)
     uint32_t k, l;
     TextRows R;
-    if (!live_interval<true>(P.ix, strand, strand, W, len, slot, K, (uint32_t)e[strand],
-                             (uint32_t)(e[strand] >> 32), k, l, R))
-      continue;
-    if (R.n ? R.n != 1u : k != l) {
-      P.counts[rd] = kMapWaits;
-      return;
+    if (!live_interval<true>(P.ix, strand, strand, bases, len, k, l, R)) continue;
+    if (R.n == 0u) {
+      if (k != l) {
+        P.counts[rd] = kMapWaits;
+        return;
+      }
+      R.n = 1u;
+      R.q[0] = sa_value(dir_of(P.ix, strand), P.ix.ratio, n, k);
     }
-    const uint32_t q = R.n ? R.q[0] : sa_value(dir_of(P.ix, strand), P.ix.ratio, n, k);
-    // direction: the record's dir is 0; + keeps it, - flips it
-    const uint64_t key = strand ? (uint64_t)n + 1u - q - (uint64_t)len - 1u : (uint64_t)q;
-    const uint32_t c = contig_of(P.koff, P.kcount, key, (uint64_t)len);
-    if (c == 0u) continue;
-    if (nout < P.cap)
-      store_mapping(P.out + (uint64_t)rd * P.cap + nout, P.kstart[c - 1] + (key - P.koff[c - 1]),
-                    c - 1u, rd, strand, nout > 0 ? 1u : 0u, len);
-    ++nout;
+    tot += R.n - 1u;
+    if (tot > P.filter) { st = 1u; break; }
+    uint64_t pos[kTextRows];
+    uint32_t chrom[kTextRows];               // contig + 1, 0: no alignment
+#pragma unroll
+    for (uint32_t j = 0; j < kTextRows; ++j) {
+      pos[j] = 0u;
+      chrom[j] = 0u;
+      if (j >= R.n) continue;
+      // direction: the record's dir is 0; + keeps it, - flips it
+      const uint64_t key = strand ? (uint64_t)n + 1u - R.q[j] - (uint64_t)len - 1u : (uint64_t)R.q[j];
+      chrom[j] = contig_of(P.koff, P.kcount, key, (uint64_t)len);
+      if (chrom[j]) pos[j] = P.kstart[chrom[j] - 1u] + (key - P.koff[chrom[j] - 1u]);
+    }
+    // within 10 bp on the int positions an earlier alignment drops a later
+    // one; the others are handed over from the last to the first
+#pragma unroll
+    for (int32_t a1 = (int32_t)kTextRows - 1; a1 >= 0; --a1) {
+      bool stays = chrom[a1] != 0u;
+#pragma unroll
+      for (int32_t a2 = 0; a2 < a1; ++a2) {
+        const int32_t d = (int32_t)((uint32_t)pos[a1] - (uint32_t)pos[a2]);
+        const int64_t ad = d < 0 ? -(int64_t)d : (int64_t)d;
+        if (chrom[a2] == chrom[a1] && ad < 10) stays = false;
+      }
+      if (!stays) continue;
+      if (nout < P.cap)
+        store_mapping(P.out + (uint64_t)rd * P.cap + nout, pos[a1], chrom[a1] - 1u, rd, strand,
+                      nout > 0 ? 1u : 0u, len);
+      ++nout;
+    }
   }
   P.counts[rd] = nout;
-  P.status[rd] = 0;
+  P.status[rd] = st;
 }
 
 __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
@@ -198,13 +210,7 @@ __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
     const uint8_t *W = P.reads + off;
     fmi_read_mapping *out = P.out + (uint64_t)rd * P.cap;
     const int32_t len = (int32_t)(P.offsets[rd + 1] - off);
-    const uint32_t K = P.ix.kmer_k && len >= (int32_t)P.ix.kmer_k ? P.ix.kmer_k : 0u;
-    uint32_t code = 0u, bad = 0u;
-    for (uint32_t j = 0; j < K; ++j) {
-      const uint32_t s = W[len - 1 - (int32_t)j];
-      bad |= s > 3u ? 1u : 0u;
-      code |= (s & 3u) << (2u * j);
-    }
+    const ReadBases<false> bases{W, nullptr};
     uint64_t tot = 0;
     uint32_t nout = 0;
     uint8_t st = 0;
@@ -214,11 +220,8 @@ __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
       const DevDir &D = dir_of(P.ix, dsel);
       uint32_t k, l;
       TextRows R;
-      const uint64_t e = K && !bad ? P.ix.kmer[dsel][dsel ? code ^ ((1u << (2u * K)) - 1u) : code]
-                                   : 0ull;
       uint32_t m = 0;
-      if (!bad && live_interval<false>(P.ix, dsel, dsel, W, len, nullptr, K, (uint32_t)e,
-                                       (uint32_t)(e >> 32), k, l, R)) {
+      if (live_interval<false>(P.ix, dsel, dsel, bases, len, k, l, R)) {
         if (R.n) { k = 0u; l = R.n - 1u; }             // the rows' suffixes are known
         tot += (uint64_t)(l - k);
         if (tot > P.filter) { st |= 1u; break; }
