@@ -631,13 +631,17 @@ def summarize_pmc(fetch_dir, write_dir, out_path, tuning, workload):
     def pick(acc, word):
         return [v for (k, _), v in sorted(acc.items(), key=lambda x: x[0][1]) if word in k]
 
-    # the staged search kernel of the mismatch-mode text-mode search (the
-    # last template argument, LDS staging, true), the call's dominant kernel
-    def staged(acc):
-        return [v for (k, _), v in sorted(acc.items(), key=lambda x: x[0][1])
-                if "search1_kernel<true, true, false, true," in k and k.split(">")[0].endswith("true")]
-    s_f = staged(fetch)
-    s_w = staged(write)
+    # the launches of one search of an expanded index, mismatch mode: the
+    # kernel of a thread per (read, strand), the kernel of a wave per read it
+    # leaves, and the state machine over the reads neither takes
+    names = ("search1_text_kernel<true>", "search1_wave_kernel<true>",
+             "search1_kernel<true, true, false, true,")
+
+    def search(acc):
+        calls = sum(1 for (k, _) in acc if names[0] in k)
+        return calls, sum(v for (k, _), v in acc.items() if any(w in k for w in names)) / calls
+    calls, kib_f = search(fetch)
+    _, kib_w = search(write)
     c_f, c_w = pick(fetch, "copy_kernel"), pick(write, "copy_kernel")
     g_f = pick(fetch, "gather_kernel<4>")
     copy_bytes = 1 << 30
@@ -645,10 +649,8 @@ def summarize_pmc(fetch_dir, write_dir, out_path, tuning, workload):
     write_copy = copy_bytes / (c_w[0] * 1024)
     # the first gather of the calibration runs over an index-sized buffer
     fetch_g64 = (1 << 24) * 64 / (g_f[0] * 1024)
-    kib_f = sum(s_f) / len(s_f)
-    kib_w = sum(s_w) / len(s_w)
     traffic = kib_f * 1024 * fetch_g64 + kib_w * 1024 * write_copy
-    d = {"workload": workload, "tuning": tuning, "dispatches": len(s_f),
+    d = {"workload": workload, "tuning": tuning, "dispatches": calls,
          "fetch_size_kib_per_launch": round(kib_f), "write_size_kib_per_launch": round(kib_w),
          "fetch_scale_64B_random": round(fetch_g64, 4), "fetch_scale_copy": round(fetch_copy, 4),
          "write_scale_copy": round(write_copy, 4), "traffic_bytes_per_launch": round(traffic)}
@@ -861,10 +863,14 @@ def search1_point(args, hpgfm, synth, preset, extras=True, cpu_baseline=True, se
                          "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBPS, 4),
                          "traffic": traffic},
             "traffic_source": traffic_src,
-            "kernel": ("fmi_search1_batch: fmi::read_records_kernel, then "
-                       "fmi::search1_kernel<true, true, false, %s, OWN, true> (reads staged in "
-                       "LDS), the unstaged kernel over the reads longer than 256 bases, "
-                       "fmi::text_rows_kernel" % ("true" if text_mode else "false")),
+            "kernel": ("fmi_search1_batch: fmi::read_records_kernel, " +
+                       ("fmi::search1_text_kernel (a thread per read and strand), "
+                        "fmi::search1_wave_kernel (a wave per read of wide intervals), "
+                        "fmi::search1_kernel over the reads they leave, "
+                        if text_mode else
+                        "fmi::search1_kernel<true, true, false, false, false, true> (reads "
+                        "staged in LDS), the unstaged kernel over the reads longer than 256 "
+                        "bases, ") + "fmi::text_rows_kernel"),
             "kernel_ms_mean": round(kernel_ms, 4),
             "alg_bytes_per_launch": alg_bytes,
             "lf_queries_per_launch": lf_steps,

@@ -384,7 +384,7 @@ int fmi_set_load_mode(uint32_t mode);
 int fmi_get_load_mode(uint32_t *mode);
 /* Whether fmi_search1_batch stages reads (the default, 1): a streaming
  * kernel packs each read into a 96-byte record (2-bit codes, N flags) in
- * the stream's scratch (100 bytes per read, for batches of at most 2^27
+ * the stream's scratch (104 bytes per read, for batches of at most 2^27
  * reads) and every lane of the persistent search holds its read in LDS, so
  * no step reads it from memory again; reads longer than 256 bases are
  * searched afterwards without staging.  0 reads the read from memory at
@@ -516,7 +516,7 @@ typedef struct fmi_seed_info {
  * each strand in row order (the reference's insertion order); entries past
  * region_cap are counted but not written.  *nseeds and *nrows are written
  * on the host: the call synchronises the stream (twice, for the seed and
- * row totals) and allocates its scratch (about 24 bytes per seed). */
+ * row totals) and allocates its scratch (about 16 bytes per seed). */
 int fmi_seed_map_batch(const fmi_index *ix, const uint8_t *d_reads, const uint64_t *d_offsets,
                        uint32_t nreads, uint32_t seed_len, uint32_t stride,
                        uint32_t filter_seed_mappings, fmi_seed_info *d_seed_info,
