@@ -634,7 +634,7 @@ def summarize_pmc(fetch_dir, write_dir, out_path, tuning, workload):
     # the launches of one search of an expanded index, mismatch mode: the
     # kernel of a thread per (read, strand), the kernel of a wave per read it
     # leaves, and the state machine over the reads neither takes
-    names = ("search1_text_kernel<true>", "search1_wave_kernel<true>",
+    names = ("search1_text_kernel<true", "search1_wave_kernel<true>",
              "search1_kernel<true, true, false, true,")
 
     def search(acc):

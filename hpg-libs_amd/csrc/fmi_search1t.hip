@@ -117,12 +117,18 @@ __device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uin
 // search1_wave_kernel, one with an anchor of less than kTextHalf bases or more
 // bases than a slot to search1_kernel; its record is written from the slot.
 // Bound by the latency of a pass's chain and the lines it reads (an entry,
-// contexts, suffixes, text and the records' rows), at 4 waves per SIMD (119
-// registers).  1 M reads of 150 bases over 64 Mbp: 576 us, where the records,
+// contexts, suffixes, text and the records' rows).  At 4 waves: 1 M reads of 150 bases over 64 Mbp: 576 us, where the records,
 // the state machine and its records' rows took 1284; 2 M over 3.1 Gbp 1552
 // of 2300; a request of 500 reads 43 of 500.
-template <bool MM_ONLY>
-__global__ __launch_bounds__(512) void search1_text_kernel(S1tParams P) {
+// MINW: the waves per SIMD the registers are held to.  4 (none spilled) where
+// every group of the batch is resident at once, and a read's own chain is
+// what counts; 6 (80 VGPRs, 26 spilled: three groups a CU instead of two)
+// beyond, where more lines in flight are worth the spills.  Calls: 1 M x 150 at
+// 64 Mbp 610 to 569 us, 2 M at 3.1 Gbp 1608 to 1460, 700 K of 50-250 with indels
+// and positions at 256 Mbp 627 to 557, but 500 reads 60 to 64.  5 waves (6
+// spilled) hold no third group.
+template <bool MM_ONLY, int MINW>
+__global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
   __shared__ uint32_t slots[kReadRecordWords * 256u];
   const uint64_t t64 = (uint64_t)blockIdx.x * 512u + threadIdx.x;
   const uint32_t rd = (uint32_t)(t64 >> 1), strand = (uint32_t)t64 & 1u;
@@ -330,11 +336,14 @@ hipError_t launch_search1_text(const DevIndex &ix, bool mm_only, uint32_t strand
               wide, wide_n, list,    list_n, nreads, strand_mask, cap};
   const dim3 g((uint32_t)((2ull * nreads + 511u) / 512u));
   const dim3 w(std::min<uint32_t>((nreads + 3u) / 4u, cus * 6u));   // resident (24 KB of LDS each)
+  const bool resident = g.x <= 2u * cus;   // two groups a CU at 4 waves
   if (mm_only) {
-    hipLaunchKernelGGL(search1_text_kernel<true>, g, dim3(512), 0, s, P);
+    if (resident) hipLaunchKernelGGL((search1_text_kernel<true, 4>), g, dim3(512), 0, s, P);
+    else hipLaunchKernelGGL((search1_text_kernel<true, 6>), g, dim3(512), 0, s, P);
     hipLaunchKernelGGL(search1_wave_kernel<true>, w, dim3(256), 0, s, P);
   } else {
-    hipLaunchKernelGGL(search1_text_kernel<false>, g, dim3(512), 0, s, P);
+    if (resident) hipLaunchKernelGGL((search1_text_kernel<false, 4>), g, dim3(512), 0, s, P);
+    else hipLaunchKernelGGL((search1_text_kernel<false, 6>), g, dim3(512), 0, s, P);
     hipLaunchKernelGGL(search1_wave_kernel<false>, w, dim3(256), 0, s, P);
   }
   return hipGetLastError();

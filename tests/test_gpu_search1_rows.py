@@ -74,3 +74,35 @@ def test_search1_rows(gpu_engine, copies, kmer):
     finally:
         batch.free()
         ix.close()
+
+
+@pytest.mark.parametrize("nreads", [131_072, 131_073])
+def test_search1_rows_batch_size(gpu_engine, copies, nreads):
+    """The last batch whose groups are all resident and the first past it
+    (registers held for more waves): the same reads over and over have the
+    records of the one batch that meets the oracle above."""
+    hp = gpu_engine
+    g, reads, offs, _ = copies
+    ix = hp.Index.build(g, 16).to_device()
+    ix.expand()
+    ix.kmer_table(11)
+    lens = np.diff(offs.astype(np.int64))
+    m = len(lens)
+    times = -(-nreads // m)
+    many = np.concatenate([[0], np.cumsum(np.tile(lens, times)[:nreads])]).astype(np.uint64)
+    few = hp.ReadBatch(reads, offs)
+    batch = hp.ReadBatch(np.tile(reads, times)[:int(many[-1])], many)
+    try:
+        for mode in (hp.MODE_EDIT, hp.MODE_MISMATCH):
+            wc, wh = hp.search1_batch(ix, few, cap=4, mode=mode)
+            counts, hits = hp.search1_batch(ix, batch, cap=4, mode=mode)
+            assert np.array_equal(counts, np.tile(wc, (times, 1))[:nreads])
+            stored = np.minimum(wc, 4)[..., None] > np.arange(4)
+            for t in range(times):
+                part = hits[t * m:min((t + 1) * m, nreads)]
+                keep = stored[:len(part)]
+                assert part[keep].tobytes() == wh[:len(part)][keep].tobytes()
+    finally:
+        batch.free()
+        few.free()
+        ix.close()
