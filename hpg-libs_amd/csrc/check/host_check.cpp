@@ -10,6 +10,9 @@
 //                              recomputed); format records of random fields
 //   host_check load PATH       load one index file, print its status
 //   host_check import DIR      import one reference directory, print status
+//   host_check items 32|64     share out a wavefront's items at and around the
+//                              most that each item type is taken for: every 64
+//                              of them are one wavefront's, once
 //
 // Exit status 0 unless a check fails (a sanitizer report aborts first).
 #include <cstdint>
@@ -22,6 +25,7 @@
 
 #include "../../../include/fmi.h"
 #include "../fmi_index.h"
+#include "../fmi_items.h"
 
 namespace {
 
@@ -125,12 +129,46 @@ int selftest(uint32_t seed, const std::string &tmp) {
   return 0;
 }
 
+// The steps of every 509th wavefront of a launch over `lanes` lanes of at most
+// `per_lane` items, 64 of which bring `total`.
+template <class T>
+int shares(uint64_t lanes, uint64_t per_lane, uint64_t total) {
+  const uint32_t parts = fmi::item_parts(lanes, per_lane);
+  for (uint32_t i = 0; i <= parts / 509u; ++i) {
+    const uint32_t part = i < parts / 509u ? 509u * i : parts - 1u;
+    uint64_t want = 64ull * part;
+    T base = (T)want;
+    if (want != (uint64_t)base) return fail("a wavefront starts at another place");
+    while (want < total) {
+      if ((uint64_t)base != want) return fail("a wavefront steps to another place");
+      want += 64ull * parts;
+      if (fmi::items_next<T>(base, (T)total, parts) != (want < total))
+        return fail(want < total ? "a wavefront ends early" : "a wavefront does not end");
+    }
+  }
+  return 0;
+}
+
+int items(uint32_t bits) {
+  std::vector<uint64_t> per{1, 63, 64, 65, 1000, 1ull << 20, fmi::kItems32 - 1, fmi::kItems32};
+  if (bits == 64) per.insert(per.end(), {fmi::kItems32 + 1, 1ull << 26, 1ull << 30});
+  for (uint64_t lanes : {1ull, 64ull, 65ull, 1000ull, 1ull << 20})
+    for (uint64_t p : per)
+      for (uint64_t total : {(uint64_t)1, p, 63 * p + 1, 64 * p - 1, 64 * p}) {
+        const int rc = bits == 32 ? shares<uint32_t>(lanes, p, total)
+                                  : shares<uint64_t>(lanes, p, total);
+        if (rc) return rc;
+      }
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-  if (argc < 3) return fail("usage: host_check selftest SEED [TMPDIR] | load PATH | import DIR");
+  if (argc < 3) return fail("usage: host_check selftest SEED [TMPDIR] | load PATH | import DIR | items BITS");
   const std::string cmd = argv[1];
   if (cmd == "selftest") return selftest((uint32_t)strtoul(argv[2], nullptr, 10), argc > 3 ? argv[3] : "/tmp");
+  if (cmd == "items") return items((uint32_t)strtoul(argv[2], nullptr, 10));
   if (cmd == "load") {
     printf("%d\n", load_status(argv[2]));
     return 0;

@@ -8,6 +8,7 @@
 
 #include "../../include/fmi.h"
 #include "fmi_internal.h"
+#include "fmi_items.h"
 
 namespace fmi {
 
@@ -541,7 +542,8 @@ __device__ __forceinline__ void wave_items(T count, uint32_t part, uint32_t part
     if (lane >= d) incl += v;
   }
   const T total = __shfl(incl, 63), excl = incl - count;
-  for (T base = 64u * (T)part; base < total; base += 64u * (T)parts) {
+  T base = 64u * (T)part;
+  for (bool more = base < total; more; more = items_next(base, total, parts)) {
     const T t = base + lane;
     uint32_t s = 0u;                             // the first lane whose items reach past t
 #pragma unroll

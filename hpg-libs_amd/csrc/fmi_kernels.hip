@@ -1765,16 +1765,6 @@ hipError_t launch_zero(uint32_t *p, uint32_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Wavefronts per 64 lanes of wave_items: one where there are enough to fill
-// the device twice (256 CUs of 32), else as many as do, at most one per 64
-// items the 64 lanes can bring.  Few wide intervals need them: 1 M rows of one
-// interval take 12 us, as a thread per row did, where 8192 took 18.
-static uint32_t item_parts(uint64_t lanes, uint64_t items_per_lane) {
-  const uint64_t waves = (lanes + 63) / 64;
-  const uint64_t fill = std::max<uint64_t>(16384 / std::max<uint64_t>(waves, 1), 1);
-  return (uint32_t)std::min<uint64_t>(fill, items_per_lane);
-}
-
 hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, const int64_t *l,
                          uint32_t stride, uint32_t nintervals, uint32_t cap, uint64_t *pos,
                          uint32_t *nrows, hipStream_t s) {
@@ -1782,7 +1772,7 @@ hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, co
   const uint64_t grid = ((uint64_t)nintervals + 255) / 256;
   if (grid == 0 || cap == 0) return hipSuccess;
   const dim3 g((uint32_t)grid, item_parts(nintervals, cap));
-  if (cap < (1u << 26)) hipLaunchKernelGGL(locate_kernel<uint32_t>, g, dim3(256), 0, s, P);
+  if (cap <= kItems32) hipLaunchKernelGGL(locate_kernel<uint32_t>, g, dim3(256), 0, s, P);
   else hipLaunchKernelGGL(locate_kernel<unsigned long long>, g, dim3(256), 0, s, P);
   return hipGetLastError();
 }
@@ -1837,7 +1827,7 @@ hipError_t launch_resolve(const DevIndex &ix, const fmi_hit *hits, const uint32_
   if (grid == 0 || cap == 0 || row_cap == 0) return hipSuccess;
   const uint64_t per_slot = (uint64_t)cap * row_cap;
   const dim3 g((uint32_t)grid, item_parts(2ull * nreads, per_slot));
-  if (per_slot < (1u << 26)) hipLaunchKernelGGL(resolve_kernel<uint32_t>, g, dim3(256), 0, s, P);
+  if (per_slot <= kItems32) hipLaunchKernelGGL(resolve_kernel<uint32_t>, g, dim3(256), 0, s, P);
   else hipLaunchKernelGGL(resolve_kernel<unsigned long long>, g, dim3(256), 0, s, P);
   return hipGetLastError();
 }
