@@ -26,6 +26,7 @@
 #include "fmi_device.h"
 #include "fmi_index.h"
 #include "fmi_internal.h"
+#include "fmi_kernels.h"
 #include "fmi_vhelper.h"
 #include "fmi_window.h"
 
@@ -57,27 +58,30 @@ __device__ __forceinline__ uint64_t owner(const uint64_t *base, uint64_t n, uint
   return lo;
 }
 
+// The last i in [lo, hi) with base[i] <= g (base is non-decreasing, base[lo] <=
+// g), by 64 probes a round of the whole wavefront, whose lanes all call it with
+// the same arguments.
+__device__ __forceinline__ uint64_t wave_last(const uint64_t *base, uint64_t lo, uint64_t hi,
+                                              uint64_t g) {
+  const uint32_t lane = threadIdx.x & 63u;
+  while (hi - lo > 1u) {
+    const uint64_t step = (hi - lo + 63u) / 64u, idx = lo + lane * step;
+    const uint64_t yes = __ballot(lane == 0u || (idx < hi && base[idx] <= g));
+    lo += (63u - (uint32_t)__builtin_clzll(yes)) * step;
+    hi = min(lo + step, hi);
+  }
+  return lo;
+}
+
 // owner for the lanes of a wavefront that hold consecutive g's (lane i:
-// g0 + i, g0 + i < total): the owners of the first and the last by 64 probes a
-// round of the whole wavefront, then a lane's own among those between them.
-// Every lane of the wavefront calls it; lanes past total get any answer.
+// g0 + i, g0 + i < total): the owners of the first and the last by the whole
+// wavefront, then a lane's own among those between them.  Every lane of the
+// wavefront calls it; lanes past total get any answer.
 __device__ __forceinline__ uint64_t wave_owner(const uint64_t *base, uint64_t n, uint64_t total,
                                                uint64_t g0) {
-  const uint32_t lane = threadIdx.x & 63u;
-  uint64_t ends[2];
-#pragma unroll
-  for (uint32_t e = 0; e < 2u; ++e) {
-    const uint64_t g = e ? min(g0 + 63u, total - 1u) : g0;
-    uint64_t lo = e ? ends[0] : 0u, hi = n;
-    while (hi - lo > 1u) {
-      const uint64_t step = (hi - lo + 63u) / 64u, idx = lo + lane * step;
-      const uint64_t yes = __ballot(lane == 0u || (idx < hi && base[idx] <= g));
-      lo += (63u - (uint32_t)__builtin_clzll(yes)) * step;
-      hi = min(lo + step, hi);
-    }
-    ends[e] = lo;
-  }
-  return ends[0] + owner(base + ends[0], ends[1] - ends[0] + 1u, g0 + lane);
+  const uint64_t a = wave_last(base, 0u, n, g0);
+  const uint64_t b = wave_last(base, a, n, min(g0 + 63u, total - 1u));
+  return a + owner(base + a, b - a + 1u, g0 + (threadIdx.x & 63u));
 }
 
 struct SeedParams {
@@ -94,7 +98,16 @@ struct SeedParams {
   // position), y the rows (or kRowKnown)
   uint2 *slots;
   uint64_t *sums;              // rows of seeds 64 i .. 64 i + 63
+  unsigned long long *most;    // the largest of them, if above kSeedBlockRows
 };
+
+// Rows of 64 seeds that one wavefront locates (seed_rows_kernel).
+constexpr uint32_t kSeedBlockRows = 2048;
+
+__device__ __forceinline__ void put_sum(const SeedParams &P, uint64_t i, uint64_t sum) {
+  P.sums[i] = sum;
+  if (sum > kSeedBlockRows) atomicMax(P.most, (unsigned long long)sum);
+}
 
 // A slot with one row whose text position is known (rows are below 2^32 - 2).
 constexpr uint32_t kRowKnown = 0xFFFFFFFFu;
@@ -190,7 +203,7 @@ __global__ __launch_bounds__(256) void seed_search_kernel(SeedParams P) {
       }
     }
     const uint64_t sum = wave_sum((uint64_t)rp + rm);
-    if (lane == 0u) P.sums[g0 >> 6] = sum;
+    if (lane == 0u) put_sum(P, g0 >> 6, sum);
   }
 }
 
@@ -285,7 +298,7 @@ __global__ __launch_bounds__(256) void seed_context_kernel(SeedParams P) {
       }
     }
     const uint64_t sum = wave_sum((uint64_t)rp + rm);
-    if (lane == 0u) P.sums[g0 >> 6] = sum;
+    if (lane == 0u) put_sum(P, g0 >> 6, sum);
   }
 }
 
@@ -299,83 +312,118 @@ struct RowParams {
   const uint64_t *kstart;
   uint64_t nseeds, nrows;      // rows to write
   uint32_t nreads, seed_len, stride, kcount;
+  uint32_t tile;               // rows of a wavefront, a multiple of 64
   fmi_seed_region *out;
 };
 
-// A wavefront takes 64 seeds, whose rows are neighbours in out, and shares
-// them out among its lanes (wave_items).  Bound by the slots read and the
-// regions written (and a line of SA per row that the search did not locate);
-// a thread per row took a binary search over the scanned row counts, 27
-// dependent loads for 94 M slots: 57 M rows in 3.2 ms (and 0.6 to scan the
-// counts), 2.0 as below.
-__global__ __launch_bounds__(256) void seed_rows_kernel(RowParams P) {
+// The region of one row at text position key.
+__device__ __forceinline__ void store_row(const RowParams &P, uint64_t row, uint64_t key,
+                                          uint32_t sid, uint32_t read, uint32_t seq_len,
+                                          uint32_t strand) {
+  const uint64_t seq_start = (uint64_t)sid * P.stride;
+  const uint64_t seq_end = seq_start + P.seed_len - 1;
+  const uint64_t len = seq_end - seq_start;
+  uint64_t lo = 0, size = P.kcount;            // binsearch, search/io.h:43-64
+  while (size > 0) {
+    const uint64_t w = size / 2;
+    if (P.koff[lo + w] <= key) { lo += w + 1; size -= w + 1; }
+    else size = w;
+  }
+  uint64_t start = 0, end = 0;
+  uint32_t valid = 0u;
+  if (lo >= 1 && key + len <= P.koff[lo]) {
+    start = P.kstart[lo - 1] + (key - P.koff[lo - 1]) + 1;
+    end = start + len;
+    valid = 1u;
+  }
+  const uint32_t ss = (uint16_t)(strand ? seq_len - seq_end - 1 : seq_start);
+  const uint32_t se = (uint16_t)(strand ? seq_len - seq_start - 1 : seq_end);
+  uint4 *dst = reinterpret_cast<uint4 *>(P.out + row);
+  dst[0] = make_uint4((uint32_t)start, (uint32_t)(start >> 32), (uint32_t)end,
+                      (uint32_t)(end >> 32));
+  dst[1] = make_uint4((uint32_t)lo, read, ss | (se << 16),
+                      (uint32_t)(uint16_t)sid | (strand << 16) | (valid << 24));
+}
+
+// Rows row .. end - 1 of out, all of seeds 64 b .. 64 b + 63, shared out among
+// the wavefront's lanes 64 at a time (every lane calls it).
+__device__ __forceinline__ void block_rows(const RowParams &P, uint64_t b, uint64_t row,
+                                           uint64_t end) {
   const DevDir &D = P.ix.d[0];
   const uint32_t lane = threadIdx.x & 63u;
-  for (uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; g0 < P.nseeds;
-       g0 += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t first = P.sum_base[g0 >> 6];
-    if (first >= P.nrows) continue;
-    const uint64_t own = wave_owner(P.seed_base, P.nreads, P.nseeds, g0);
-    const bool mine = g0 + lane < P.nseeds;
-    uint4 sl = make_uint4(0u, 0u, 0u, 0u);         // + and - of the lane's seed
-    uint32_t seed = 0u, rd = 0u, rlen = 0u;
-    if (mine) {
-      sl = reinterpret_cast<const uint4 *>(P.slots)[g0 + lane];
-      rd = (uint32_t)own;
-      seed = (uint32_t)(g0 + lane - P.seed_base[own]);
-      rlen = (uint32_t)(P.offsets[own + 1] - P.offsets[own]);
-    }
-    const uint32_t rp = sl.y == kRowKnown ? 1u : sl.y, rm = sl.w == kRowKnown ? 1u : sl.w;
-    uint64_t done = 0;                             // rows of the rounds before
-    const uint64_t rows = (uint64_t)rp + rm, total = wave_sum(rows);
-    unsigned long long incl = rows;                // rows of lanes 0..i
+  const uint64_t first = P.sum_base[b], g0 = 64u * b;
+  const uint64_t own = wave_owner(P.seed_base, P.nreads, P.nseeds, g0);
+  uint4 sl = make_uint4(0u, 0u, 0u, 0u);           // + and - of the lane's seed
+  uint32_t seed = 0u, rd = 0u, rlen = 0u;
+  if (g0 + lane < P.nseeds) {
+    sl = reinterpret_cast<const uint4 *>(P.slots)[g0 + lane];
+    rd = (uint32_t)own;
+    seed = (uint32_t)(g0 + lane - P.seed_base[own]);
+    rlen = (uint32_t)(P.offsets[own + 1] - P.offsets[own]);
+  }
+  const uint32_t rp = sl.y == kRowKnown ? 1u : sl.y, rm = sl.w == kRowKnown ? 1u : sl.w;
+  const uint64_t rows = (uint64_t)rp + rm;
+  unsigned long long incl = rows;                  // rows of lanes 0..i
 #pragma unroll
-    for (uint32_t d = 1u; d < 64u; d <<= 1) {
-      const unsigned long long v = __shfl_up(incl, d);
-      if (lane >= d) incl += v;
-    }
-    const unsigned long long excl = incl - rows;
-    for (; done < total && first + done < P.nrows; done += 64u) {
-      const unsigned long long t = done + lane;
-      uint32_t o = 0u;                             // the first lane whose rows reach past t
+  for (uint32_t d = 1u; d < 64u; d <<= 1) {
+    const unsigned long long v = __shfl_up(incl, d);
+    if (lane >= d) incl += v;
+  }
+  const unsigned long long excl = incl - rows;
+  for (; row < end; row += 64u) {
+    const unsigned long long t = row - first + lane;
+    uint32_t o = 0u;                               // the first lane whose rows reach past t
 #pragma unroll
-      for (uint32_t d = 32u; d >= 1u; d >>= 1)
-        if (__shfl(incl, (int)(o + d - 1u)) <= t) o += d;
-      const int src = (int)min(o, 63u);
-      uint64_t j = t - __shfl(excl, src);
-      const uint32_t np = __shfl(rp, src);
-      const uint32_t strand = j >= np ? 1u : 0u;
-      const uint32_t px = __shfl(sl.x, src), py = __shfl(sl.y, src);
-      const uint32_t mx = __shfl(sl.z, src), my = __shfl(sl.w, src);
-      const uint32_t sid = __shfl(seed, src), read = __shfl(rd, src), seq_len = __shfl(rlen, src);
-      if (t >= total || first + t >= P.nrows) continue;
-      if (strand) j -= np;
-      const uint32_t x = strand ? mx : px;
-      const bool known = (strand ? my : py) == kRowKnown;
-      const uint64_t key = known ? x : sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)(x + j));
-      const uint64_t seq_start = (uint64_t)sid * P.stride;
-      const uint64_t seq_end = seq_start + P.seed_len - 1;
-      const uint64_t len = seq_end - seq_start;
-      uint64_t lo = 0, size = P.kcount;            // binsearch, search/io.h:43-64
-      while (size > 0) {
-        const uint64_t w = size / 2;
-        if (P.koff[lo + w] <= key) { lo += w + 1; size -= w + 1; }
-        else size = w;
-      }
-      uint64_t start = 0, end = 0;
-      uint32_t valid = 0u;
-      if (lo >= 1 && key + len <= P.koff[lo]) {
-        start = P.kstart[lo - 1] + (key - P.koff[lo - 1]) + 1;
-        end = start + len;
-        valid = 1u;
-      }
-      const uint32_t ss = (uint16_t)(strand ? seq_len - seq_end - 1 : seq_start);
-      const uint32_t se = (uint16_t)(strand ? seq_len - seq_start - 1 : seq_end);
-      uint4 *dst = reinterpret_cast<uint4 *>(P.out + first + t);
-      dst[0] = make_uint4((uint32_t)start, (uint32_t)(start >> 32), (uint32_t)end,
-                          (uint32_t)(end >> 32));
-      dst[1] = make_uint4((uint32_t)lo, read, ss | (se << 16),
-                          (uint32_t)(uint16_t)sid | (strand << 16) | (valid << 24));
+    for (uint32_t d = 32u; d >= 1u; d >>= 1)
+      if (__shfl(incl, (int)(o + d - 1u)) <= t) o += d;
+    const int src = (int)min(o, 63u);
+    uint64_t j = t - __shfl(excl, src);
+    const uint32_t np = __shfl(rp, src);
+    const uint32_t strand = j >= np ? 1u : 0u;
+    const uint32_t px = __shfl(sl.x, src), py = __shfl(sl.y, src);
+    const uint32_t mx = __shfl(sl.z, src), my = __shfl(sl.w, src);
+    const uint32_t sid = __shfl(seed, src), read = __shfl(rd, src), seq_len = __shfl(rlen, src);
+    if (row + lane >= end) continue;
+    if (strand) j -= np;
+    const uint32_t x = strand ? mx : px;
+    const bool known = (strand ? my : py) == kRowKnown;
+    const uint64_t key = known ? x : sa_value(D, P.ix.ratio, P.ix.n, (uint32_t)(x + j));
+    store_row(P, row + lane, key, sid, read, seq_len, strand);
+  }
+}
+
+// A wavefront takes the rows of 64 seeds, which are neighbours in out.  Bound by
+// the slots read and the regions written (and a line of SA per row that the
+// search did not locate); a thread per row took a binary search over the
+// scanned row counts, 27 dependent loads for 94 M slots: 57 M rows in 3.2 ms
+// (and 0.6 to scan the counts), 2.0 as below.
+// TILED: a wavefront takes `tile` neighbouring rows instead, of as many seeds as
+// they are.  A batch is taken so where some 64 seeds bring more than kSeedBlockRows
+// rows: those of one wavefront are a chain, 0.95 us per 64 (6.5 on a compact
+// index), and a single seed of 2 M rows took 29.4 ms (203), 0.1 (0.2) by tiles.
+// Where all bring fewer, tiles look most of the 64 seeds up twice: 1.4 M rows of
+// 1.7 M seeds TILECOST.
+template <bool TILED>
+__global__ __launch_bounds__(256) void seed_rows_kernel(RowParams P) {
+  const uint64_t nsums = (P.nseeds + 63u) / 64u;
+  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x >> 6);
+  if (!TILED) {
+    for (uint64_t b = wave; b < nsums; b += waves) {
+      const uint64_t row = P.sum_base[b], end = min(P.sum_base[b + 1u], P.nrows);
+      if (row < end) block_rows(P, b, row, end);
+    }
+    return;
+  }
+  for (uint64_t at = wave * P.tile; at < P.nrows; at += waves * P.tile) {
+    const uint64_t last = min(at + P.tile, P.nrows);
+    uint64_t row = at, b = wave_last(P.sum_base, 0u, nsums, at);
+    for (;;) {
+      const uint64_t end = min(P.sum_base[b + 1u], last);
+      block_rows(P, b, row, end);
+      if (end == last) break;
+      row = end;
+      b = P.sum_base[b + 2u] > row ? b + 1u : wave_last(P.sum_base, b + 1u, nsums, row);
     }
   }
 }
@@ -831,7 +879,7 @@ int seed_map(const fmi_index *ix, const uint8_t *reads, const uint64_t *offsets,
   uint2 *slots = nullptr;
   void *tmp = nullptr;
   size_t tmp_bytes = 0, need = 0;
-  uint64_t nseeds = 0, nrows = 0, nsums = 0;
+  uint64_t nseeds = 0, nsums = 0, totals[2] = {0, 0};   // rows; the most of 64 seeds
   *nseeds_out = 0;
   *nrows_out = 0;
   SEED_TRY(hipMalloc(&cnt, (uint64_t)(nreads + 1) * 8));
@@ -849,11 +897,12 @@ int seed_map(const fmi_index *ix, const uint8_t *reads, const uint64_t *offsets,
   if (nseeds == 0) goto done;
   nsums = (nseeds + 63) / 64;
   SEED_TRY(hipMalloc(&slots, 2 * nseeds * sizeof(uint2)));
-  SEED_TRY(hipMalloc(&sums, (nsums + 1) * 8));
+  SEED_TRY(hipMalloc(&sums, (nsums + 2) * 8));
+  SEED_TRY(launch_zero(reinterpret_cast<uint32_t *>(sums + nsums + 1), 2, s));
   {
     SeedParams P{ix->dev, reads, offsets, base, nseeds, nreads, seed_len, stride,
                  (int32_t)(filter > (uint32_t)INT32_MAX ? INT32_MAX : filter), info, info_cap,
-                 slots, sums};
+                 slots, sums, reinterpret_cast<unsigned long long *>(sums + nsums + 1)};
     const uint32_t K = ix->dev.kmer_k;
     if (!info && ix->dev.d[0].ctx && K && seed_len >= K && seed_len <= 32u)
       seed_context_kernel<<<grid_for(nseeds), 256, 0, s>>>(P);
@@ -872,14 +921,22 @@ int seed_map(const fmi_index *ix, const uint8_t *reads, const uint64_t *offsets,
   }
   SEED_TRY(rocprim::exclusive_scan(tmp, need, sums, sums, (uint64_t)0, nsums + 1,
                                    rocprim::plus<uint64_t>(), s));
-  SEED_TRY(hipMemcpyAsync(&nrows, sums + nsums, 8, hipMemcpyDeviceToHost, s));
+  SEED_TRY(hipMemcpyAsync(totals, sums + nsums, 16, hipMemcpyDeviceToHost, s));
   SEED_TRY(hipStreamSynchronize(s));
-  *nrows_out = nrows;
-  if (nrows && region_cap && regions) {
+  *nrows_out = totals[0];
+  if (totals[0] && region_cap && regions) {
+    // tiles of 512 rows (128 on a compact index, whose rows take 7 times as
+    // long: 1.12 ms for 18 M of few seeds, 1.39 at 512), smaller where they
+    // would be fewer wavefronts than fill the device twice
+    const uint64_t rows = std::min(totals[0], region_cap);
+    const uint32_t tile = (uint32_t)std::clamp<uint64_t>(rows / 16384 / 64 * 64, 64,
+                                                         ix->dev.d[0].sa ? 512 : 128);
     RowParams R{ix->dev, offsets, base, sums, slots, ix->d_koffset, ix->d_kstart, nseeds,
-                nrows < region_cap ? nrows : region_cap, nreads, seed_len, stride,
-                (uint32_t)ix->kstart.size(), regions};
-    seed_rows_kernel<<<grid_for(nseeds), 256, 0, s>>>(R);
+                rows, nreads, seed_len, stride, (uint32_t)ix->kstart.size(), tile, regions};
+    if (totals[1] > rows / 2048)
+      seed_rows_kernel<true><<<grid_for((rows + tile - 1) / tile * 64), 256, 0, s>>>(R);
+    else
+      seed_rows_kernel<false><<<grid_for(nseeds), 256, 0, s>>>(R);
     SEED_TRY(hipGetLastError());
   }
 done:

@@ -6,6 +6,9 @@ coordinate on the right strand, with the one-short length of bwt.c:1214;
 occurrences crossing a contig end yield none; the cumulative filter skips
 exactly the strands the reference's running `int` count exceeds.
 GPU: fmi_seed_map_batch equals the oracle region for region, in order."""
+import ctypes as C
+import time
+
 import numpy as np
 import pytest
 
@@ -176,5 +179,66 @@ def test_gpu_seed_map_by_context(gpu_engine, kmer, seed_len, stride):
                                                     region_cap=cap, with_info=False)
                 assert nr2 == nr and regs.tobytes() == want[:cap].tobytes()
     finally:
+        batch.free()
+        ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("expanded", [False, True])
+def test_gpu_seed_map_rows_of_few_seeds(gpu_engine, expanded):
+    """Seeds whose rows are many more than a wavefront writes at a time -- a run
+    of one base and 700 exact copies, among seeds of no row -- equal to the
+    oracle, whole and at every edge of a tile of rows; and one seed of 300,000
+    rows, which has to be the work of the whole device: 0.1 ms where it is, 4.4
+    ms (30 on a compact index) where one wavefront writes them all."""
+    hp = gpu_engine
+    rng = np.random.default_rng(71)
+    n = 700_000
+    g = rng.integers(0, 4, n).astype(np.uint8)
+    g[1000:1000 + 1500] = 2
+    for i in range(700):
+        g[10_000 + 60 * i:10_030 + 60 * i] = g[10_000:10_030]
+    g[390_000:690_030] = 0
+    g[389_999] = g[690_030] = 1
+    koff, kstart = karyotype(n, [60_000])
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(kstart, kstart + np.diff(koff) - 1)
+    ix.to_device()
+    if expanded:
+        ix.expand()
+        ix.kmer_table(9)
+    o = fo.Oracle(g, ratio=8)
+    reads = [np.full(33, 2, np.uint8), g[10_000:10_030]]
+    reads += [rng.integers(0, 4, 1000).astype(np.uint8) for _ in range(4)]
+    reads += [g[10_000:10_024], g[200_000:200_030], synth.revcomp(g[10_000:10_030])]
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads).astype(np.uint8), offs)
+    want = []
+    for i, W in enumerate(reads):
+        regs, _ = o.seed_map(W, 18, 3, 1 << 30, koff, kstart)
+        regs = regs.copy()
+        regs["read"] = i
+        want.append(regs)
+    want = np.concatenate(want)
+    one = hp.ReadBatch(np.zeros(20, np.uint8), np.array([0, 20], np.uint64))
+    try:
+        assert len(want) > 10_000
+        for cap in (None, 1, 63, 64, 65, 511, 512, 513, len(want) - 1):
+            _, nr, regs, _ = hp.seed_map_batch(ix, batch, 18, 3, 1 << 30, region_cap=cap,
+                                               with_info=False)
+            assert nr == len(want) and regs.tobytes() == want[:cap].tobytes()
+        L, got = hp.lib(), (C.c_uint64(), C.c_uint64())
+        rows = hp.DeviceBuffer(32 * 400_000)
+        took = []
+        for _ in range(5):
+            t = time.perf_counter()
+            hp.check(L.fmi_seed_map_batch(ix.h, one.d_reads.ptr, one.d_offsets.ptr, 1, 18, 5, 1 << 30,
+                                          None, 0, rows.ptr, 400_000, C.byref(got[0]),
+                                          C.byref(got[1]), None))
+            took.append(time.perf_counter() - t)
+        rows.free()
+        assert got[1].value == 300_013 and min(took) < 1.5e-3, (got[1].value, took)
+    finally:
+        one.free()
         batch.free()
         ix.close()
