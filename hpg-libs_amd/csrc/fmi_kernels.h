@@ -44,13 +44,14 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
                           void *staged = nullptr);
 // The staged launch's first part on an expanded index (fmi_search1t.hip): the
 // reads searched on the text; those it leaves are appended to list, with their
-// records in rec.  wide: scratch for as many reads; wide_n and list_n are
-// zeroed by the caller.
+// records in rec, or, longer than a slot, stored from wide[nreads - 1] downward.
+// wide: nreads entries, of which the others are scratch; wide_n, long_n and
+// list_n are zeroed by the caller.
 hipError_t launch_search1_text(const DevIndex &ix, bool mm_only, uint32_t strand_mask,
                                const uint8_t *reads, const uint64_t *offsets, uint32_t nreads,
                                uint32_t cap, fmi_hit *hits, uint32_t *counts, uint32_t *rec,
-                               uint32_t *wide, uint32_t *wide_n, uint32_t *list, uint32_t *list_n,
-                               uint32_t cus, hipStream_t s);
+                               uint32_t *wide, uint32_t *wide_n, uint32_t *long_n, uint32_t *list,
+                               uint32_t *list_n, uint32_t cus, hipStream_t s);
 hipError_t launch_zero(uint32_t *p, uint32_t n, hipStream_t s);
 // Byte fill of bytes bytes with v (a kernel, so a captured graph holds no
 // memset node).

@@ -244,8 +244,9 @@ struct S1Params {
   uint32_t refill_min;             // idle lanes before a wave takes new tasks
   uint32_t split;                  // 1: a task is one strand of a read (staged, both asked)
   const uint4 *rec;                // staged launch: the read records (kRecWords words each)
-  const uint32_t *list;            // when set: the tasks are list[0 .. *list_n)
-  const uint32_t *list_n;
+  const uint32_t *list;            // when set: the tasks are list[0 .. *list_n), or
+  const uint32_t *list_n;          // with list_dir -1 list[0], list[-1], ...
+  int32_t list_dir;
 };
 
 // The staged launch keeps every lane's read in LDS for the whole task: a
@@ -1070,6 +1071,10 @@ struct S1 {
   }
 };
 
+__device__ __forceinline__ uint32_t listed(const S1Params &P, uint32_t i) {
+  return P.list[(int64_t)P.list_dir * i];
+}
+
 __device__ __forceinline__ uint32_t lane_id() {
   return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }
@@ -1134,16 +1139,13 @@ void search1_kernel(S1Params P) {
           wbase = wq_next;
           wend = min(wbase + 64u, wq_end);
           if (wbase + lane < wend) {
-            const uint32_t h_task = P.list ? P.list[wbase + lane] : wbase + lane;
+            const uint32_t h_task = P.list ? listed(P, wbase + lane) : wbase + lane;
             if (LDS) {
               const uint32_t h_read = h_task >> P.split;
               const uint32_t len = (uint32_t)(P.offsets[h_read + 1] - P.offsets[h_read]);
               h_len = len > kStagedMaxLen ? 0xFFFFFFFFu : len;   // longer: the unstaged kernel's
             } else {
-              // of a list the reads that fit a slot are the staged kernel's
-              if (P.list && P.offsets[h_task + 1] - P.offsets[h_task] <= kStagedMaxLen)
-                h_len = 0xFFFFFFFFu;
-              else m.task_info(h_task, h_off, h_len, h_kc0, h_kc1);
+              m.task_info(h_task, h_off, h_len, h_kc0, h_kc1);
             }
           }
         }
@@ -1152,7 +1154,7 @@ void search1_kernel(S1Params P) {
         const uint32_t avail = wend - wq_next;
         const int src = (int)((wq_next - wbase + rank) & 63u);   // the holder of task wq_next + rank
         uint32_t task = wq_next + rank;
-        if (P.list && rank < avail) task = P.list[task];
+        if (P.list && rank < avail) task = listed(P, task);
         const uint32_t len = __shfl(h_len, src);
         if (LDS) {
           if (L.phase == PH_IDLE && rank < avail && len != 0xFFFFFFFFu) m.stage_with(task, len);
@@ -1161,7 +1163,7 @@ void search1_kernel(S1Params P) {
           const uint32_t kc1 = __shfl(h_kc1, src);
           const uint32_t off_lo = __shfl((uint32_t)h_off, src);
           const uint32_t off_hi = __shfl((uint32_t)(h_off >> 32), src);
-          if (L.phase == PH_IDLE && rank < avail && len != 0xFFFFFFFFu)
+          if (L.phase == PH_IDLE && rank < avail)
             m.start_with(task, ((uint64_t)off_hi << 32) | off_lo, len, kc0, kc1);
         }
         wq_next += min(avail, nidle);
@@ -1184,15 +1186,18 @@ void search1_kernel(S1Params P) {
 // The rows of the records search1_kernel stored as text positions (k's high
 // word kTextRowTag, l = q): k = l = ISA[q] in the record's direction (dir ^
 // strand: the pass's direction).  One thread per (read, strand) slot, of the
-// listed reads where there is a list.
+// reads list[0 .. *list_n) and far[0], far[-1], ... (*far_n) where there are lists.
 __global__ __launch_bounds__(256) void text_rows_kernel(DevIndex ix, fmi_hit *hits,
                                                         const uint32_t *counts, uint32_t nslots,
                                                         uint32_t cap, const uint32_t *list,
-                                                        const uint32_t *list_n) {
-  const uint64_t n = list ? 2ull * *list_n : nslots;
+                                                        const uint32_t *list_n, const uint32_t *far,
+                                                        const uint32_t *far_n) {
+  const uint64_t near = list ? 2ull * *list_n : nslots, n = list ? near + 2ull * *far_n : nslots;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t t = list ? 2u * list[i >> 1] + (uint32_t)(i & 1u) : (uint32_t)i;
+    uint32_t t = (uint32_t)i;
+    if (list)
+      t = 2u * (i < near ? list[i >> 1] : far[-(int64_t)((i - near) >> 1)]) + (uint32_t)(i & 1u);
     const uint32_t c = min(counts[t], cap);
     uint4 *h = reinterpret_cast<uint4 *>(hits + (size_t)t * cap);
     for (uint32_t j = 0; j < c; ++j) {
@@ -1641,32 +1646,36 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
                           void *staged) {
   const uint32_t ntasks = nreads;   // one task per read (both strands in turn)
   S1Params P{ix, reads, offsets, hits, counts, queue, stats, ntasks, strand_mask, cap, chunk,
-             refill_min, 0u, nullptr, nullptr, nullptr};
+             refill_min, 0u, nullptr, nullptr, nullptr, 1};
   if (ntasks == 0) return hipSuccess;
   const bool text = ix.text != nullptr;   // expanded index: text mode
+  const uint32_t *list = nullptr, *list_n = nullptr, *far = nullptr, *far_n = nullptr;
   if (persistent) {
     if (grid_persistent == 0 || chunk == 0 || refill_min == 0 || refill_min > 64)
       return hipErrorInvalidValue;
     const dim3 g(grid_persistent), b(256);
     if (staged && !count && ntasks <= kStagedMaxTasks) {
       // scratch: [0] the unstaged kernel's work counter, [1] the list's
-      // length, [2] the wide list's; the list from byte 64; the records from
-      // the next 128 bytes, then the wide list
+      // length, [2] the wide list's, [3] the long reads'; the list from byte
+      // 64; the records from the next 128 bytes, then the wide list and, from
+      // its end downward, the long reads
       uint32_t *head = static_cast<uint32_t *>(staged);
-      uint32_t *list = head + 16;
+      uint32_t *left = head + 16;
       uint32_t *rec = reinterpret_cast<uint32_t *>(static_cast<char *>(staged) +
                                                    ((64ull + 4ull * ntasks + 127ull) & ~127ull));
-      hipError_t e = launch_zero(head, 3, s);
+      hipError_t e = launch_zero(head, 4, s);
       if (e != hipSuccess) return e;
       P.rec = reinterpret_cast<const uint4 *>(rec);
       if (text) {
         // on the text first; the two kernels below take the reads it leaves
+        uint32_t *wide = rec + (uint64_t)kRecWords * ntasks;
         e = launch_search1_text(ix, mm_only, strand_mask, reads, offsets, ntasks, cap, hits,
-                                counts, rec, rec + (uint64_t)kRecWords * ntasks, head + 2, list,
-                                head + 1, 256u, s);
+                                counts, rec, wide, head + 2, head + 3, left, head + 1, 256u, s);
         if (e != hipSuccess) return e;
-        P.list = list;
-        P.list_n = head + 1;
+        P.list = list = left;
+        P.list_n = list_n = head + 1;
+        far = wide + (ntasks - 1u);
+        far_n = head + 3;
       } else {
         // a strand a task: a lane's chain is half as long, and a lane that ends
         // early takes the next (200 K
@@ -1676,7 +1685,7 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
           P.split = 1u;
           P.ntasks = 2u * ntasks;
         }
-        RecParams R{reads, offsets, ntasks, rec, list, head + 1};
+        RecParams R{reads, offsets, ntasks, rec, left, head + 1};
         hipLaunchKernelGGL(read_records_kernel, dim3((uint32_t)((8ull * ntasks + 255) / 256)),
                            dim3(256), 0, s, R);
       }
@@ -1690,11 +1699,12 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
       if (mm_only) FMI_S1_STAGED(true);
       else FMI_S1_STAGED(false);
 #undef FMI_S1_STAGED
-      // the reads longer than a slot, unstaged, from the list
+      // the reads longer than a slot, unstaged, from their list
       P.split = 0u;
       P.rec = nullptr;
-      P.list = list;
-      P.list_n = head + 1;
+      P.list = text ? far : left;
+      P.list_n = text ? far_n : head + 1;
+      P.list_dir = text ? -1 : 1;
       P.queue = head;
     }
 #define FMI_S1_LAUNCH(MM, CNT)                                                                \
@@ -1725,8 +1735,8 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
   if (!count && ix.text != nullptr && cap > 0) {
     const uint64_t nslots = 2ull * ntasks, grid = (nslots + 255) / 256;
     hipLaunchKernelGGL(text_rows_kernel,
-                       dim3((uint32_t)(P.list ? std::min<uint64_t>(grid, 1024u) : grid)), dim3(256),
-                       0, s, ix, hits, counts, (uint32_t)nslots, cap, P.list, P.list_n);
+                       dim3((uint32_t)(list ? std::min<uint64_t>(grid, 1024u) : grid)), dim3(256),
+                       0, s, ix, hits, counts, (uint32_t)nslots, cap, list, list_n, far, far_n);
   }
   return hipGetLastError();
 }

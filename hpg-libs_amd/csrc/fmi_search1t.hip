@@ -30,10 +30,15 @@ struct S1tParams {
   fmi_hit *hits;
   uint32_t *counts;
   uint32_t *rec;                   // the left reads' records (kReadRecordWords words each)
-  uint32_t *wide, *wide_n;         // the reads left to search1_wave_kernel
-  uint32_t *list, *list_n;         // the reads left to search1_kernel
+  // the reads left to search1_wave_kernel, and from wide[nreads - 1] downward
+  // those longer than a slot, left to search1_kernel unstaged
+  uint32_t *wide, *wide_n, *long_n;
+  uint32_t *list, *list_n;         // the reads left to search1_kernel staged
   uint32_t nreads, strand_mask, cap;
 };
+
+// Where a read goes on: nowhere, in search1_wave_kernel, in search1_kernel.
+enum : uint32_t { kDone = 0u, kToWave = 1u, kToList = 2u };
 
 // Anchor halves shorter than this go to search1_kernel at once: they have more
 // than kTextRows rows in a repeat (and from 3.1 Gbp, 4^16, by chance), and the
@@ -66,11 +71,12 @@ __device__ __forceinline__ void add_string(S1tOut &O, const DevDir &D, uint32_t 
 }
 
 // One pass (0: the right half backward on the pair's first index, then the
-// left; 1: the left half forward on the second, then the right); false when
-// the anchor has more rows than it can take.
+// left; 1: the left half forward on the second, then the right); where the
+// read goes on when the anchor has more rows than it can take.
 template <bool MM_ONLY>
-__device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uint32_t strand,
-                                          const ReadBases<true> &rd, int32_t len, S1tOut &O) {
+__device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass, uint32_t strand,
+                                              const ReadBases<true> &rd, int32_t len,
+                                              S1tOut &O) {
   const uint32_t dsel = pass ^ strand;
   const DevDir &D = dir_of(ix, dsel);
   const int32_t half = len / 2, d = pass ? 1 : -1, p0 = pass ? 0 : len - 1;
@@ -78,7 +84,8 @@ __device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uin
   TextRows R;
   uint32_t k, l;
   const uint32_t found = search_rows<true>(ix, dsel, strand, rd, p0, d, m0, R, k, l);
-  if (found != kRowsFew) return found == kRowsNone;
+  if (found == kRowsNone) return kDone;
+  if (found == kRowsMany) return kToWave;
   int32_t run[kTextRows] = {-1, -1, -1, -1};
 #pragma unroll
   for (uint32_t j = 0; j < kTextRows; ++j)
@@ -109,7 +116,7 @@ __device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uin
       }
     if (rows) O.add(D, first, rows, 0, -1, len - 1, 0, 0u, 0u, 0u, 0u);
   }
-  return true;
+  return kDone;
 }
 
 // A thread per (read, strand); a read's two threads pack it into one LDS slot.
@@ -130,6 +137,7 @@ __device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uin
 template <bool MM_ONLY, int MINW>
 __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
   __shared__ uint32_t slots[kReadRecordWords * 256u];
+  __shared__ uint32_t ids[256], nids, narrived;    // the group's left reads
   const uint64_t t64 = (uint64_t)blockIdx.x * 512u + threadIdx.x;
   const uint32_t rd = (uint32_t)(t64 >> 1), strand = (uint32_t)t64 & 1u;
   const bool mine = t64 < 2ull * P.nreads;
@@ -166,45 +174,77 @@ __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
       slot[(16u + u) * 256u] = (uint32_t)(fl >> mis);
     }
   }
+  if (threadIdx.x == 0u) nids = narrived = 0u;
   __syncthreads();
-  bool left = false;
+  uint32_t left = kDone;
   if (mine) {
     const bool asked = ((P.strand_mask >> strand) & 1u) != 0u;
     S1tOut O{P.hits + (uint64_t)t64 * P.cap, P.cap, 0u, strand};
     if (!staged || len / 2 < kTextHalf) {
-      left = true;
+      left = kToList;
     } else if (asked) {
       const ReadBases<true> bases{nullptr, slot};
-      for (uint32_t pass = 0; pass < 2u && !left; ++pass)
-        left = !text_pass<MM_ONLY>(P.ix, pass, strand, bases, len, O);
+      for (uint32_t pass = 0; pass < 2u && left == kDone; ++pass)
+        left = text_pass<MM_ONLY>(P.ix, pass, strand, bases, len, O);
     }
     P.counts[t64] = O.cnt;
   }
-  // the left reads: a wavefront takes their places in a list together
-  const uint64_t any = __ballot(left);
-  const uint64_t reads = (any | (any >> 1)) & 0x5555555555555555ull;
-  if (reads == 0ull) return;
-  const bool towave = staged && len / 2 >= kTextHalf;
+  // the left reads, their records first
+  const uint64_t pair = 0x5555555555555555ull;
+  uint64_t wide = __ballot(left == kToWave), list = __ballot(left == kToList);
+  list = (list | (list >> 1)) & pair;
+  wide = (wide | (wide >> 1)) & pair & ~list;      // a strand's wider anchor decides
   const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t me = 1ull << (lane & ~1u);
-  const uint64_t towide = reads & __ballot(towave), tolist = reads & ~__ballot(towave);
-  uint32_t at_wide = 0u, at_list = 0u;
-  if (lane == 0u) {
-    if (towide) at_wide = atomicAdd(P.wide_n, (uint32_t)__popcll(towide));
-    if (tolist) at_list = atomicAdd(P.list_n, (uint32_t)__popcll(tolist));
-  }
-  at_wide = __shfl(at_wide, 0);
-  at_list = __shfl(at_list, 0);
-  if (!(reads & me)) return;
-  if (strand == 0u) {
-    if (towave) P.wide[at_wide + (uint32_t)__popcll(towide & (me - 1ull))] = rd;
-    else P.list[at_list + (uint32_t)__popcll(tolist & (me - 1ull))] = rd;
-  }
-  if (staged) {
+  const uint64_t me = 1ull << (lane & ~1u), any = wide | list;
+  if ((any & me) && staged) {
     uint4 *out = reinterpret_cast<uint4 *>(P.rec + (uint64_t)rd * kReadRecordWords);
     for (uint32_t i = strand; i < kReadRecordWords / 4u; i += 2u)
       out[i] = make_uint4(slot[(4u * i) * 256u], slot[(4u * i + 1u) * 256u],
                           slot[(4u * i + 2u) * 256u], slot[(4u * i + 3u) * 256u]);
+  }
+  // The group's last wavefront to come here appends them all to the lists: an
+  // atomic per group.  One per wavefront, 3125 to one address, took 30 of the
+  // 42 us that listing 100 K reads of 20 bases took.
+  uint32_t at = 0u;
+  if (lane == 0u && any) at = atomicAdd(&nids, (uint32_t)__popcll(any));
+  at = __shfl(at, 0);
+  if ((any & me) && strand == 0u) {
+    const uint32_t to = (wide & me) ? 0u : (staged ? 1u : 2u);
+    ids[at + (uint32_t)__popcll(any & (me - 1ull))] = (threadIdx.x >> 1) | (to << 8);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  uint32_t before = 0u;
+  if (lane == 0u) before = atomicAdd(&narrived, 1u);
+  if (__shfl(before, 0) != 512u / 64u - 1u) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  const uint32_t n = nids, rd0 = blockIdx.x * 256u;
+  auto places = [&](uint32_t i, uint32_t &id, uint64_t (&m)[3]) {
+    id = i + lane < n ? ids[i + lane] : 3u << 8;
+#pragma unroll
+    for (uint32_t c = 0; c < 3u; ++c) m[c] = __ballot((id >> 8) == c);
+  };
+  uint32_t id, cnt[3] = {0u, 0u, 0u};
+  uint64_t m[3];
+  for (uint32_t i = 0; i < n; i += 64u) {
+    places(i, id, m);
+#pragma unroll
+    for (uint32_t c = 0; c < 3u; ++c) cnt[c] += (uint32_t)__popcll(m[c]);
+  }
+  uint32_t first = 0u;                             // of lanes 0, 1, 2: the three lists'
+  const uint32_t mine3 = lane == 0u ? cnt[0] : (lane == 1u ? cnt[1] : (lane == 2u ? cnt[2] : 0u));
+  if (mine3) first = atomicAdd(lane == 0u ? P.wide_n : (lane == 1u ? P.list_n : P.long_n), mine3);
+  uint32_t f[3] = {__shfl(first, 0), __shfl(first, 1), __shfl(first, 2)};
+  for (uint32_t i = 0; i < n; i += 64u) {
+    places(i, id, m);
+    const uint32_t r = rd0 + (id & 255u), c = id >> 8;
+    const uint64_t mc = c == 0u ? m[0] : (c == 1u ? m[1] : m[2]);
+    const uint32_t p = (c == 0u ? f[0] : (c == 1u ? f[1] : f[2])) +
+                       (uint32_t)__popcll(mc & ((1ull << lane) - 1ull));
+    if (c == 0u) P.wide[p] = r;
+    else if (c == 1u) P.list[p] = r;
+    else if (c == 2u) P.wide[P.nreads - 1u - p] = r;
+#pragma unroll
+    for (uint32_t e = 0; e < 3u; ++e) f[e] += (uint32_t)__popcll(m[e]);
   }
 }
 
@@ -330,10 +370,10 @@ __global__ __launch_bounds__(256) void search1_wave_kernel(S1tParams P) {
 hipError_t launch_search1_text(const DevIndex &ix, bool mm_only, uint32_t strand_mask,
                                const uint8_t *reads, const uint64_t *offsets, uint32_t nreads,
                                uint32_t cap, fmi_hit *hits, uint32_t *counts, uint32_t *rec,
-                               uint32_t *wide, uint32_t *wide_n, uint32_t *list, uint32_t *list_n,
-                               uint32_t cus, hipStream_t s) {
-  S1tParams P{ix,   reads,  offsets, hits,   counts, rec,
-              wide, wide_n, list,    list_n, nreads, strand_mask, cap};
+                               uint32_t *wide, uint32_t *wide_n, uint32_t *long_n, uint32_t *list,
+                               uint32_t *list_n, uint32_t cus, hipStream_t s) {
+  S1tParams P{ix,     reads,  offsets, hits,   counts, rec,         wide,
+              wide_n, long_n, list,    list_n, nreads, strand_mask, cap};
   const dim3 g((uint32_t)((2ull * nreads + 511u) / 512u));
   const dim3 w(std::min<uint32_t>((nreads + 3u) / 4u, cus * 6u));   // resident (24 KB of LDS each)
   const bool resident = g.x <= 2u * cus;   // two groups a CU at 4 waves

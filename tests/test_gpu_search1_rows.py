@@ -3,6 +3,8 @@ anchors of one to four rows (a thread per strand), five to 64 (a wavefront per
 read), more (step by step), halves of 15 and 16 bases, reads of 256 and 257,
 on copies of every such number, runs of one base and both ends of the text,
 with N bases and one error anywhere, against the oracle record for record."""
+import time
+
 import numpy as np
 import pytest
 
@@ -105,4 +107,101 @@ def test_search1_rows_batch_size(gpu_engine, copies, nreads):
     finally:
         batch.free()
         few.free()
+        ix.close()
+
+
+@pytest.fixture(scope="module")
+def satellite():
+    """1200, 90 and 40 exact copies of 300 bases, and reads of them with
+    reads longer than a slot and too short for an anchor in between."""
+    rng = np.random.default_rng(411)
+    g = rng.integers(0, 4, 1_500_000).astype(np.uint8)
+    spots, at = [], 500
+    for count in (1200, 90, 40):
+        unit = rng.integers(0, 4, 300).astype(np.uint8)
+        spots.append(at)
+        for _ in range(count):
+            g[at:at + 300] = unit
+            at += 310
+    assert at < len(g) - 1000
+    return g, spots
+
+
+def _batch(g, spots, lens, seed):
+    rng = np.random.default_rng(seed)
+    reads = []
+    for L in lens:
+        p = int(rng.choice(spots)) + int(rng.integers(0, max(301 - L, 1))) if rng.random() < 0.8 \
+            else int(rng.integers(0, len(g) - L))
+        w = g[p:p + L].copy()
+        if L and rng.random() < 0.6:
+            e = int(rng.integers(0, L))
+            w[e] = (w[e] + 1) % 4
+        reads.append(synth.revcomp(w) if rng.random() < 0.5 else w)
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    return np.concatenate(reads).astype(np.uint8), offs
+
+
+@pytest.mark.parametrize("nreads", [1, 255, 256, 257, 700])
+def test_search1_left_reads(gpu_engine, satellite, nreads):
+    """Groups whose reads go on in all three lists, part full and over a group's
+    edge: record for record the oracle's."""
+    hp = gpu_engine
+    g, spots = satellite
+    ix = hp.Index.build_gpu(g, 16)
+    ix.expand()
+    ix.kmer_table(11)
+    o = fo.Oracle(bwts=(*ix.bwt(0), *ix.bwt(1)), ratio=16)
+    rng = np.random.default_rng(412)
+    lens = rng.choice([0, 20, 31, 32, 60, 100, 150, 256, 257, 290], nreads)
+    reads, offs = _batch(g, spots, lens, 413)
+    batch = hp.ReadBatch(reads, offs)
+    try:
+        for mode in (hp.MODE_EDIT, hp.MODE_MISMATCH):
+            _, oc, oh = o.search1_batch(reads, offs, cap=8, mismatch_only=mode == hp.MODE_MISMATCH)
+            oc, oh = oc.reshape(-1, 2), oh.reshape(-1, 2, 8)
+            counts, hits = hp.search1_batch(ix, batch, cap=8, mode=mode)
+            assert np.array_equal(counts, oc)
+            for i in range(nreads):
+                for s in (0, 1):
+                    c = min(int(oc[i, s]), 8)
+                    assert fo.hits_equal(hits[i, s, :c], oh[i, s, :c]), (mode, i, s)
+    finally:
+        batch.free()
+        ix.close()
+
+
+@pytest.mark.parametrize("kind", ["short"])
+def test_search1_left_reads_cost(gpu_engine, satellite, kind):
+    """Reads that the text kernels leave cost what the step-by-step search of
+    them does (the same batch without staging never meets the text kernels), not
+    a multiple of it: at most 1.25 times, where a walk over the
+    other kernel's reads made it 1.33."""
+    hp = gpu_engine
+    g, spots = satellite
+    ix = hp.Index.build_gpu(g, 16)
+    ix.expand()
+    ix.kmer_table(13)
+    n = 60_000
+    reads, offs = _batch(g, spots[:1], np.full(500, {"short": 30}[kind]),
+                         414)
+    batch = hp.ReadBatch(np.tile(reads, n // 500),
+                         np.arange(n + 1, dtype=np.uint64) * (offs[1] - offs[0]))
+    out = hp.Search1Output(n, 4)
+    took = {}
+    try:
+        for staging in (True, False, True, False):
+            hp.set_staging(staging)
+            for _ in range(6):
+                hp.sync()
+                t = time.perf_counter()
+                hp.search1_launch(ix, batch, out)
+                hp.sync()
+                took[staging] = min(took.get(staging, 1.0), time.perf_counter() - t)
+        print(kind, took)
+        assert took[True] < 1.25 * took[False], took
+    finally:
+        hp.set_staging(True)
+        out.free()
+        batch.free()
         ix.close()
