@@ -35,6 +35,7 @@ struct S1tParams {
   uint32_t *wide, *wide_n, *long_n;
   uint32_t *list, *list_n;         // the reads left to search1_kernel staged
   uint32_t nreads, strand_mask, cap;
+  int32_t wide_m;                  // rows_wide_m
 };
 
 // Where a read goes on: nowhere, in search1_wave_kernel, in search1_kernel.
@@ -76,16 +77,16 @@ __device__ __forceinline__ void add_string(S1tOut &O, const DevDir &D, uint32_t 
 template <bool MM_ONLY>
 __device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass, uint32_t strand,
                                               const ReadBases<true> &rd, int32_t len,
-                                              S1tOut &O) {
+                                              int32_t wide_m, S1tOut &O) {
   const uint32_t dsel = pass ^ strand;
   const DevDir &D = dir_of(ix, dsel);
   const int32_t half = len / 2, d = pass ? 1 : -1, p0 = pass ? 0 : len - 1;
   const int32_t m0 = pass ? half : len - half, N = len - m0;
   TextRows R;
   uint32_t k, l;
-  const uint32_t found = search_rows<true>(ix, dsel, strand, rd, p0, d, m0, R, k, l);
+  const uint32_t found = search_rows<true>(ix, dsel, strand, rd, p0, d, m0, R, k, l, wide_m);
   if (found == kRowsNone) return kDone;
-  if (found == kRowsMany) return kToWave;
+  if (found == kRowsMany) return l - k < 64u ? kToWave : kToList;
   int32_t run[kTextRows] = {-1, -1, -1, -1};
 #pragma unroll
   for (uint32_t j = 0; j < kTextRows; ++j)
@@ -121,8 +122,9 @@ __device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass,
 
 // A thread per (read, strand); a read's two threads pack it into one LDS slot.
 // A read with more than kTextRows rows at half of it is left to
-// search1_wave_kernel, one with an anchor of less than kTextHalf bases or more
-// bases than a slot to search1_kernel; its record is written from the slot.
+// search1_wave_kernel, one with more than 64, an anchor of less than kTextHalf
+// bases or more bases than a slot to search1_kernel; its record is written from
+// the slot.
 // Bound by the latency of a pass's chain and the lines it reads (an entry,
 // contexts, suffixes, text and the records' rows).  At 4 waves: 1 M reads of 150 bases over 64 Mbp: 576 us, where the records,
 // the state machine and its records' rows took 1284; 2 M over 3.1 Gbp 1552
@@ -185,7 +187,7 @@ __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
     } else if (asked) {
       const ReadBases<true> bases{nullptr, slot};
       for (uint32_t pass = 0; pass < 2u && left == kDone; ++pass)
-        left = text_pass<MM_ONLY>(P.ix, pass, strand, bases, len, O);
+        left = text_pass<MM_ONLY>(P.ix, pass, strand, bases, len, P.wide_m, O);
     }
     P.counts[t64] = O.cnt;
   }
@@ -332,8 +334,10 @@ __device__ __forceinline__ bool wave_pass(const DevIndex &ix, uint32_t pass, uin
   return true;
 }
 
-// The reads that search1_text_kernel left for their rows, a wavefront per
-// read; one with more than 64 rows goes on to search1_kernel, which takes a
+// The reads that search1_text_kernel left for their 5 to 64 rows, a wavefront
+// per read (with those of more rows, whose steps it takes in vain, 100 K reads
+// of a repeat of 3000 copies took 1.3 ms here); one whose second pass has more
+// goes on to search1_kernel, which takes a
 // step per memory access (a read of a repeat then takes 0.3-1 ms from its
 // first step to its last, which a launch waits for: with these reads there
 // the batches above took 870 and 2370 us, and 700 K reads of 50-250 bases
@@ -373,7 +377,8 @@ hipError_t launch_search1_text(const DevIndex &ix, bool mm_only, uint32_t strand
                                uint32_t *wide, uint32_t *wide_n, uint32_t *long_n, uint32_t *list,
                                uint32_t *list_n, uint32_t cus, hipStream_t s) {
   S1tParams P{ix,     reads,  offsets, hits,   counts, rec,         wide,
-              wide_n, long_n, list,    list_n, nreads, strand_mask, cap};
+              wide_n, long_n, list,    list_n, nreads, strand_mask, cap,
+              rows_wide_m(ix.n)};
   const dim3 g((uint32_t)((2ull * nreads + 511u) / 512u));
   const dim3 w(std::min<uint32_t>((nreads + 3u) / 4u, cus * 6u));   // resident (24 KB of LDS each)
   const bool resident = g.x <= 2u * cus;   // two groups a CU at 4 waves
