@@ -15,7 +15,8 @@
 //
 // Two launches.  map_single_kernel, a thread per read, settles every read of
 // at most kStagedMaxLen bases whose strands have at most kTextRows rows each
-// (one on a compact index) and marks the others in counts;
+// (one on a compact index) or more than the filter lets through, and marks the
+// others in counts;
 // map_reads_kernel's lanes stride over the marked reads, a lane keeping the
 // current strand's alignments in its scratch slice (at most filter + 1 of
 // them: a strand's rows number l - k + 1 <= filter + 1 once the count has
@@ -51,6 +52,7 @@ struct MapParams {
   uint32_t *counts;
   uint8_t *status;
   MapTmp *scratch;            // lanes * (filter + 1)
+  int32_t wide_m;             // of map_single_kernel's searches (search_rows)
 };
 
 // A read's count while the read waits for map_reads_kernel (a count is at
@@ -58,37 +60,38 @@ struct MapParams {
 constexpr uint32_t kMapWaits = 0xFFFFFFFFu;
 
 // BWExactSearchBackward of the whole read from [0, n] on one view: whether its
-// interval is not empty (an empty one is not formed: no caller sees it), and
-// then its rows' suffixes R, or on a compact index, or where there are more of
-// them, the rows k..l (R.n = 0).
+// interval is not empty (kRowsNone: an empty one is not formed, no caller sees
+// it), and then its rows' suffixes R, or on a compact index, or where there are
+// more of them, the rows k..l (R.n = 0).  wide_m, kRowsCut: as search_rows.
 template <bool STAGED>
-__device__ __forceinline__ bool live_interval(const DevIndex &ix, uint32_t dsel, uint32_t comp,
-                                              const ReadBases<STAGED> &rd, int32_t len,
-                                              uint32_t &k, uint32_t &l, TextRows &R) {
+__device__ __forceinline__ uint32_t live_interval(const DevIndex &ix, uint32_t dsel, uint32_t comp,
+                                                  const ReadBases<STAGED> &rd, int32_t len,
+                                                  uint32_t &k, uint32_t &l, TextRows &R,
+                                                  int32_t wide_m = INT32_MAX) {
   const DevDir &D = dir_of(ix, dsel);
   R.n = 0u;
   if (ix.text != nullptr)
-    return search_rows<STAGED>(ix, dsel, comp, rd, len - 1, -1, len, R, k, l) != kRowsNone;
+    return search_rows<STAGED>(ix, dsel, comp, rd, len - 1, -1, len, R, k, l, wide_m);
   const int32_t K = ix.kmer_k && len >= (int32_t)ix.kmer_k ? (int32_t)ix.kmer_k : 0;
   k = 0u;
   l = ix.n;
   if (K) {
     uint32_t c;
-    if (!rd.code(len - 1, -1, K, comp, c)) return false;
+    if (!rd.code(len - 1, -1, K, comp, c)) return kRowsNone;
     const uint64_t e = (dsel ? ix.kmer[1] : ix.kmer[0])[c];
     k = (uint32_t)e;
     l = (uint32_t)(e >> 32);
-    if (k > l) return false;
+    if (k > l) return kRowsNone;
   }
   for (int32_t i = len - 1 - K; i >= 0; --i) {
     uint32_t a, b;
     const uint32_t sym = STAGED ? lf_sym(D, k, l, rd.at(i), comp, a, b)
                                 : lf_read(D, k, l, rd.W + i, comp, a, b);
-    if (sym > 3u || a > b) return false;
+    if (sym > 3u || a > b) return kRowsNone;
     k = a;
     l = b;
   }
-  return true;
+  return kRowsMany;
 }
 
 // The contig of an occurrence at text position key of len bases (binsearch,
@@ -126,7 +129,10 @@ __device__ __forceinline__ void store_mapping(fmi_read_mapping *out, uint64_t po
 // (24 KB a workgroup) leave 6 workgroups a CU.  500 K reads of 100 bases over
 // 64 Mbp: 145 us, where one launch of 64 K lanes (the scratch allows no more)
 // took 1540, and 125 went to the marked reads when they were those with more
-// than one row.
+// than one row.  A strand over the filter ends its read here: 100 K reads of 3000
+// copies 209 us at a filter of 50, where searching them again took 479 (LF steps
+// alone 318).  Reads of 5 copies to the filter are searched twice: of 130 copies
+// at a filter of 1000 4.03 ms, 3.80 by LF steps alone.
 __global__ __launch_bounds__(256) void map_single_kernel(MapParams P) {
   __shared__ uint32_t slots[kReadRecordWords * 256u];
   const uint32_t rd = blockIdx.x * 256u + threadIdx.x;
@@ -154,9 +160,14 @@ __global__ __launch_bounds__(256) void map_single_kernel(MapParams P) {
     // + strand: BACKWARD; - strand: FORWARD_REV (bwt.c:1996-2001)
     uint32_t k, l;
     TextRows R;
-    if (!live_interval<true>(P.ix, strand, strand, bases, len, k, l, R)) continue;
+    const uint32_t found = live_interval<true>(P.ix, strand, strand, bases, len, k, l, R, P.wide_m);
+    if (found == kRowsNone) continue;
     if (R.n == 0u) {
-      if (k != l) {
+      if (found == kRowsMany && k != l && l - k > P.filter - tot) {
+        st = 1u;
+        break;
+      }
+      if (found == kRowsCut || k != l) {
         P.counts[rd] = kMapWaits;
         return;
       }
@@ -221,7 +232,7 @@ __global__ __launch_bounds__(256) void map_reads_kernel(MapParams P) {
       uint32_t k, l;
       TextRows R;
       uint32_t m = 0;
-      if (live_interval<false>(P.ix, dsel, dsel, bases, len, k, l, R)) {
+      if (live_interval<false>(P.ix, dsel, dsel, bases, len, k, l, R) != kRowsNone) {
         if (R.n) { k = 0u; l = R.n - 1u; }             // the rows' suffixes are known
         tot += (uint64_t)(l - k);
         if (tot > P.filter) { st |= 1u; break; }
@@ -289,8 +300,11 @@ hipError_t launch_map_reads(const DevIndex &ix, const uint8_t *reads, const uint
                             uint32_t *counts, uint8_t *status, void *scratch, uint32_t lanes,
                             hipStream_t s) {
   if (nreads == 0 || lanes == 0) return hipSuccess;
+  // With a filter below kManyRows an interval of that many rows most likely ends
+  // its read, once it is known, in map_single_kernel itself.
   MapParams P{ix,     reads,  offsets, koff,   kstart, kcount, nreads, filter, cap,
-              out,    counts, status,  static_cast<MapTmp *>(scratch)};
+              out,    counts, status,  static_cast<MapTmp *>(scratch),
+              filter < kManyRows ? INT32_MAX : rows_wide_m(ix.n)};
   hipLaunchKernelGGL(map_single_kernel, dim3((nreads + 255u) / 256u), dim3(256), 0, s, P);
   hipLaunchKernelGGL(map_reads_kernel, dim3(lanes / 256), dim3(256), 0, s, P);
   return hipGetLastError();

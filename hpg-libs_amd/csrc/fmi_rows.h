@@ -75,7 +75,7 @@ inline int32_t rows_wide_m(uint32_t n) {
   return m;
 }
 
-enum : uint32_t { kRowsNone = 0u, kRowsFew = 1u, kRowsMany = 2u };
+enum : uint32_t { kRowsNone = 0u, kRowsFew = 1u, kRowsMany = 2u, kRowsCut = 3u };
 
 // The search for the m0 bases W[p0], W[p0 + d], ... from the whole index:
 // kRowsNone when they occur nowhere, kRowsFew with their rows' suffixes in R,
@@ -86,8 +86,7 @@ enum : uint32_t { kRowsNone = 0u, kRowsFew = 1u, kRowsMany = 2u };
 // rows (and none of the rows that a k-mer has by chance) without a look at
 // their suffixes; a wider one takes an LF step.  wide_m (rows_wide_m, for
 // callers that do without such rows): a step to that many bases or more that
-// leaves more than kManyRows rows ends the search, kRowsMany with the rows so far
-// in k..l.
+// leaves more than kManyRows rows ends the search with kRowsCut.
 template <bool STAGED>
 __device__ __forceinline__ uint32_t search_rows(const DevIndex &ix, uint32_t dsel, uint32_t comp,
                                                 const ReadBases<STAGED> &rd, int32_t p0, int32_t d,
@@ -148,7 +147,7 @@ __device__ __forceinline__ uint32_t search_rows(const DevIndex &ix, uint32_t dse
     k = a;
     l = b;
     ++m;
-    if (m >= wide_m && l - k >= kManyRows) return kRowsMany;
+    if (m >= wide_m && l - k >= kManyRows) return kRowsCut;
   }
   if (l - k >= kTextRows) return kRowsMany;
   R = text_rows(D, k, l);

@@ -86,7 +86,7 @@ __device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass,
   uint32_t k, l;
   const uint32_t found = search_rows<true>(ix, dsel, strand, rd, p0, d, m0, R, k, l, wide_m);
   if (found == kRowsNone) return kDone;
-  if (found == kRowsMany) return l - k < 64u ? kToWave : kToList;
+  if (found != kRowsFew) return found == kRowsMany && l - k < 64u ? kToWave : kToList;
   int32_t run[kTextRows] = {-1, -1, -1, -1};
 #pragma unroll
   for (uint32_t j = 0; j < kTextRows; ++j)

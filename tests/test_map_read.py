@@ -14,6 +14,8 @@ and the flags -- on a genome with tandem repeats (occurrences 1-7 bp apart),
 far-apart copies, copies across contig ends, short reads, reads with N and
 filters that are exceeded on either strand.
 GPU: fmi_map_reads_batch against the oracle, record for record."""
+import time
+
 import numpy as np
 import pytest
 
@@ -215,4 +217,78 @@ def test_map_read_lengths(gpu_engine, stage):
                     assert np.array_equal(recs[i, :m][key], orecs[key]), (filt, i, key)
     finally:
         batch.free()
+        ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("table", [0, 10])
+def test_map_read_many_rows(gpu_engine, table):
+    """Reads of 5, 60, 70 and 1200 copies, forward and reverse, at filters below,
+    at and above their rows (a read over the filter ends where its rows are
+    first known, one with more rows than that launch holds in the second),
+    against the oracle; and a batch of reads over the filter costs their search,
+    at most 1.6 times the exact search of both strands: 0.96 measured, 2.2 where
+    the second launch repeats it."""
+    hp = gpu_engine
+    rng = np.random.default_rng(21)
+    g = rng.integers(0, 4, 900_000).astype(np.uint8)
+    at, reads = 100, []
+    for count in (5, 60, 70, 1200):
+        unit = rng.integers(0, 4, 300).astype(np.uint8)
+        for _ in range(count):
+            g[at:at + 300] = unit
+            at += 320
+        for L in (40, 100, 256, 280):
+            reads += [unit[3:3 + L].copy(), COMP[unit[2:2 + L]][::-1].copy()]
+    koff, kstart = np.array([0, len(g)], np.uint64), np.ones(1, np.uint64)
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(kstart, np.array([len(g)], np.uint64))
+    ix.to_device()
+    o = fo.Oracle(bwts=(*ix.bwt(0), *ix.bwt(1)), ratio=16)
+    ix.expand()
+    if table:
+        ix.kmer_table(table)
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads).astype(np.uint8), offs)
+    n = 100_000
+    rep = hp.ReadBatch(np.tile(reads[-6], n), np.arange(n + 1, dtype=np.uint64) * len(reads[-6]))
+    try:
+        for filt in (1, 3, 4, 58, 59, 60, 69, 1198, 1199, 1500):
+            st, cnt, recs = hp.map_reads_batch(ix, batch, filt, 8)
+            for i, W in enumerate(reads):
+                ost, orecs, ototal = o.map_read(W, filt, koff, kstart, read=i, cap=8)
+                assert (int(st[i]), int(cnt[i])) == (ost, ototal), (filt, i)
+                m = min(ototal, 8)
+                for key in ("position", "chromosome", "read", "strand", "secondary", "cigar_len"):
+                    assert np.array_equal(recs[i, :m][key], orecs[key]), (filt, i, key)
+        assert len(reads[-6]) == 100
+        L, d = hp.lib(), rep
+        bufs = [hp.DeviceBuffer(b) for b in (24 * n, 4 * n, n, 32 * n)]
+
+        def mapped():
+            hp.check(L.fmi_map_reads_batch(ix.h, d.d_reads.ptr, d.d_offsets.ptr, n, 50, 1,
+                                           bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, None))
+
+        def exact():
+            for t, view in ((0, hp.VIEW_BACKWARD), (1, hp.VIEW_BACKWARD_REV)):
+                hp.check(L.fmi_exact_batch(ix.h, view, t, d.d_reads.ptr, d.d_offsets.ptr, n,
+                                           bufs[3].ptr, None, None))
+
+        took = []
+        for f in (mapped, exact):
+            best = 1.0
+            for _ in range(8):
+                hp.sync()
+                t0 = time.perf_counter()
+                f()
+                hp.sync()
+                best = min(best, time.perf_counter() - t0)
+            took.append(best)
+        for b in bufs:
+            b.free()
+        print(took)
+        assert took[0] < 1.6 * took[1], took
+    finally:
+        batch.free()
+        rep.free()
         ix.close()
