@@ -37,6 +37,7 @@ struct VhParams {
   uint32_t *counts;
   uint2 *scratch;           // lanes * (kMaxReadLen + 3) intervals
   uint32_t nreads, cap, strand_mask, mm_only;
+  int32_t wide_m;           // rows_wide_m
 };
 
 // The count of a (read, strand) that waits for vhelper_kernel.
@@ -75,13 +76,13 @@ __device__ __forceinline__ bool vh_window(const VhParams &P, uint32_t t, const u
 template <bool STAGED>
 __device__ __forceinline__ bool vt_half(const DevIndex &ix, uint32_t dir, uint32_t strand,
                                         const ReadBases<STAGED> &rd, int32_t start, int32_t end,
-                                        VhRec &r, VtSink &S) {
+                                        int32_t wide_m, VhRec &r, VtSink &S) {
   const uint32_t dsel = dir ^ strand, comp = strand;
   const int32_t L = end - start + 1, d = dir ? 1 : -1, p0 = dir ? start : end;
   const int32_t m0 = dir ? (L - 1) / 2 : L - (L - 1) / 2;
   TextRows R;
   uint32_t k, l;
-  const uint32_t found = search_rows<STAGED>(ix, dsel, comp, rd, p0, d, m0, R, k, l);
+  const uint32_t found = search_rows<STAGED>(ix, dsel, comp, rd, p0, d, m0, R, k, l, wide_m);
   if (found != kRowsFew) return found == kRowsNone;   // without rows no node is alive
   // how far each row goes on with the window: it ends at a node
   const int32_t N = L - m0;
@@ -154,7 +155,7 @@ __device__ __forceinline__ uint32_t vt_task(const VhParams &P, uint32_t t, const
   VhRec r{0, 0, -1, 0, 0, 0, 0, 0};
   for (uint32_t dir = 0; dir < 2u; ++dir) {
     r.dir = dir;
-    if (!vt_half<STAGED>(P.ix, dir, strand, rd, start, end, r, S)) return kVhWaits;
+    if (!vt_half<STAGED>(P.ix, dir, strand, rd, start, end, P.wide_m, r, S)) return kVhWaits;
   }
   return S.cnt;
 }
@@ -244,7 +245,7 @@ hipError_t launch_vhelper(const DevIndex &ix, bool mm_only, uint32_t strand_mask
                           uint32_t nreads, uint32_t cap, fmi_hit *hits, uint32_t *counts,
                           void *scratch, uint32_t lanes, hipStream_t s) {
   VhParams P{ix, reads, offsets, bounds, hits, counts, static_cast<uint2 *>(scratch), nreads, cap,
-             strand_mask, mm_only ? 1u : 0u};
+             strand_mask, mm_only ? 1u : 0u, rows_wide_m(ix.n)};
   if (nreads == 0 || lanes == 0) return hipSuccess;
   if (ix.text != nullptr) {
     const uint32_t grid = (uint32_t)((2ull * nreads + 255) / 256);

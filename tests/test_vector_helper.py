@@ -277,3 +277,40 @@ def test_gpu_vector_helper_on_text(gpu_engine, n, kmer):
     finally:
         batch.free()
         ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kmer", [0, 9])
+def test_gpu_vector_helper_many_copies(gpu_engine, kmer):
+    """Windows of 1200 exact copies (a half's interval is given up early), with
+    and without one error, against the oracle."""
+    hp = gpu_engine
+    rng = np.random.default_rng(91)
+    g = rng.integers(0, 4, 200_000).astype(np.uint8)
+    unit = rng.integers(0, 4, 130).astype(np.uint8)
+    for i in range(1200):
+        g[50 + 140 * i:180 + 140 * i] = unit
+    ix = hp.Index.build(g, 16).to_device()
+    ix.expand()
+    if kmer:
+        ix.kmer_table(kmer)
+    o = fo.Oracle(bwts=(*ix.bwt(0), *ix.bwt(1)), ratio=16)
+    reads = []
+    for L in (31, 40, 60, 120, 130):
+        for e in (-1, 0, L // 2 - 1, L // 2, L - 1):
+            w = unit[:L].copy()
+            if e >= 0:
+                w[e] = (w[e] + 1) % 4
+            reads += [w, synth.revcomp(w)]
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    batch = hp.ReadBatch(np.concatenate(reads).astype(np.uint8), offs)
+    try:
+        counts, hits = hp.search1_vector_batch(ix, batch, cap=30, mode=hp.MODE_EDIT)
+        for i, W in enumerate(reads):
+            for s in (0, 1):
+                m, h = o.search1_vector(s, W, 0, len(W) - 1, cap=30, mismatch_only=False)[:2]
+                assert int(counts[i, s]) == m, (i, s)
+                assert fo.hits_equal(hits[i, s, :min(m, 30)], h), (i, s)
+    finally:
+        batch.free()
+        ix.close()
