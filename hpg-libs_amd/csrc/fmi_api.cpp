@@ -235,6 +235,18 @@ int end_timed(hipStream_t s, hipError_t launch_err, const char *what) {
   return FMI_OK;
 }
 
+// Whether a graph captured here is alive: it may hold the addresses of any
+// index's arrays.
+bool graphs_alive() {
+  std::lock_guard<std::mutex> lk(g_mu);
+  return !g_graph_stream.empty();
+}
+
+// fmi_index_kmer_table's tables of k bases and, from k = 8 on, of k - 4.
+uint64_t kmer_table_bytes(uint32_t k) {
+  return 2 * sizeof(uint64_t) * ((1ull << (2 * k)) + (k >= 8 ? 1ull << (2 * (k - 4)) : 0ull));
+}
+
 int need_device(const fmi_index *ix) {
   if (!ix) return fail(FMI_EINVAL, "index is NULL");
   if (!ix->on_device) return fail(FMI_ESTATE, "index is not on the device (call fmi_index_to_device)");
@@ -432,13 +444,13 @@ uint64_t fmi_index_device_bytes(const fmi_index *ix) {
   uint64_t b = 0;
   for (int d = 0; d < 2; ++d)
     b += ix->h[d].nblocks * sizeof(fmi::OccBlock) + 2 * ((ix->h[d].nsamp * 4 + 255) & ~255ull);
-  return b + ix->full_bytes + ix->kmer_bytes;
+  return b + ix->full_bytes + ix->ctx_bytes + ix->kmer_bytes;
 }
 
 int fmi_index_device_layout(const fmi_index *ix, uint64_t *out) {
   if (!ix || !out) return fail(FMI_EINVAL, "NULL argument");
-  out[0] = fmi_index_device_bytes(ix) - ix->full_bytes - ix->kmer_bytes;
-  out[1] = ix->full_bytes;
+  out[1] = ix->full_bytes + ix->ctx_bytes;
+  out[0] = fmi_index_device_bytes(ix) - out[1] - ix->kmer_bytes;
   out[2] = ix->kmer_bytes;
   return FMI_OK;
 }
@@ -478,10 +490,13 @@ int fmi_index_expand(fmi_index *ix) {
   ix->dev.text = text;
   ix->d_full = mem;
   ix->full_bytes = bytes;
-  // The row contexts, 8 bytes per base, only where they leave at least as
-  // much memory free as they take: the searches do without them.
+  // The row contexts, 8 bytes per base, only where they leave room for the
+  // largest k-mer table and as much again as they take: the searches do without
+  // them, and what a program allocates next has to fit as it did.
+  const uint64_t reserve = ix->d_kmer ? 0 : kmer_table_bytes(15);
   size_t free_bytes = 0, total_bytes = 0;
-  if (ix->n && hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && free_bytes >= 4 * arr) {
+  if (ix->n && hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess &&
+      free_bytes >= 4 * arr + reserve) {
     void *ctx = nullptr;
     if (hipMalloc(&ctx, 2 * arr) != hipSuccess) {
       (void)hipGetLastError();
@@ -499,8 +514,20 @@ int fmi_index_expand(fmi_index *ix) {
     for (int d = 0; d < 2; ++d)
       ix->dev.d[d].ctx = reinterpret_cast<const uint32_t *>(static_cast<char *>(ctx) + d * arr);
     ix->d_ctx = ctx;
-    ix->full_bytes += 2 * arr;
+    ix->ctx_bytes = 2 * arr;
   }
+  return FMI_OK;
+}
+
+int fmi_index_drop_contexts(fmi_index *ix) {
+  int rc = need_device(ix);
+  if (rc) return rc;
+  if (!ix->d_ctx) return FMI_OK;
+  HIP_TRY(hipDeviceSynchronize(), "drain before freeing the row contexts");
+  (void)hipFree(ix->d_ctx);
+  ix->d_ctx = nullptr;
+  ix->ctx_bytes = 0;
+  ix->dev.d[0].ctx = ix->dev.d[1].ctx = nullptr;
   return FMI_OK;
 }
 
@@ -525,6 +552,12 @@ int fmi_index_kmer_table(fmi_index *ix, uint32_t k) {
   const uint64_t per2 = k2 ? (1ull << (2 * k2)) * sizeof(uint64_t) : 0;
   void *mem = nullptr;
   hipError_t e = hipMalloc(&mem, 2 * (per + per2));
+  if (e != hipSuccess && ix->d_ctx && !graphs_alive()) {
+    (void)hipGetLastError();
+    rc = fmi_index_drop_contexts(ix);
+    if (rc) return rc;
+    e = hipMalloc(&mem, 2 * (per + per2));
+  }
   if (e != hipSuccess)
     return fail(FMI_ENOMEM, "hipMalloc(k-mer table, " + std::to_string(2 * (per + per2)) + " bytes)");
   char *base = static_cast<char *>(mem);

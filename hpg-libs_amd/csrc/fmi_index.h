@@ -25,8 +25,9 @@ struct fmi_index {
   uint64_t *d_kstart = nullptr;
   uint64_t device_bytes = 0;
   void *d_full = nullptr;         // full SA / ISA of both directions + 2-bit text
-  void *d_ctx = nullptr;          // row contexts of both directions (room permitting)
   uint64_t full_bytes = 0;
+  void *d_ctx = nullptr;          // row contexts of both directions (room permitting)
+  uint64_t ctx_bytes = 0;
   void *d_kmer = nullptr;         // k-mer interval tables of both directions
   uint64_t kmer_bytes = 0;
   fmi::DevIndex dev{};

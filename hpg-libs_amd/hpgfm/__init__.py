@@ -55,7 +55,7 @@ EXPORTS = [
     "fmi_gather_bench", "fmi_gather_probe",
     "fmi_search1_count_blocks", "fmi_timing_begin", "fmi_timing_end",
     "fmi_seed_map_batch", "fmi_map_inexact_seeds_batch", "fmi_map_reads_batch", "fmi_format_results", "fmi_inverse_locate_batch", "fmi_encode_bases", "fmi_copy_bench",
-    "fmi_search1_vector_batch", "fmi_index_expand", "fmi_index_kmer_table", "fmi_index_get_kmer_table",
+    "fmi_search1_vector_batch", "fmi_index_expand", "fmi_index_drop_contexts", "fmi_index_kmer_table", "fmi_index_get_kmer_table",
     "fmi_index_get_full", "fmi_index_sample_count", "fmi_index_get_samples",
     "fmi_search1_count_work", "fmi_search_k_count_work", "fmi_exact_count_work", "fmi_search_k_batch", "fmi_plain_create", "fmi_plain_search1", "fmi_plain_words",
     "fmi_plain_get_layout", "fmi_plain_device_bytes", "fmi_plain_free",
@@ -160,6 +160,7 @@ def _bind(lib):
         "fmi_copy_bench": ([_p, _p, _u64, C.POINTER(C.c_float), _p], _i),
         "fmi_search1_vector_batch": ([_p, _i, _i, _p, _p, _p, _u32, _u32, _p, _p, _p], _i),
         "fmi_index_expand": ([_p], _i),
+        "fmi_index_drop_contexts": ([_p], _i),
         "fmi_index_kmer_table": ([_p, _u32], _i),
         "fmi_index_get_kmer_table": ([_p, _i, _p], _i),
         "fmi_search1_count_work": ([_p, _i, _i, _p, _p, _u32, _u32, _p], _i),
@@ -506,6 +507,11 @@ class Index:
         """fmi_index_expand: full SA / ISA of both directions and the 2-bit
         text on the device, for the text-comparison continuation."""
         check(lib().fmi_index_expand(self.h))
+        return self
+
+    def drop_contexts(self):
+        """fmi_index_drop_contexts: frees the row contexts that expand() kept."""
+        check(lib().fmi_index_drop_contexts(self.h))
         return self
 
     def kmer_table(self, k):

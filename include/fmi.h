@@ -139,19 +139,25 @@ void fmi_index_free(fmi_index *ix);
  * searches then continue every single-row interval by comparing the read
  * with the text at that row's suffix (one SA read to enter, one ISA read per
  * record) instead of one occurrence-block load per base; the records are
- * the same.  Where at least twice their size is free after that, the row
- * contexts of both directions are kept too (the 16 text bases before every
- * row's suffix, 8 bytes per base; 3.1 Gbp: 25 GB): several searches then tell
- * from one line how any bases extend the rows of an interval.  Results do not
- * depend on them.  No reference counterpart (it trades HBM for dependent
- * loads). */
+ * the same.  Where that leaves room for the largest k-mer table
+ * (fmi_index_kmer_table) and twice their size, the row contexts of both
+ * directions are kept too (the 16 text bases before every row's suffix, 8
+ * bytes per base; 3.1 Gbp: 25 GB): several searches then tell from one line
+ * how any bases extend the rows of an interval.  Results do not depend on
+ * them.  No reference counterpart (it trades HBM for dependent loads). */
 int fmi_index_expand(fmi_index *ix);
+/* Frees the row contexts that fmi_index_expand kept, for a program that needs
+ * their memory more; the searches do without them, with the same results.
+ * Waits for the device; as with the k-mer table, no call on the index may be
+ * under way and no graph that holds one may be launched afterwards. */
+int fmi_index_drop_contexts(fmi_index *ix);
 /* A table of the interval of every string of k bases in each direction
  * (4^k entries of 8 bytes per direction: k = 12 takes 128 MiB, k = 13 512
  * MiB, k = 15 8 GiB), built on the device from the occurrence blocks.
  * fmi_search1_batch then takes the first k LF steps of each exact phase in
  * one read of the table; the records are the same.  k = 0 frees the table;
- * otherwise k is 4..15.  No reference counterpart (it trades HBM for the widest, most
+ * otherwise k is 4..15.  Where the table does not fit, the row contexts are
+ * given up for it (unless a captured graph is alive).  No reference counterpart (it trades HBM for the widest, most
  * expensive LF steps of every search). */
 int fmi_index_kmer_table(fmi_index *ix, uint32_t k);
 /* Copies one direction's table (4^k entries, k | l << 32, an empty
@@ -175,8 +181,7 @@ uint64_t fmi_index_size_sa(const fmi_index *ix);
 uint32_t fmi_index_sa_ratio(const fmi_index *ix);
 /* Bytes of the device copy by part: out[0] occurrence blocks and S / R
  * samples of both directions, out[1] the full SA / ISA, 2-bit text and row
- * contexts
- * (fmi_index_expand), out[2] the k-mer tables (fmi_index_kmer_table). */
+ * contexts (fmi_index_expand), out[2] the k-mer tables (fmi_index_kmer_table). */
 int fmi_index_device_layout(const fmi_index *ix, uint64_t *out);
 /* Bytes the device copy occupies. */
 uint64_t fmi_index_device_bytes(const fmi_index *ix);
@@ -375,7 +380,8 @@ int fmi_get_tuning(uint32_t *wg_per_cu, uint32_t *chunk, uint32_t *refill_min);
  * data it reads anyway (fewer instructions); FMI_LOADS_OWN — each lane
  * issues only the loads its step needs (fewer memory requests, faster once
  * the index spreads over tens of GB); FMI_LOADS_AUTO (the default) — OWN for
- * an index of more than 16 GiB on the device, else ALL.  No reference
+ * an index of more than 16 GiB on the device (row contexts, which this search
+ * does not read, apart), else ALL.  No reference
  * counterpart. */
 #define FMI_LOADS_AUTO 0u
 #define FMI_LOADS_ALL 1u
