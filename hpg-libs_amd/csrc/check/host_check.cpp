@@ -10,6 +10,8 @@
 //                              recomputed); format records of random fields
 //   host_check load PATH       load one index file, print its status
 //   host_check import DIR      import one reference directory, print status
+//   host_check spread N        the memory that decides the 1-error search's load
+//                              mode: its own arrays, whatever else is kept
 //   host_check items 32|64     share out a wavefront's items at and around the
 //                              most that each item type is taken for: every 64
 //                              of them are one wavefront's, once
@@ -162,12 +164,27 @@ int items(uint32_t bits) {
   return 0;
 }
 
+int spread(uint64_t n) {
+  std::vector<uint8_t> text(n, 1);
+  fmi_index ix;
+  std::string err;
+  if (fmi::build_index(text.data(), n, 16, &ix, &err) != FMI_OK) return fail("build_index");
+  const uint64_t compact = fmi::search1_spread_bytes(&ix);
+  if (compact < n / 3 || compact > 64 * n + 4096) return fail("the compact index's bytes");
+  ix.full_bytes = 16 * n;
+  ix.kmer_bytes = 1 << 20;
+  ix.ctx_bytes = 8 * n;                          // read by other searches only
+  return fmi::search1_spread_bytes(&ix) == compact + 16 * n + (1 << 20)
+             ? 0 : fail("the row contexts move the load mode");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-  if (argc < 3) return fail("usage: host_check selftest SEED [TMPDIR] | load PATH | import DIR | items BITS");
+  if (argc < 3) return fail("usage: host_check selftest SEED [TMPDIR] | load PATH | import DIR | items BITS | spread N");
   const std::string cmd = argv[1];
   if (cmd == "selftest") return selftest((uint32_t)strtoul(argv[2], nullptr, 10), argc > 3 ? argv[3] : "/tmp");
+  if (cmd == "spread") return spread(strtoull(argv[2], nullptr, 10));
   if (cmd == "items") return items((uint32_t)strtoul(argv[2], nullptr, 10));
   if (cmd == "load") {
     printf("%d\n", load_status(argv[2]));

@@ -46,9 +46,9 @@ constexpr uint32_t kDefaultWgPerCu = 8;
 constexpr uint32_t kDefaultChunk = 64;
 constexpr uint32_t kDefaultRefill = 16;
 
-// An index whose device arrays exceed this spreads the search's accesses
-// over enough memory that issuing only the loads a step needs pays
-// (FMI_LOADS_AUTO).
+// An index whose device arrays (search1_spread_bytes) exceed this spreads the
+// search's accesses over enough memory that issuing only the loads a step
+// needs pays (FMI_LOADS_AUTO).
 constexpr uint64_t kOwnLoadsBytes = 16ull << 30;
 
 struct Tuning {
@@ -300,7 +300,7 @@ int search1_common(const fmi_index *ix, int mode, int strand_mask, const uint8_t
   rc = begin_timed(st);
   if (rc) return rc;
   const bool own = t.loads == FMI_LOADS_OWN ||
-                   (t.loads == FMI_LOADS_AUTO && fmi_index_device_bytes(ix) > kOwnLoadsBytes);
+                   (t.loads == FMI_LOADS_AUTO && fmi::search1_spread_bytes(ix) > kOwnLoadsBytes);
   hipError_t e = fmi::launch_search1(ix->dev, mode == FMI_MODE_MISMATCH, persistent, false,
                                      (uint32_t)strand_mask, d_reads, d_offsets, nreads, cap,
                                      d_hits, d_counts, w.queue, w.stats, grid, t.chunk,
@@ -440,11 +440,7 @@ int fmi_index_get_samples(const fmi_index *ix, int forward, uint32_t *S, uint32_
 uint32_t fmi_index_sa_ratio(const fmi_index *ix) { return ix ? ix->ratio : 0; }
 
 uint64_t fmi_index_device_bytes(const fmi_index *ix) {
-  if (!ix) return 0;
-  uint64_t b = 0;
-  for (int d = 0; d < 2; ++d)
-    b += ix->h[d].nblocks * sizeof(fmi::OccBlock) + 2 * ((ix->h[d].nsamp * 4 + 255) & ~255ull);
-  return b + ix->full_bytes + ix->ctx_bytes + ix->kmer_bytes;
+  return ix ? fmi::search1_spread_bytes(ix) + ix->ctx_bytes : 0;
 }
 
 int fmi_index_device_layout(const fmi_index *ix, uint64_t *out) {
@@ -1044,7 +1040,7 @@ int fmi_search1_batch_noalloc(const fmi_index *ix, int mode, int strand_mask,
   // memset), on the call's stream, before the search reads it
   HIP_TRY(fmi::launch_zero(queue, 1, st), "zero queue");
   const bool own = t.loads == FMI_LOADS_OWN ||
-                   (t.loads == FMI_LOADS_AUTO && fmi_index_device_bytes(ix) > kOwnLoadsBytes);
+                   (t.loads == FMI_LOADS_AUTO && fmi::search1_spread_bytes(ix) > kOwnLoadsBytes);
   HIP_TRY(fmi::launch_search1(ix->dev, mode == FMI_MODE_MISMATCH, true, false,
                               (uint32_t)strand_mask, d_reads, d_offsets, nreads, cap, d_hits,
                               d_counts, queue, stats, grid, t.chunk, t.refill_min, own, st),

@@ -37,6 +37,15 @@ struct fmi_index {
 
 namespace fmi {
 
+// The device memory that the step-by-step 1-error search spreads its accesses
+// over: all of the index but the row contexts, which it does not read.
+inline uint64_t search1_spread_bytes(const fmi_index *ix) {
+  uint64_t b = ix->full_bytes + ix->kmer_bytes;
+  for (int d = 0; d < 2; ++d)
+    b += ix->h[d].nblocks * sizeof(OccBlock) + 2 * ((ix->h[d].nsamp * 4 + 255) & ~255ull);
+  return b;
+}
+
 // Builds both directions from codes 0..3; returns an fmi_status.
 int build_index(const uint8_t *text, uint64_t n, uint32_t ratio, fmi_index *ix,
                 std::string *err);
