@@ -469,6 +469,8 @@ struct InexactParams {
   const uint64_t *kstart;
   uint32_t kcount;
   uint2 *vscratch;             // lanes * (seed_size + 3)
+  uint32_t min_len;            // context_seed_kernel: shorter windows are left
+  uint32_t *list, *list_n;     // the list of the windows left
   fmi_inexact_region *out;     // 2 * nwin * region_cap
   uint32_t *nreg;
   uint8_t *status;
@@ -501,6 +503,7 @@ struct RegionSink {
   int32_t start, len;
   int32_t *final_pos;
   uint8_t st;
+  __device__ __forceinline__ bool full() const { return false; }   // its caps are counted past
   __device__ __forceinline__ void add(const VhRec &r) {
     add(r, (type ? r.dir : !r.dir) ? 1u : 0u, WinIv{r.k, kWinNone, r.l - r.k + 1u});
   }
@@ -576,8 +579,8 @@ __device__ __forceinline__ uint32_t dedup_list(fmi_inexact_region *out, uint32_t
 
 // ---- windows by row contexts: the records of a window and strand are kept
 // (16 bytes each) and become regions together, one region a lane.
-constexpr uint32_t kWinRecs = 64;      // records and rows a wavefront takes at once
-constexpr uint8_t kWinRedo = 0x80;     // status of a window with more of them
+constexpr uint32_t kWinRecs = 64;      // rows of its records that a wavefront takes at once
+constexpr uint8_t kWinLeft = 0x80;     // status of a window with more of them
 
 // A kept record: x the first row, or (known) that row's suffix; y its rows (as
 // many as it gives regions for) | known << 8 | direction << 9 | (len_calc - len
@@ -588,6 +591,7 @@ struct RecordSink {
   int32_t start, len;
   int32_t final_pos;
   uint8_t st;
+  __device__ __forceinline__ bool full() const { return total > kWinRecs; }
   __device__ __forceinline__ void add(const VhRec &r, uint32_t dsel, const WinIv &iv) {
     if (nrec++ >= rec_cap) { st |= 1; return; }      // the reference's list holds 20000
     int32_t dl, final_err;
@@ -750,25 +754,36 @@ __device__ __forceinline__ uint32_t regions_of(const InexactParams &P, const Rec
 // over 64 Mbp).  REGS (seed_size <= 32): the window's bases are packed into
 // registers once (vh_regs) for both strands, so the helper's LF steps and
 // comparisons read no read bytes from memory.
-// REDO: only the windows that context_seed_kernel left (status kWinRedo).
-template <bool REGS, bool REDO>
+// kWinsLeft: only the windows that context_seed_kernel left for their rows
+// (kWinLeft), by their contexts too: with LF steps the longest of them took 0.6 ms
+// more of 5.7 for 2 M windows over 64 Mbp.
+// kWinsListed: P.list[0 .. *P.list_n), by LF steps: the windows left where some
+// have fewer than min_len bases, in one launch with those (each kind is a few
+// long chains, and launches one after the other take their sum).
+enum : int { kWinsAll, kWinsLeft, kWinsListed };
+
+template <bool REGS, int WHICH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void inexact_seed_kernel(InexactParams P) {
-  __shared__ uint32_t words[REDO ? kWinWords * 256u : 1u];
+  constexpr bool LEFT = WHICH == kWinsLeft, LISTED = WHICH == kWinsListed;
+  __shared__ uint32_t words[LEFT ? kWinWords * 256u : 1u];
   const uint64_t lane = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   uint2 *vb = P.vscratch + lane * (uint64_t)(P.seed_size + 3);
-  const uint64_t wlane = lane & 63u;
+  const uint64_t wlane = lane & 63u, count = LISTED ? (uint64_t)*P.list_n : P.nwin;
   // a wavefront's lanes take consecutive windows and go on together
-  for (uint64_t g0 = lane - wlane; g0 < P.nwin; g0 += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t rd0 = wave_owner(P.win_base, P.nreads, P.nwin, g0);
-    const bool mine = g0 + wlane < P.nwin;
-    const uint64_t g = mine ? g0 + wlane : P.nwin - 1u, rd = mine ? rd0 : P.nreads - 1u;
+  for (uint64_t g0 = lane - wlane; g0 < count; g0 += (uint64_t)gridDim.x * blockDim.x) {
+    uint64_t g = g0 + wlane, rd = 0;
+    if (!LISTED) rd = wave_owner(P.win_base, P.nreads, P.nwin, g0);
+    if (g >= count || (LEFT && P.status[2 * g] != kWinLeft)) continue;
+    if (LISTED) {
+      g = P.list[g];
+      rd = owner(P.win_base, P.nreads, g);
+    }
     const uint64_t off = P.offsets[rd];
     const int32_t len = (int32_t)(P.offsets[rd + 1] - off);
     const int32_t w = (int32_t)(g - P.win_base[rd]);
     const int32_t num_seeds = len / (int32_t)P.seed_size;
     const int32_t ws = w * (int32_t)P.seed_size;
     const int32_t we = w < num_seeds ? ws + (int32_t)P.seed_size - 1 : len - 1;
-    if (!mine || (REDO && P.status[2 * g] != kWinRedo)) continue;
     const bool run = we - ws >= 2;
     int32_t final_pos = 0;
     VhRegs WR{0ull, 0u, ws};
@@ -781,7 +796,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
                    type ? (uint32_t)we : (uint32_t)(len - ws - 1), (uint32_t)len, (uint32_t)w,
                    ws, we - ws + 1, &final_pos, 0};
       if (run) {
-        if (REDO) win_run(P.ix, WR, ws, we, s, vb, words + threadIdx.x, S);
+        if (LEFT) win_run(P.ix, WR, ws, we, s, vb, words + threadIdx.x, S);
         else if (REGS) vh_run(P.ix, WR, ws, we, s, 0u, vb, S);
         else vh_run(P.ix, VhBytes{P.reads + off}, ws, we, s, 0u, vb, S);
       }
@@ -794,11 +809,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
 // The same windows on an index with row contexts, seed_size <= kWinMax: they go
 // by their rows' contexts and the k-mer table instead of an LF step per base
 // and branch (win_run), and their records become regions a wavefront at a time
-// (regions_of).  A window with more than kWinRecs records or rows on a
-// strand is left to inexact_seed_kernel.  vscratch: per lane seed_size + 3
-// intervals and kWinRecs records.  At 4 waves per SIMD 31 registers spill;
-// 3 waves (none) took 8.6 ms where 4 took 7.6, 5 waves 10.0 (before the loops
-// were parted).
+// (regions_of).  A window with more than kWinRecs rows on a strand, or of fewer
+// than min_len bases, is left to inexact_seed_kernel.  vscratch: per lane seed_size + 3 intervals and kWinRecs
+// records.  At 4 waves per SIMD 31 registers spill; 3 waves (none) took 8.6 ms
+// where 4 took 7.6, 5 waves 10.0 (before the loops were parted).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void context_seed_kernel(InexactParams P) {
   __shared__ uint32_t words[kWinWords * 256u];
   const uint64_t lane = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -818,9 +832,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     const int32_t num_seeds = len / (int32_t)P.seed_size;
     const int32_t ws = w * (int32_t)P.seed_size;
     const int32_t we = w < num_seeds ? ws + (int32_t)P.seed_size - 1 : len - 1;
-    const bool run = mine && we - ws >= 2;
+    const bool any = mine && we - ws >= 2, run = any && (uint32_t)(we - ws + 1) >= P.min_len;
     int32_t final_pos = 0;
-    bool redo = false;
+    bool left = any && !run;
     VhRegs WR{0ull, 0u, ws};
     if (run) WR = vh_regs(P.reads + off, ws, (uint32_t)(we - ws + 1));
     for (uint32_t s = 0; s < 2; ++s) {
@@ -830,7 +844,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
                    final_pos, 0};
       if (run) win_run(P.ix, WR, ws, we, s, vb, words + threadIdx.x, S);
       final_pos = S.final_pos;
-      redo |= S.n > kWinRecs || S.total > kWinRecs;
+      left |= S.full();
       const WinOf wo{(uint32_t)rd,
                      (uint32_t)(uint16_t)(type ? ws : len - we - 1),
                      (uint32_t)(uint16_t)(type ? we : len - ws - 1),
@@ -840,14 +854,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
                      we - ws + 1};
       uint8_t st = S.st;
       const uint32_t kept =
-          regions_of(P, S, redo ? 0u : S.n, wo, P.out + slot * P.region_cap, st);
+          regions_of(P, S, left ? 0u : S.n, wo, P.out + slot * P.region_cap, st);
       if (mine) {
         P.nreg[slot] = kept;
         P.status[slot] = st;
       }
     }
-    if (redo) P.status[2 * g] = kWinRedo;
+    if (left) P.status[2 * g] = kWinLeft;
   }
+}
+
+// The windows that context_seed_kernel left, in the order of their numbers within
+// a group's 4096: appended to list with an atomic per group.
+__global__ __launch_bounds__(256) void left_windows_kernel(InexactParams P) {
+  __shared__ uint32_t waves[4], base;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint64_t g0 = (uint64_t)blockIdx.x * 4096u + 16u * threadIdx.x;
+  uint32_t marks = 0u;
+  for (uint32_t j = 0; j < 16u; ++j)
+    if (g0 + j < P.nwin && P.status[2 * (g0 + j)] == kWinLeft) marks |= 1u << j;
+  const uint32_t own = (uint32_t)__builtin_popcount(marks);
+  uint32_t incl = own;
+#pragma unroll
+  for (uint32_t d = 1u; d < 64u; d <<= 1) {
+    const uint32_t v = __shfl_up(incl, d);
+    if (lane >= d) incl += v;
+  }
+  if (lane == 63u) waves[wave] = incl;
+  __syncthreads();
+  const uint32_t w0 = waves[0], w1 = waves[1], w2 = waves[2], all = w0 + w1 + w2 + waves[3];
+  if (threadIdx.x == 0u && all) base = atomicAdd(P.list_n, all);
+  __syncthreads();
+  if (!own) return;
+  uint32_t at = base + (wave > 0u ? w0 : 0u) + (wave > 1u ? w1 : 0u) + (wave > 2u ? w2 : 0u) + incl - own;
+  for (; marks; marks &= marks - 1u) P.list[at++] = (uint32_t)g0 + (uint32_t)__builtin_ctz(marks);
 }
 
 inline dim3 grid_for(uint64_t m) {
@@ -989,24 +1029,44 @@ int map_inexact_seeds(const fmi_index *ix, const uint8_t *reads, const uint64_t 
     const uint64_t per = (uint64_t)(seed_size + 3) * sizeof(uint2);
     const uint64_t max_lanes = std::min<uint64_t>(1ull << 19, ((1ull << 30) / per) / 256 * 256);
     if (lanes > max_lanes) lanes = max_lanes;
-    // windows by context: as many lanes as are resident (4 waves per SIMD),
-    // each with its record list too
-    const bool ctx = seed_size <= kWinMax && ix->dev.d[0].ctx;
+    // Windows by context where the table holds the first bases of their strings
+    // (a base shorter than the window) and a string occurs in few places by
+    // chance: at 1/16 row a string, or 1/256 where the table holds fewer than
+    // log4 n bases.  By LF steps and by contexts, 100 K windows of 15 and 16 bases
+    // over 64 Mbp: k = 15 1.98, 2.34 and 1.61, 1.10 ms; k = 12 1.99, 1.51 and
+    // 1.60, 1.14; no table 1.97, 2.31 and 1.61, 1.81, and 1.29, 1.13 of 18 bases.
+    const uint32_t K = ix->dev.kmer_k;
+    uint32_t once = 0u;
+    while ((1ull << (2u * once)) < ix->n) ++once;
+    const uint32_t min_len = std::max(K + 1u, once + (K + 1u >= once ? 2u : 4u));
+    // as many lanes as are resident (4 waves per SIMD), each with its record list
+    // too, then the list of the windows left (numbers of 32 bits)
+    const bool ctx = ix->dev.d[0].ctx && seed_size <= kWinMax && seed_size >= min_len &&
+                     nwin < (1ull << 32);
+    const bool some_short = ctx && min_seed_size < min_len;
     const uint64_t ctx_lanes = std::min<uint64_t>(lanes, 1ull << 18);
-    SEED_TRY(hipMalloc(&vscr, std::max<uint64_t>(
-                                  lanes * per, ctx ? ctx_lanes * (per + kWinRecs * 16ull) : 0ull)));
+    const uint64_t lane_bytes =
+        std::max<uint64_t>(lanes * per, ctx ? ctx_lanes * (per + kWinRecs * 16ull) : 0ull);
+    SEED_TRY(hipMalloc(&vscr, lane_bytes + (some_short ? 64ull + 4ull * nwin : 0ull)));
+    uint32_t *list = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(vscr) + lane_bytes);
     InexactParams P{ix->dev, reads, offsets, base, nwin, nreads, seed_size, rec_cap, region_cap,
-                    ix->d_koffset, ix->d_kstart, (uint32_t)ix->kstart.size(), vscr, regions,
-                    nregions, status};
+                    ix->d_koffset, ix->d_kstart, (uint32_t)ix->kstart.size(), vscr, min_len,
+                    list + 16, list, regions, nregions, status};
     // windows are at most seed_size bases (the remainder window is shorter)
     const dim3 grid((uint32_t)(lanes / 256));
     if (ctx) {
       context_seed_kernel<<<dim3((uint32_t)(ctx_lanes / 256)), 256, 0, s>>>(P);
-      inexact_seed_kernel<true, true><<<grid, 256, 0, s>>>(P);
+      if (some_short) {
+        SEED_TRY(launch_zero(list, 1, s));
+        left_windows_kernel<<<dim3((uint32_t)((nwin + 4095) / 4096)), 256, 0, s>>>(P);
+        inexact_seed_kernel<true, kWinsListed><<<grid, 256, 0, s>>>(P);
+      } else {
+        inexact_seed_kernel<true, kWinsLeft><<<grid, 256, 0, s>>>(P);
+      }
     } else if (seed_size <= 32u) {
-      inexact_seed_kernel<true, false><<<grid, 256, 0, s>>>(P);
+      inexact_seed_kernel<true, kWinsAll><<<grid, 256, 0, s>>>(P);
     } else {
-      inexact_seed_kernel<false, false><<<grid, 256, 0, s>>>(P);
+      inexact_seed_kernel<false, kWinsAll><<<grid, 256, 0, s>>>(P);
     }
     SEED_TRY(hipGetLastError());
   }

@@ -47,6 +47,7 @@ constexpr uint32_t kVhWaits = 0xFFFFFFFFu;
 struct VtSink : VhSink {
   const DevIndex *ix;
   using VhSink::add;
+  __device__ __forceinline__ bool full() const { return false; }   // it counts them all
   __device__ __forceinline__ void add(VhRec &r, uint32_t dsel, const WinIv &iv) {
     if (mm_only && r.nmm && r.kind != FMI_MISMATCH) return;
     r.k = cnt >= cap || iv.q == kWinNone ? iv.k : dir_of(*ix, dsel).isa[iv.q];

@@ -162,8 +162,8 @@ __device__ __forceinline__ bool win_extend(const DevDir &D, uint32_t k, uint32_t
 // forward vector's.  s, nf: the window's L bases in the half's feed order as
 // physical symbols, and their N flags; vb: L intervals of scratch; lds:
 // kWinWords words in LDS, word i at lds[i * 256].  Records
-// go to S.add(r, dsel, iv) in the helper's order; r carries the record state
-// (its k, l are not used).
+// go to S.add(r, dsel, iv) in the helper's order, until S.full(); r carries the
+// record state (its k, l are not used).
 template <class Sink>
 __device__ __forceinline__ void win_half(const DevIndex &ix, uint32_t dir, uint32_t strand,
                                          uint64_t s, uint32_t nf, uint32_t L, int32_t start,
@@ -296,7 +296,7 @@ __device__ __forceinline__ void win_half(const DevIndex &ix, uint32_t dir, uint3
     S.add(r, dsel, WinIv{k, kWinNone, l - k + 1u});
     nodes ^= 1u << L;
   }
-  for (nodes &= ~wide; nodes;) {
+  for (nodes &= ~wide; nodes && !S.full();) {
     m = 31u - (uint32_t)__builtin_clz(nodes);
     nodes ^= 1u << m;
     const bool exact = m == L, last = m == L - 1u;
@@ -348,7 +348,7 @@ __device__ __forceinline__ void win_half(const DevIndex &ix, uint32_t dir, uint3
       }
     }
   }
-  while (wide) {
+  while (wide && !S.full()) {
     m = 31u - (uint32_t)__builtin_clz(wide);
     wide ^= 1u << m;
     const bool last = m == L - 1u;
@@ -428,8 +428,8 @@ __device__ __forceinline__ void win_run(const DevIndex &ix, const VhRegs &W, int
   VhRec r{0, 0, -1, 0, 0, 0, 0, 0};
   for (uint32_t dir = 0; dir < 2u; ++dir) {
     r.dir = dir;
-    win_half(ix, dir, strand, dir ? code : rev, dir ? nf : rnf, L, start, end, vb, lds,
-             r, S);
+    if (!S.full())
+      win_half(ix, dir, strand, dir ? code : rev, dir ? nf : rnf, L, start, end, vb, lds, r, S);
   }
 }
 

@@ -13,6 +13,9 @@ region differs from the text in exactly one base, and the kept regions of a
 strand are at least 10 apart on a contig (the dedup's fixed point).
 GPU: fmi_map_inexact_seeds_batch through the C ABI against the oracle,
 record for record, status bits included."""
+import ctypes as C
+import time
+
 import numpy as np
 import pytest
 
@@ -212,5 +215,104 @@ def test_gpu_inexact_windows_by_context(gpu_engine, n, kmer):
                     got = res.regions(w, s)
                     assert got.tobytes() == regs.tobytes(), (seed_size, i, t)
     finally:
+        batch.free()
+        ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,kmer", [(4096, 0), (4096, 6), (4097, 6), (60_000, 0), (60_000, 9),
+                                    (60_000, 12)])
+def test_gpu_inexact_windows_left(gpu_engine, n, kmer):
+    """Windows around the length from which they go by contexts (8 to 20 bases
+    here), with remainder windows shorter than it and without, among windows of
+    many rows (90 copies) and copies of which a window has one more than a
+    wavefront takes: in more windows than one group lists, region for region the
+    oracle's."""
+    hp = gpu_engine
+    rng = np.random.default_rng(55)
+    g = rng.integers(0, 4, n).astype(np.uint8)
+    if n > 10_000:
+        for i in range(90):
+            g[1000 + 50 * i:1040 + 50 * i] = g[1000:1040]
+        for i in range(30):
+            g[9000 + 50 * i:9040 + 50 * i] = g[9000:9040]
+            g[9010 + 50 * i + int(rng.integers(0, 20))] ^= 1
+    koff, kstart, lens = karyo(n, 2)
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(kstart, kstart + np.array(lens, np.uint64) - 1)
+    ix.to_device()
+    ix.expand()
+    if kmer:
+        ix.kmer_table(kmer)
+    o = fo.Oracle(g, ratio=16)
+    reads = []
+    for i in range(300):
+        L = int(rng.integers(0, 120))
+        at = int(rng.choice([1000, 9000])) + 50 * int(rng.integers(0, 20)) \
+            if n > 10_000 and i % 3 == 0 else int(rng.integers(0, n - 120))
+        w = g[at:at + L].copy()
+        e = rng.random(L) < 0.03
+        w[e] = rng.integers(0, 5, int(e.sum()))
+        reads.append(w)
+    offs = np.concatenate([[0], np.cumsum([len(r) for r in reads])]).astype(np.uint64)
+    many = 8                                         # the batch over: 13,000 windows and more
+    batch = hp.ReadBatch(np.tile(np.concatenate(reads).astype(np.uint8), many),
+                         np.concatenate([[0], np.cumsum(np.tile(np.diff(offs.astype(np.int64)), many))])
+                         .astype(np.uint64))
+    try:
+        for seed_size, min_seed in ((9, 3), (9, 9), (10, 5), (11, 11), (12, 4), (13, 13), (18, 3),
+                                    (20, 16)):
+            res = hp.map_inexact_seeds_batch(ix, batch, seed_size, min_seed, 256, 32)
+            per = int(res.window_base[len(reads)])
+            for i, W in enumerate(reads):
+                want = o.map_inexact_seeds(W, seed_size, min_seed, koff, kstart, read=i,
+                                           rec_cap=256, region_cap=32)
+                for c in (0, many - 1):
+                    w0 = int(res.window_base[i]) + c * per
+                    for t, (regs, st) in enumerate(want):
+                        w, s = w0 + t // 2, t % 2
+                        assert int(res.status[w, s]) == st, (seed_size, i, t)
+                        got = res.regions(w, s).copy()
+                        got["read"] -= c * len(reads)
+                        assert got.tobytes() == regs.tobytes(), (seed_size, i, t)
+    finally:
+        batch.free()
+        ix.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seed_size,min_seed", [(12, 12), (18, 3)])
+def test_gpu_inexact_short_windows_cost(gpu_engine, seed_size, min_seed):
+    """Windows so short that most have more rows than a wavefront takes at once
+    (12 bases over 16 Mbp, remainders of 10) are searched once: the call takes at
+    most 1.25 times what it takes without row contexts, 2.2 and 2.3 times where
+    they were searched by them first and again."""
+    hp = gpu_engine
+    rng = np.random.default_rng(56)
+    g = rng.integers(0, 4, 16_000_000).astype(np.uint8)
+    koff, kstart, lens = karyo(len(g), 2)
+    n, L = 20_000, 100
+    at = rng.integers(0, len(g) - L, n)
+    batch = hp.ReadBatch(g[at[:, None] + np.arange(L)].reshape(-1), np.arange(n + 1, dtype=np.uint64) * L)
+    took = {}
+    ix = hp.Index.build_gpu(g, 16).expand()
+    ix.kmer_table(13)
+    got, nwin = C.c_uint64(), n * (L // seed_size + 1)
+    bufs = [hp.DeviceBuffer(b) for b in (2 * nwin * 16 * 48, 2 * nwin * 4, 2 * nwin)]
+    try:
+        for form in ("contexts", "none"):
+            if form == "none":
+                ix.drop_contexts()
+            for _ in range(6):
+                t = time.perf_counter()
+                hp.check(hp.lib().fmi_map_inexact_seeds_batch(
+                    ix.h, batch.d_reads.ptr, batch.d_offsets.ptr, n, seed_size, min_seed, 256, 16, nwin,
+                    bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, C.byref(got), None))
+                took[form] = min(took.get(form, 1.0), time.perf_counter() - t)
+        print(seed_size, took)
+        assert took["contexts"] < 1.25 * took["none"], took
+    finally:
+        for b in bufs:
+            b.free()
         batch.free()
         ix.close()
