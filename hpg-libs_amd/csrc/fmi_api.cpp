@@ -726,7 +726,10 @@ int fmi_device_alloc(void **d_ptr, size_t bytes) {
   if (!d_ptr) return fail(FMI_EINVAL, "NULL argument");
   *d_ptr = nullptr;
   hipError_t e = hipMalloc(d_ptr, bytes ? bytes : 1);
-  if (e != hipSuccess) return fail(FMI_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();   // else the next launch's check reports it
+    return fail(FMI_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+  }
   return FMI_OK;
 }
 

@@ -66,6 +66,19 @@ def test_contexts_give_way_to_a_table(gpu_engine, text):
         ix.close()
 
 
+def test_failed_allocation_leaves_no_error(gpu_engine):
+    hp = gpu_engine
+    g = np.random.default_rng(504).integers(0, 4, 5000).astype(np.uint8)
+    ix = hp.Index.build(g, 16).to_device()
+    batch = hp.ReadBatch(g[:100], np.array([0, 100], np.uint64))
+    with pytest.raises(hp.FmiError):
+        hp.DeviceBuffer(1 << 60)
+    counts, _ = hp.search1_batch(ix, batch, cap=4)   # its launch's check saw that failure
+    assert counts[0, 0] >= 1
+    batch.free()
+    ix.close()
+
+
 def test_dropped_contexts(gpu_engine):
     hp = gpu_engine
     g = np.random.default_rng(502).integers(0, 4, 50_000).astype(np.uint8)
