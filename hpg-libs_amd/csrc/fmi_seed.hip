@@ -1041,13 +1041,19 @@ int map_inexact_seeds(const fmi_index *ix, const uint8_t *reads, const uint64_t 
     const uint32_t min_len = std::max(K + 1u, once + (K + 1u >= once ? 2u : 4u));
     // as many lanes as are resident (4 waves per SIMD), each with its record list
     // too, then the list of the windows left (numbers of 32 bits)
-    const bool ctx = ix->dev.d[0].ctx && seed_size <= kWinMax && seed_size >= min_len &&
-                     nwin < (1ull << 32);
+    bool ctx = ix->dev.d[0].ctx && seed_size <= kWinMax && seed_size >= min_len &&
+               nwin < (1ull << 32);
     const bool some_short = ctx && min_seed_size < min_len;
     const uint64_t ctx_lanes = std::min<uint64_t>(lanes, 1ull << 18);
     const uint64_t lane_bytes =
         std::max<uint64_t>(lanes * per, ctx ? ctx_lanes * (per + kWinRecs * 16ull) : 0ull);
-    SEED_TRY(hipMalloc(&vscr, lane_bytes + (some_short ? 64ull + 4ull * nwin : 0ull)));
+    hipError_t got = hipMalloc(&vscr, lane_bytes + (some_short ? 64ull + 4ull * nwin : 0ull));
+    if (got != hipSuccess && ctx) {              // LF steps need 88 MB of the 310
+      (void)hipGetLastError();
+      ctx = false;
+      got = hipMalloc(&vscr, lanes * per);
+    }
+    SEED_TRY(got);
     uint32_t *list = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(vscr) + lane_bytes);
     InexactParams P{ix->dev, reads, offsets, base, nwin, nreads, seed_size, rec_cap, region_cap,
                     ix->d_koffset, ix->d_kstart, (uint32_t)ix->kstart.size(), vscr, min_len,

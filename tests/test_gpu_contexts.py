@@ -2,6 +2,8 @@
 allocates after fmi_index_expand fits as if there were none (the k-mer tables,
 also where other memory ran short meanwhile), they can be given up, and the
 searches answer alike with and without them, record for record the oracle's."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -77,6 +79,52 @@ def test_failed_allocation_leaves_no_error(gpu_engine):
     assert counts[0, 0] >= 1
     batch.free()
     ix.close()
+
+
+def test_inexact_seeds_in_little_memory(gpu_engine):
+    """600 K windows with 200 MB free: the lanes' record lists (312 MB with their
+    intervals) do not fit, the intervals (88 MB) do, and the regions are the
+    same."""
+    hp = gpu_engine
+    rng = np.random.default_rng(503)
+    g = rng.integers(0, 4, 200_000).astype(np.uint8)
+    ix = hp.Index.build(g, 16)
+    ix.set_karyotype(np.ones(1, np.uint64), np.array([len(g)], np.uint64))
+    ix.to_device().expand()
+    ix.kmer_table(10)
+    n, nwin = 100_000, 600_000
+    at = rng.integers(0, len(g) - 108, n)
+    batch = hp.ReadBatch(g[at[:, None] + np.arange(108)].reshape(-1), np.arange(n + 1, dtype=np.uint64) * 108)
+    bufs = [hp.DeviceBuffer(b) for b in (2 * nwin * 48, 2 * nwin * 4, 2 * nwin)]
+    got, out, blocks = C.c_uint64(), [], []
+
+    def call():
+        hp.check(hp.lib().fmi_map_inexact_seeds_batch(ix.h, batch.d_reads.ptr, batch.d_offsets.ptr, n, 18,
+                                                      16, 64, 1, nwin, bufs[0].ptr, bufs[1].ptr,
+                                                      bufs[2].ptr, C.byref(got), None))
+        out.append([b.download(np.uint8, b.nbytes) for b in bufs])
+
+    try:
+        call()
+        blocks = [fill(hp, 1 << 30)]
+        try:
+            for _ in range(256):
+                blocks.append(hp.DeviceBuffer(40 * MB))
+        except hp.FmiError:
+            pass
+        for b in blocks[-5:]:
+            b.free()
+        call()
+        assert got.value == nwin and np.array_equal(out[0][1], out[1][1])
+        assert np.array_equal(out[0][2], out[1][2])
+        kept = out[0][1].view(np.uint32) > 0
+        assert kept.sum() > nwin and np.array_equal(out[0][0].reshape(-1, 48)[kept],
+                                                    out[1][0].reshape(-1, 48)[kept])
+    finally:
+        for b in blocks + bufs:
+            b.free()
+        batch.free()
+        ix.close()
 
 
 def test_dropped_contexts(gpu_engine):
