@@ -49,12 +49,9 @@ __device__ __forceinline__ uint32_t wave_owner(const int32_t *di, uint32_t n, in
   return lo;
 }
 
-constexpr uint32_t kEncTile = 8192;   // bytes of seq per workgroup and round
-constexpr uint32_t kEncEnds = 1024;   // reads of a tile whose ends fit in LDS
-
 // The bytes seq[data_indices[0] + p], p < nbytes = data_indices[nreads] -
 // data_indices[0] (data_indices index seq, as the reference's
-// batch->seq[batch->data_indices[r]]), in tiles of kEncTile aligned bytes:
+// batch->seq[batch->data_indices[r]]), in tiles of TILE aligned bytes:
 // every NUL terminator is dropped, every other byte p of read r goes to
 // codes[base_off + p - r].  Threads also write offsets[read_off + i] =
 // data_indices[i] - data_indices[0] - i, i <= nreads (from 0: a caller
@@ -68,14 +65,16 @@ constexpr uint32_t kEncEnds = 1024;   // reads of a tile whose ends fit in LDS
 // two wavefronts find the reads of a tile's first and last byte, a
 // thread takes 16 bytes with one short search among the tile's reads, and
 // the tile's codes leave through LDS, laid out like their 16-byte pieces in
-// codes, as whole 16-byte stores: 60 us, 1.7 TB/s.
+// codes, as whole 16-byte stores: 59 us, 1.7 TB/s.
+template <uint32_t TILE>
 __global__ __launch_bounds__(256) void fastq_encode_kernel(const char *seq, const int32_t *di,
                                                            uint32_t nreads, uint64_t nbytes,
                                                            uint64_t ntiles, uint64_t base_off,
                                                            uint64_t read_off, uint8_t *codes,
                                                            uint64_t *offsets) {
-  __shared__ __align__(16) uint8_t out[kEncTile + 32u];
-  __shared__ int64_t ends[kEncEnds];
+  constexpr uint32_t kEnds = TILE / 8u;            // reads of a tile whose ends fit in LDS
+  __shared__ __align__(16) uint8_t out[TILE + 32u];
+  __shared__ int64_t ends[kEnds];
   __shared__ uint32_t bounds[2];
   const int64_t d0 = di[0];
   for (uint64_t p = (uint64_t)blockIdx.x * 256u + threadIdx.x; p <= nreads;
@@ -87,9 +86,9 @@ __global__ __launch_bounds__(256) void fastq_encode_kernel(const char *seq, cons
   const int64_t mis = (int64_t)(reinterpret_cast<uintptr_t>(first) & 15u);
   const uint8_t *base = first - mis;           // byte x of base is byte p = x - mis
   for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t x0 = (int64_t)(tile * kEncTile);
+    const int64_t x0 = (int64_t)(tile * TILE);
     const int64_t pf = max(x0 - mis, (int64_t)0);
-    const int64_t pl = min(x0 + (int64_t)kEncTile - mis, (int64_t)nbytes) - 1;
+    const int64_t pl = min(x0 + (int64_t)TILE - mis, (int64_t)nbytes) - 1;
     if (pf > pl) break;                        // past the last byte
     const uint32_t wave = threadIdx.x >> 6;
     if (wave < 2u) {
@@ -100,7 +99,7 @@ __global__ __launch_bounds__(256) void fastq_encode_kernel(const char *seq, cons
     const uint32_t r0 = bounds[0], r1 = bounds[1];
     // where read r0 + i ends, its NUL included
     const uint32_t nin = r1 >= r0 ? r1 - r0 + 1u : 1u;
-    const bool staged = nin <= kEncEnds;
+    const bool staged = nin <= kEnds;
     if (staged)
       for (uint32_t i = threadIdx.x; i < nin; i += 256u) ends[i] = (int64_t)di[r0 + i + 1u] - d0;
     __syncthreads();
@@ -110,7 +109,7 @@ __global__ __launch_bounds__(256) void fastq_encode_kernel(const char *seq, cons
     auto end_of = [&](uint32_t i) -> int64_t {
       return staged ? ends[i] : (int64_t)di[r0 + i + 1u] - d0;
     };
-    for (uint32_t c = threadIdx.x; c < kEncTile / 16u; c += 256u) {
+    for (uint32_t c = threadIdx.x; c < TILE / 16u; c += 256u) {
       const int64_t pc = x0 + 16 * (int64_t)c - mis;
       if (pc > pl || pc + 15 < pf) continue;
       const uint4 v = *reinterpret_cast<const uint4 *>(base + x0 + 16 * (int64_t)c);
@@ -132,14 +131,14 @@ __global__ __launch_bounds__(256) void fastq_encode_kernel(const char *seq, cons
           continue;
         }
         const int64_t o = p - (int64_t)lo - pf;
-        if (o >= 0 && o < (int64_t)kEncTile)
+        if (o >= 0 && o < (int64_t)TILE)
           out[m + (uint32_t)o] = (uint8_t)(e[j >> 2] >> (8u * (j & 3u)));
       }
     }
     __syncthreads();
     // codes o0 .. of the tile: its bytes less the NULs among them
     int64_t n = pl + 1 - (int64_t)r1 - (end_of(nin - 1u) - 1 == pl ? 1 : 0) - o0;
-    n = o0 < 0 ? 0 : min(min(n, (int64_t)kEncTile), ncodes - o0);
+    n = o0 < 0 ? 0 : min(min(n, (int64_t)TILE), ncodes - o0);
     for (uint32_t c = threadIdx.x; 16 * (int64_t)c < (int64_t)m + n; c += 256u) {
       const uint32_t a = 16u * c;
       if (a >= m && (int64_t)a + 16 <= (int64_t)m + n) {
@@ -151,6 +150,31 @@ __global__ __launch_bounds__(256) void fastq_encode_kernel(const char *seq, cons
     }
     __syncthreads();
   }
+}
+
+// The same, a thread per byte with a search of its own: for a small batch, whose
+// tiles are a few workgroups with a chain of loads each.
+__global__ __launch_bounds__(256) void fastq_encode_small_kernel(const char *seq, const int32_t *di,
+                                                                 uint32_t nreads, uint64_t nbytes,
+                                                                 uint64_t base_off,
+                                                                 uint64_t read_off, uint8_t *codes,
+                                                                 uint64_t *offsets) {
+  const uint64_t p = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+  const int64_t d0 = di[0];
+  if (p <= nreads) offsets[read_off + p] = (uint64_t)((int64_t)di[p] - d0 - (int64_t)p);
+  if (p >= nbytes || nreads == 0) return;
+  const int64_t at = d0 + (int64_t)p;
+  const uint32_t c = (uint8_t)seq[at];               // before the search it does not depend on
+  uint32_t lo = 0, hi = nreads;                      // the last read that starts at or before it
+  while (hi - lo > 1u) {
+    const uint32_t mid = lo + (hi - lo) / 2u;
+    if ((int64_t)di[mid] <= at) lo = mid;
+    else hi = mid;
+  }
+  if (at == (int64_t)di[lo + 1] - 1) return;         // its NUL
+  const int64_t o = (int64_t)p - (int64_t)lo;
+  if (o >= 0 && nbytes >= nreads && (uint64_t)o < nbytes - nreads)
+    codes[base_off + (uint64_t)o] = (uint8_t)encode4(c);
 }
 
 // 2-bit packing of nbases codes: thread t packs bases 16t .. 16t + 15 into
@@ -180,13 +204,28 @@ __global__ __launch_bounds__(256) void pack_codes_kernel(const uint8_t *codes, u
 hipError_t launch_fastq_encode(const char *seq, const int32_t *data_indices, uint32_t nreads,
                                uint64_t nbytes, uint64_t base_off, uint64_t read_off,
                                uint8_t *codes, uint64_t *offsets, hipStream_t s) {
-  // a tile more than the bytes fill: they may start 15 bytes into the first.
-  // With no bytes the one workgroup writes the offsets alone.
-  const uint64_t ntiles = nbytes ? (nbytes + 15u + kEncTile - 1u) / kEncTile : 0u;
+  // A thread per byte up to 512 KiB: 6.2 us for 100 reads of 100 bases, 7.1 for
+  // 3000, where tiles take 8.1 and 8.7, but 11.8 and 9.1 for 10,000.
+  if (nbytes <= (512u << 10) && nreads <= (512u << 10)) {
+    const uint64_t work = std::max<uint64_t>(nbytes, (uint64_t)nreads + 1u);
+    hipLaunchKernelGGL(fastq_encode_small_kernel, dim3((uint32_t)((work + 255u) / 256u)), dim3(256),
+                       0, s, seq, data_indices, nreads, nbytes, base_off, read_off, codes, offsets);
+    return hipGetLastError();
+  }
+  // Tiles of 4096 bytes where those of 8192 would be too few to fill the device:
+  // 9.1 us for 1 MB where they take 12.4, 18.5 and 18.9 for 10 MB, but 61.0 and
+  // 59.2 for 50 MB.  A tile more than the bytes fill: they may start 15 bytes into
+  // the first.  With no bytes the one workgroup writes the offsets alone.
+  const uint32_t tile = nbytes <= (16u << 20) ? 4096u : 8192u;
+  const uint64_t ntiles = nbytes ? (nbytes + 15u + tile - 1u) / tile : 0u;
   const uint64_t want = std::max<uint64_t>(ntiles, ((uint64_t)nreads + 2048u) / 2048u);
-  const uint32_t grid = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(want, 1u), 65536u);
-  hipLaunchKernelGGL(fastq_encode_kernel, dim3(grid), dim3(256), 0, s, seq, data_indices, nreads,
-                     nbytes, ntiles, base_off, read_off, codes, offsets);
+  const dim3 grid((uint32_t)std::min<uint64_t>(std::max<uint64_t>(want, 1u), 65536u));
+  if (tile == 4096u)
+    hipLaunchKernelGGL(fastq_encode_kernel<4096u>, grid, dim3(256), 0, s, seq, data_indices, nreads,
+                       nbytes, ntiles, base_off, read_off, codes, offsets);
+  else
+    hipLaunchKernelGGL(fastq_encode_kernel<8192u>, grid, dim3(256), 0, s, seq, data_indices, nreads,
+                       nbytes, ntiles, base_off, read_off, codes, offsets);
   return hipGetLastError();
 }
 
