@@ -1258,6 +1258,17 @@ struct LocateParams {
   uint32_t *nrows;
 };
 
+// A thread per (interval, slot of cap).
+__global__ __launch_bounds__(256) void locate_slots_kernel(LocateParams P) {
+  const uint32_t g = blockIdx.x * 256u + threadIdx.x, iv = g / P.cap, j = g - iv * P.cap;
+  if (iv >= P.nintervals) return;
+  const int64_t k = P.k[(uint64_t)iv * P.stride], l = P.l[(uint64_t)iv * P.stride];
+  const int64_t cnt = k >= 0 && l <= (int64_t)P.ix.n && k <= l ? l - k + 1 : 0;
+  const uint32_t rows = cnt < (int64_t)P.cap ? (uint32_t)cnt : P.cap;
+  if (j == 0u) P.nrows[iv] = rows;
+  if (j < rows) P.pos[g] = sa_value(dir_of(P.ix, P.dsel), P.ix.ratio, P.ix.n, (uint32_t)(k + j));
+}
+
 // A lane reads its interval and writes its row count; the rows of a
 // wavefront's 64 intervals are then shared out among its lanes (wave_items).
 // Bound by the records read and a 64-byte piece written per located row.  A
@@ -1775,15 +1786,35 @@ hipError_t launch_zero(uint32_t *p, uint32_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
+// A launch of wave_items over `lanes` lanes: a wavefront a group where several
+// share one set of lanes, so that few lanes launch no empty wavefronts beside
+// theirs (of one interval three in four: 1 M of its rows on a compact index 308
+// us so, 285 now).
+struct ItemGrid {
+  dim3 grid, block;
+};
+static ItemGrid item_grid(uint64_t lanes, uint64_t items_per_lane) {
+  const uint32_t parts = item_parts(lanes, items_per_lane), block = parts > 1u ? 64u : 256u;
+  return {dim3((uint32_t)((lanes + block - 1u) / block), parts), dim3(block)};
+}
+
 hipError_t launch_locate(const DevIndex &ix, uint32_t dsel, const int64_t *k, const int64_t *l,
                          uint32_t stride, uint32_t nintervals, uint32_t cap, uint64_t *pos,
                          uint32_t *nrows, hipStream_t s) {
   LocateParams P{ix, dsel, nintervals, cap, stride, k, l, pos, nrows};
-  const uint64_t grid = ((uint64_t)nintervals + 255) / 256;
-  if (grid == 0 || cap == 0) return hipSuccess;
-  const dim3 g((uint32_t)grid, item_parts(nintervals, cap));
-  if (cap <= kItems32) hipLaunchKernelGGL(locate_kernel<uint32_t>, g, dim3(256), 0, s, P);
-  else hipLaunchKernelGGL(locate_kernel<unsigned long long>, g, dim3(256), 0, s, P);
+  if (nintervals == 0 || cap == 0) return hipSuccess;
+  // Few intervals of an expanded index: 1 M rows of one 6.0 us, and no more where
+  // they have fewer rows; 12.3 by wave_items, whose setup serves 64 rows then.  (On
+  // a compact index, whose rows are chains, the two take 297 and 285 us.)
+  const uint64_t slots = (uint64_t)nintervals * cap;
+  if ((dsel ? ix.d[1] : ix.d[0]).sa && nintervals <= 16384u && slots <= (4u << 20)) {
+    hipLaunchKernelGGL(locate_slots_kernel, dim3((uint32_t)((slots + 255u) / 256u)), dim3(256), 0, s,
+                       P);
+    return hipGetLastError();
+  }
+  const ItemGrid g = item_grid(nintervals, cap);
+  if (cap <= kItems32) hipLaunchKernelGGL(locate_kernel<uint32_t>, g.grid, g.block, 0, s, P);
+  else hipLaunchKernelGGL(locate_kernel<unsigned long long>, g.grid, g.block, 0, s, P);
   return hipGetLastError();
 }
 
@@ -1833,12 +1864,11 @@ hipError_t launch_resolve(const DevIndex &ix, const fmi_hit *hits, const uint32_
                           hipStream_t s) {
   ResolveParams P{ix, hits, counts, offsets, koff, kstart, 2u * nreads, cap, row_cap, kcount,
                   record_len, chrom, coord};
-  const uint64_t grid = (2ull * nreads + 255) / 256;
-  if (grid == 0 || cap == 0 || row_cap == 0) return hipSuccess;
+  if (nreads == 0 || cap == 0 || row_cap == 0) return hipSuccess;
   const uint64_t per_slot = (uint64_t)cap * row_cap;
-  const dim3 g((uint32_t)grid, item_parts(2ull * nreads, per_slot));
-  if (per_slot <= kItems32) hipLaunchKernelGGL(resolve_kernel<uint32_t>, g, dim3(256), 0, s, P);
-  else hipLaunchKernelGGL(resolve_kernel<unsigned long long>, g, dim3(256), 0, s, P);
+  const ItemGrid g = item_grid(2ull * nreads, per_slot);
+  if (per_slot <= kItems32) hipLaunchKernelGGL(resolve_kernel<uint32_t>, g.grid, g.block, 0, s, P);
+  else hipLaunchKernelGGL(resolve_kernel<unsigned long long>, g.grid, g.block, 0, s, P);
   return hipGetLastError();
 }
 
