@@ -280,13 +280,13 @@ int search1_common(const fmi_index *ix, int mode, int strand_mask, const uint8_t
   rc = workspace_for(st, &w);
   if (rc) return rc;
   uint32_t grid = 0;
+  int cus = 256;
   Tuning t;
   {
     std::lock_guard<std::mutex> lk(g_mu);
     t = g_tuning;
   }
   if (persistent) {
-    int cus = 0;
     rc = cu_count(&cus);
     if (rc) return rc;
     grid = (uint32_t)cus * (t.wg_per_cu ? t.wg_per_cu : kDefaultWgPerCu);
@@ -304,7 +304,7 @@ int search1_common(const fmi_index *ix, int mode, int strand_mask, const uint8_t
   hipError_t e = fmi::launch_search1(ix->dev, mode == FMI_MODE_MISMATCH, persistent, false,
                                      (uint32_t)strand_mask, d_reads, d_offsets, nreads, cap,
                                      d_hits, d_counts, w.queue, w.stats, grid, t.chunk,
-                                     t.refill_min, own, st, staged);
+                                     t.refill_min, own, st, staged, (uint32_t)cus);
   return end_timed(st, e, "search1 launch");
 }
 

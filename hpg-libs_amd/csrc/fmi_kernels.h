@@ -41,7 +41,7 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
                           uint32_t nreads, uint32_t cap, fmi_hit *hits, uint32_t *counts,
                           uint32_t *queue, unsigned long long *stats, uint32_t grid_persistent,
                           uint32_t chunk, uint32_t refill_min, bool own_loads, hipStream_t s,
-                          void *staged = nullptr);
+                          void *staged = nullptr, uint32_t cus = 256u);
 // The staged launch's first part on an expanded index (fmi_search1t.hip): the
 // reads searched on the text; those it leaves are appended to list, with their
 // records in rec, or, longer than a slot, stored from wide[nreads - 1] downward.

@@ -1654,7 +1654,7 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
                           uint32_t nreads, uint32_t cap, fmi_hit *hits, uint32_t *counts,
                           uint32_t *queue, unsigned long long *stats, uint32_t grid_persistent,
                           uint32_t chunk, uint32_t refill_min, bool own_loads, hipStream_t s,
-                          void *staged) {
+                          void *staged, uint32_t cus) {
   const uint32_t ntasks = nreads;   // one task per read (both strands in turn)
   S1Params P{ix, reads, offsets, hits, counts, queue, stats, ntasks, strand_mask, cap, chunk,
              refill_min, 0u, nullptr, nullptr, nullptr, 1};
@@ -1681,7 +1681,7 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
         // on the text first; the two kernels below take the reads it leaves
         uint32_t *wide = rec + (uint64_t)kRecWords * ntasks;
         e = launch_search1_text(ix, mm_only, strand_mask, reads, offsets, ntasks, cap, hits,
-                                counts, rec, wide, head + 2, head + 3, left, head + 1, 256u, s);
+                                counts, rec, wide, head + 2, head + 3, left, head + 1, cus, s);
         if (e != hipSuccess) return e;
         P.list = list = left;
         P.list_n = list_n = head + 1;
@@ -1689,9 +1689,8 @@ hipError_t launch_search1(const DevIndex &ix, bool mm_only, bool persistent, boo
         far_n = head + 3;
       } else {
         // a strand a task: a lane's chain is half as long, and a lane that ends
-        // early takes the next (200 K
-        // reads of 100 bases over 64 Mbp 1402 to 1149 us, 1 M 4029 to 3672,
-        // 2000 893 to 564)
+        // early takes the next (200 K reads of 100 bases over 64 Mbp 1402 to
+        // 1149 us, 1 M 4029 to 3672, 2000 893 to 564)
         if (strand_mask == 3u) {
           P.split = 1u;
           P.ntasks = 2u * ntasks;

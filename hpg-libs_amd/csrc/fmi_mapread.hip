@@ -184,7 +184,8 @@ __global__ __launch_bounds__(256) void map_single_kernel(MapParams P) {
       chrom[j] = 0u;
       if (j >= R.n) continue;
       // direction: the record's dir is 0; + keeps it, - flips it
-      const uint64_t key = strand ? (uint64_t)n + 1u - R.q[j] - (uint64_t)len - 1u : (uint64_t)R.q[j];
+      const uint64_t key =
+          strand ? (uint64_t)n + 1u - R.q[j] - (uint64_t)len - 1u : (uint64_t)R.q[j];
       chrom[j] = contig_of(P.koff, P.kcount, key, (uint64_t)len);
       if (chrom[j]) pos[j] = P.kstart[chrom[j] - 1u] + (key - P.koff[chrom[j] - 1u]);
     }

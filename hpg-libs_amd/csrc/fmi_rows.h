@@ -168,8 +168,9 @@ struct NodeStrings {
 template <bool STAGED, bool MM_ONLY>
 __device__ __forceinline__ NodeStrings node_strings(const DevIndex &ix, uint32_t dsel,
                                                     uint32_t comp, const ReadBases<STAGED> &rd,
-                                                    const TextRows &R, const int32_t (&run)[kTextRows],
-                                                    int32_t a, int32_t p, int32_t d, int32_t c1) {
+                                                    const TextRows &R,
+                                                    const int32_t (&run)[kTextRows], int32_t a,
+                                                    int32_t p, int32_t d, int32_t c1) {
   NodeStrings S;
   S.live = 0u;
   S.cnts = 0u;

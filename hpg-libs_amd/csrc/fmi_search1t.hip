@@ -38,13 +38,14 @@ struct S1tParams {
   int32_t wide_m;                  // rows_wide_m
 };
 
-// Where a read goes on: nowhere, in search1_wave_kernel, in search1_kernel.
-enum : uint32_t { kDone = 0u, kToWave = 1u, kToList = 2u };
-
 // Anchor halves shorter than this go to search1_kernel at once: they have more
 // than kTextRows rows in a repeat (and from 3.1 Gbp, 4^16, by chance), and the
 // passes here would mostly be run in vain.
 constexpr int32_t kTextHalf = 16;
+
+// In the count of a read left to search1_kernel (which writes it anew): no
+// wavefront can take it, for one of its anchors' more than 64 rows or its length.
+constexpr uint32_t kManyRead = 0x80000000u;
 
 struct S1tOut {
   fmi_hit *out;
@@ -72,12 +73,12 @@ __device__ __forceinline__ void add_string(S1tOut &O, const DevDir &D, uint32_t 
 }
 
 // One pass (0: the right half backward on the pair's first index, then the
-// left; 1: the left half forward on the second, then the right); where the
-// read goes on when the anchor has more rows than it can take.
+// left; 1: the left half forward on the second, then the right); false when
+// the anchor has more rows than it can take (then kManyRead in the count).
 template <bool MM_ONLY>
-__device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass, uint32_t strand,
-                                              const ReadBases<true> &rd, int32_t len,
-                                              int32_t wide_m, S1tOut &O) {
+__device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uint32_t strand,
+                                          const ReadBases<true> &rd, int32_t len, int32_t wide_m,
+                                          S1tOut &O) {
   const uint32_t dsel = pass ^ strand;
   const DevDir &D = dir_of(ix, dsel);
   const int32_t half = len / 2, d = pass ? 1 : -1, p0 = pass ? 0 : len - 1;
@@ -85,8 +86,11 @@ __device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass,
   TextRows R;
   uint32_t k, l;
   const uint32_t found = search_rows<true>(ix, dsel, strand, rd, p0, d, m0, R, k, l, wide_m);
-  if (found == kRowsNone) return kDone;
-  if (found != kRowsFew) return found == kRowsMany && l - k < 64u ? kToWave : kToList;
+  if (found != kRowsFew) {
+    if (found == kRowsNone) return true;
+    if (l - k >= 64u) O.cnt |= kManyRead;
+    return false;
+  }
   int32_t run[kTextRows] = {-1, -1, -1, -1};
 #pragma unroll
   for (uint32_t j = 0; j < kTextRows; ++j)
@@ -117,7 +121,7 @@ __device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass,
       }
     if (rows) O.add(D, first, rows, 0, -1, len - 1, 0, 0u, 0u, 0u, 0u);
   }
-  return kDone;
+  return true;
 }
 
 // A thread per (read, strand); a read's two threads pack it into one LDS slot.
@@ -126,16 +130,18 @@ __device__ __forceinline__ uint32_t text_pass(const DevIndex &ix, uint32_t pass,
 // bases or more bases than a slot to search1_kernel; its record is written from
 // the slot.
 // Bound by the latency of a pass's chain and the lines it reads (an entry,
-// contexts, suffixes, text and the records' rows).  At 4 waves: 1 M reads of 150 bases over 64 Mbp: 576 us, where the records,
-// the state machine and its records' rows took 1284; 2 M over 3.1 Gbp 1552
-// of 2300; a request of 500 reads 43 of 500.
+// contexts, suffixes, text and the records' rows), with 20 of 64 lanes active:
+// the strand a read is not from ends after its table entry.  At 4 waves: 1 M
+// reads of 150 bases over 64 Mbp: 576 us, where the records, the state machine
+// and its records' rows took 1284; 2 M over 3.1 Gbp 1552 of 2300; a request of
+// 500 reads 43 of 500.
 // MINW: the waves per SIMD the registers are held to.  4 (none spilled) where
 // every group of the batch is resident at once, and a read's own chain is
-// what counts; 6 (80 VGPRs, 26 spilled: three groups a CU instead of two)
+// what counts; 6 (80 VGPRs, 24 to 28 spilled: three groups a CU instead of two)
 // beyond, where more lines in flight are worth the spills.  Calls: 1 M x 150 at
-// 64 Mbp 610 to 569 us, 2 M at 3.1 Gbp 1608 to 1460, 700 K of 50-250 with indels
-// and positions at 256 Mbp 627 to 557, but 500 reads 60 to 64.  5 waves (6
-// spilled) hold no third group.
+// 64 Mbp 610 to 569 us (554 now), 2 M at 3.1 Gbp 1608 to 1460 (1437), 700 K of
+// 50-250 with indels and positions at 256 Mbp 627 to 557 (569), but 500 reads 60
+// to 64.  5 waves (6 spilled) hold no third group.
 template <bool MM_ONLY, int MINW>
 __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
   __shared__ uint32_t slots[kReadRecordWords * 256u];
@@ -178,26 +184,29 @@ __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
   }
   if (threadIdx.x == 0u) nids = narrived = 0u;
   __syncthreads();
-  uint32_t left = kDone;
+  bool left = false;
+  uint32_t cnt = 0u;
   if (mine) {
     const bool asked = ((P.strand_mask >> strand) & 1u) != 0u;
     S1tOut O{P.hits + (uint64_t)t64 * P.cap, P.cap, 0u, strand};
     if (!staged || len / 2 < kTextHalf) {
-      left = kToList;
+      left = true;
+      O.cnt = kManyRead;
     } else if (asked) {
       const ReadBases<true> bases{nullptr, slot};
-      for (uint32_t pass = 0; pass < 2u && left == kDone; ++pass)
-        left = text_pass<MM_ONLY>(P.ix, pass, strand, bases, len, P.wide_m, O);
+      for (uint32_t pass = 0; pass < 2u && !left; ++pass)
+        left = !text_pass<MM_ONLY>(P.ix, pass, strand, bases, len, P.wide_m, O);
     }
-    P.counts[t64] = O.cnt;
+    cnt = O.cnt;
+    P.counts[t64] = cnt;
   }
   // the left reads, their records first
   const uint64_t pair = 0x5555555555555555ull;
-  uint64_t wide = __ballot(left == kToWave), list = __ballot(left == kToList);
-  list = (list | (list >> 1)) & pair;
-  wide = (wide | (wide >> 1)) & pair & ~list;      // a strand's wider anchor decides
+  uint64_t any = __ballot(left), list = __ballot(cnt >= kManyRead);
+  any = (any | (any >> 1)) & pair;
+  list = (list | (list >> 1)) & pair;              // a strand's wider anchor decides
   const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t me = 1ull << (lane & ~1u), any = wide | list;
+  const uint64_t me = 1ull << (lane & ~1u);
   if ((any & me) && staged) {
     uint4 *out = reinterpret_cast<uint4 *>(P.rec + (uint64_t)rd * kReadRecordWords);
     for (uint32_t i = strand; i < kReadRecordWords / 4u; i += 2u)
@@ -211,7 +220,7 @@ __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
   if (lane == 0u && any) at = atomicAdd(&nids, (uint32_t)__popcll(any));
   at = __shfl(at, 0);
   if ((any & me) && strand == 0u) {
-    const uint32_t to = (wide & me) ? 0u : (staged ? 1u : 2u);
+    const uint32_t to = !(list & me) ? 0u : (staged ? 1u : 2u);
     ids[at + (uint32_t)__popcll(any & (me - 1ull))] = (threadIdx.x >> 1) | (to << 8);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -219,34 +228,27 @@ __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
   if (lane == 0u) before = atomicAdd(&narrived, 1u);
   if (__shfl(before, 0) != 512u / 64u - 1u) return;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  const uint32_t n = nids, rd0 = blockIdx.x * 256u;
-  auto places = [&](uint32_t i, uint32_t &id, uint64_t (&m)[3]) {
-    id = i + lane < n ? ids[i + lane] : 3u << 8;
-#pragma unroll
-    for (uint32_t c = 0; c < 3u; ++c) m[c] = __ballot((id >> 8) == c);
-  };
-  uint32_t id, cnt[3] = {0u, 0u, 0u};
-  uint64_t m[3];
-  for (uint32_t i = 0; i < n; i += 64u) {
-    places(i, id, m);
-#pragma unroll
-    for (uint32_t c = 0; c < 3u; ++c) cnt[c] += (uint32_t)__popcll(m[c]);
-  }
-  uint32_t first = 0u;                             // of lanes 0, 1, 2: the three lists'
-  const uint32_t mine3 = lane == 0u ? cnt[0] : (lane == 1u ? cnt[1] : (lane == 2u ? cnt[2] : 0u));
-  if (mine3) first = atomicAdd(lane == 0u ? P.wide_n : (lane == 1u ? P.list_n : P.long_n), mine3);
-  uint32_t f[3] = {__shfl(first, 0), __shfl(first, 1), __shfl(first, 2)};
-  for (uint32_t i = 0; i < n; i += 64u) {
-    places(i, id, m);
-    const uint32_t r = rd0 + (id & 255u), c = id >> 8;
-    const uint64_t mc = c == 0u ? m[0] : (c == 1u ? m[1] : m[2]);
-    const uint32_t p = (c == 0u ? f[0] : (c == 1u ? f[1] : f[2])) +
-                       (uint32_t)__popcll(mc & ((1ull << lane) - 1ull));
-    if (c == 0u) P.wide[p] = r;
-    else if (c == 1u) P.list[p] = r;
-    else if (c == 2u) P.wide[P.nreads - 1u - p] = r;
-#pragma unroll
-    for (uint32_t e = 0; e < 3u; ++e) f[e] += (uint32_t)__popcll(m[e]);
+  const uint32_t n = nids;
+#pragma unroll 1
+  for (uint32_t c = 0; c < 3u; ++c) {
+    uint32_t cnt = 0u, at_c = 0u;
+#pragma unroll 1
+    for (uint32_t i = lane; i - lane < n; i += 64u)
+      cnt += (uint32_t)__popcll(__ballot(i < n && ids[min(i, 255u)] >> 8 == c));
+    if (cnt == 0u) continue;
+    if (lane == 0u) at_c = atomicAdd(c == 0u ? P.wide_n : (c == 1u ? P.list_n : P.long_n), cnt);
+    at_c = __shfl(at_c, 0);
+#pragma unroll 1
+    for (uint32_t i = lane; i - lane < n; i += 64u) {
+      const uint32_t id = ids[min(i, 255u)];
+      const bool is = i < n && id >> 8 == c;
+      const uint64_t m = __ballot(is);
+      const uint32_t p = at_c + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+      if (is)
+        (c == 1u ? P.list : P.wide)[c == 2u ? P.nreads - 1u - p : p] =
+            blockIdx.x * 256u + (id & 255u);
+      at_c += (uint32_t)__popcll(m);
+    }
   }
 }
 

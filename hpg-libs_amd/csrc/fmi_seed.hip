@@ -8,8 +8,9 @@
 //      count, as the reference's `int actual_mappings`), rows to resolve,
 //      and the rows of every 64 seeds
 //   3. exclusive scan of those sums
-//   4. the rows of 64 seeds shared out in a wavefront: locate (getScompValue) on BACKWARD, binsearch over
-//      the karyotype offsets, the contig-end check key + len <= offset[idx]
+//   4. the rows of 64 seeds (or, where some bring very many, of a tile of rows)
+//      shared out in a wavefront: locate (getScompValue) on BACKWARD, binsearch
+//      over the karyotype offsets, the contig-end check key + len <= offset[idx]
 //      with len = seq_end - seq_start (one short, bwt.c:1214), region record.
 #include <hip/hip_runtime.h>
 
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(256) void seed_context_kernel(SeedParams P) {
         const uint32_t km = (1u << (2u * K)) - 1u;
         const uint64_t e[2] = {P.ix.kmer[0][(uint32_t)code[0] & km],
                                P.ix.kmer[0][(uint32_t)code[1] & km]};
-// both strands' first rows are read together where they lie in two
+        // both strands' first rows are read together where they lie in two
         // 16-byte pieces of contexts (almost all do), then both suffixes
         const uint32_t gs = L - K, gm = (uint32_t)win_mask(min(gs, 16u));
         uint4 c[2][2];
@@ -886,7 +887,8 @@ __global__ __launch_bounds__(256) void left_windows_kernel(InexactParams P) {
   if (threadIdx.x == 0u && all) base = atomicAdd(P.list_n, all);
   __syncthreads();
   if (!own) return;
-  uint32_t at = base + (wave > 0u ? w0 : 0u) + (wave > 1u ? w1 : 0u) + (wave > 2u ? w2 : 0u) + incl - own;
+  uint32_t at = base + incl - own;
+  at += (wave > 0u ? w0 : 0u) + (wave > 1u ? w1 : 0u) + (wave > 2u ? w2 : 0u);
   for (; marks; marks &= marks - 1u) P.list[at++] = (uint32_t)g0 + (uint32_t)__builtin_ctz(marks);
 }
 
