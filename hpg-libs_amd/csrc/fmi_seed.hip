@@ -399,11 +399,12 @@ __device__ __forceinline__ void block_rows(const RowParams &P, uint64_t b, uint6
 // scanned row counts, 27 dependent loads for 94 M slots: 57 M rows in 3.2 ms
 // (and 0.6 to scan the counts), 2.0 as below.
 // TILED: a wavefront takes `tile` neighbouring rows instead, of as many seeds as
-// they are.  A batch is taken so where some 64 seeds bring more than kSeedBlockRows
-// rows: those of one wavefront are a chain, 0.95 us per 64 (6.5 on a compact
-// index), and a single seed of 2 M rows took 29.4 ms (203), 0.1 (0.2) by tiles.
-// Where all bring fewer, tiles look most of the 64 seeds up twice: 1.4 M rows of
-// 1.7 M seeds TILECOST.
+// they are.  A batch is taken so where some 64 seeds bring more than
+// kSeedBlockRows rows and 4 times what a wavefront of a full device (8192) has
+// on average: the rows of one wavefront are a chain, 0.95 us per 64 (6.5 on a
+// compact index), and a single seed of 2 M rows took 29.4 ms (203), 0.10 (0.19)
+// by tiles.  Elsewhere tiles look most of the 64 seeds up twice: 1.7 M seeds of
+// 18 bases, a row each, on a compact index 1.16 ms, 1.35 by tiles.
 template <bool TILED>
 __global__ __launch_bounds__(256) void seed_rows_kernel(RowParams P) {
   const uint64_t nsums = (P.nseeds + 63u) / 64u;
