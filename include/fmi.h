@@ -388,13 +388,16 @@ int fmi_get_tuning(uint32_t *wg_per_cu, uint32_t *chunk, uint32_t *refill_min);
 #define FMI_LOADS_OWN 2u
 int fmi_set_load_mode(uint32_t mode);
 int fmi_get_load_mode(uint32_t *mode);
-/* Whether fmi_search1_batch stages reads (the default, 1): a streaming
- * kernel packs each read into a 96-byte record (2-bit codes, N flags) in
- * the stream's scratch (104 bytes per read, for batches of at most 2^27
- * reads) and every lane of the persistent search holds its read in LDS, so
- * no step reads it from memory again; reads longer than 256 bases are
- * searched afterwards without staging.  0 reads the read from memory at
- * every step.  Results never depend on it.  No reference counterpart. */
+/* Whether fmi_search1_batch stages reads (the default, 1), for batches of at
+ * most 2^27 reads, with 104 bytes per read of the stream's scratch.  On an
+ * expanded index the reads are then searched on the text, packed into LDS by
+ * their threads, and only those with too many rows, too few bases or more
+ * than 256 go on to the step-by-step search.  On a compact index a streaming
+ * kernel packs each read into a 96-byte record (2-bit codes, N flags) and
+ * every lane of the persistent search holds its read in LDS; reads longer
+ * than 256 bases are searched afterwards without staging.  0 searches step by
+ * step and reads the read from memory at every step.  Results never depend on
+ * it.  No reference counterpart. */
 int fmi_set_staging(int enable);
 int fmi_get_staging(int *enable);
 
