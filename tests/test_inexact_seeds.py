@@ -285,7 +285,7 @@ def test_gpu_inexact_windows_left(gpu_engine, n, kmer):
 def test_gpu_inexact_short_windows_cost(gpu_engine, seed_size, min_seed):
     """Windows so short that most have more rows than a wavefront takes at once
     (12 bases over 16 Mbp, remainders of 10) are searched once: the call takes at
-    most 1.25 times what it takes without row contexts, 2.2 and 2.3 times where
+    most 1.5 times what it takes without row contexts (1.0 and 1.1), 2.2 and 2.3 where
     they were searched by them first and again."""
     hp = gpu_engine
     rng = np.random.default_rng(56)
@@ -310,7 +310,7 @@ def test_gpu_inexact_short_windows_cost(gpu_engine, seed_size, min_seed):
                     bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, C.byref(got), None))
                 took[form] = min(took.get(form, 1.0), time.perf_counter() - t)
         print(seed_size, took)
-        assert took["contexts"] < 1.25 * took["none"], took
+        assert took["contexts"] < 1.5 * took["none"], took
     finally:
         for b in bufs:
             b.free()
