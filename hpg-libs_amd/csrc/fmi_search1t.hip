@@ -140,7 +140,7 @@ __device__ __forceinline__ bool text_pass(const DevIndex &ix, uint32_t pass, uin
 // what counts; 6 (80 VGPRs, 24 to 28 spilled: three groups a CU instead of two)
 // beyond, where more lines in flight are worth the spills.  Calls: 1 M x 150 at
 // 64 Mbp 610 to 569 us (554 now), 2 M at 3.1 Gbp 1608 to 1460 (1437), 700 K of
-// 50-250 with indels and positions at 256 Mbp 627 to 557 (569), but 500 reads 60
+// 50-250 with indels and positions at 256 Mbp 627 to 557 (582), but 500 reads 60
 // to 64.  5 waves (6 spilled) hold no third group.
 template <bool MM_ONLY, int MINW>
 __global__ __launch_bounds__(512, MINW) void search1_text_kernel(S1tParams P) {
